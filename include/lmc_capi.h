@@ -68,10 +68,9 @@ void lmc_model_free(lmc_model *m);
 int32_t lmc_model_num_species(const lmc_model *m);
 /* Species code of an element string, -1 if not in the model. */
 int32_t lmc_model_species_code(const lmc_model *m, const char *element);
-/* Formulation of the jump kernels used by this model's stateless calls and as the default of
- * new KMC drivers: 0 = dense (every cluster of every jump; default), 1 = solvent baseline
- * (all-solvent sums precomputed per (solvent, migrating species); only clusters touching a
- * non-solvent site are evaluated). Both are exact; they differ in FP64 summation order. */
+/* Default formulation of new KMC drivers: 0 (default) or 1. Both evaluate a jump from all-solvent
+ * sums and the exact one- and two-site changes at the sites that hold another species; the stateless
+ * calls always do. */
 int lmc_model_set_formulation(lmc_model *m, int32_t formulation);
 /* Element string of a species code (NULL if out of range); valid while m lives. */
 const char *lmc_model_species_name(const lmc_model *m, int32_t code);
@@ -274,10 +273,9 @@ void lmc_kmc_free(lmc_kmc *k);
 int lmc_kmc_set_schedule(lmc_kmc *k, int32_t n_points, const double *time, const double *temp);
 /* Per-replica trace of the next `capacity` steps (selected neighbour, Ea, dE, time). 0 = off. */
 int lmc_kmc_set_trace(lmc_kmc *k, uint64_t capacity);
-/* Kernel of this driver: 0 dense (256 threads per replica, up to four replicas per CU),
- * 1 solvent baseline (see lmc_model_set_formulation), 2 dense wide shape (768 threads per
- * replica, one per CU: for batches of at most one replica per CU); these are first-order steps
- * and have no reference counterpart. 3: second-order residence-time steps, replacing
+/* Kernel of this driver: 0 and 1 one wave per replica, or four when every replica has a CU of its
+ * own; 2 always four waves per replica. These are first-order steps, differ in FP64 summation order
+ * only, and have no reference counterpart. 3: second-order residence-time steps, replacing
  * KineticMcChainOmpi (lmc/mc/include/KineticMcChainOmpi.h, KineticMcChainOmpi.cpp:56-151):
  * the 12 x 12 jumps out of the vacancy's first neighbours after each virtual jump, the
  * second-order probabilities and the deterministic time t_2; the previous site starts as the

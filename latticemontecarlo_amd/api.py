@@ -72,7 +72,7 @@ class Model:
         check(lib().lmc_check_errors(self.h))
 
     def set_formulation(self, formulation):
-        """0 = dense, 1 = solvent baseline (default)."""
+        """Default formulation of new KMC drivers, 0 or 1 (see lmc_model_set_formulation)."""
         check(lib().lmc_model_set_formulation(self.h, formulation))
 
 
@@ -360,8 +360,8 @@ class KineticMcFirst:
 
     def autotune(self, steps=200):
         """Times each kernel shape for `steps` steps on a scratch copy and keeps the fastest:
-        formulation 0 dense, 1 solvent baseline, 2 dense wide (tried only with at most one
-        replica per CU); ms_* per batch step (NaN when not tried)."""
+        formulations 0, 1 and 2 (2, four waves per replica, tried only with at most one replica per
+        CU); ms_* per batch step (NaN when not tried)."""
         ch, ms = C.c_int32(), (C.c_double * 3)()
         check(lib().lmc_kmc_autotune_shapes(self.h, steps, C.byref(ch), ms))
         return dict(formulation=ch.value, ms_dense=ms[0], ms_solvent=ms[1], ms_wide=ms[2])

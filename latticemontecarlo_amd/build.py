@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "liblmc.so")
 
-SOURCES = ["lmc_tables.cpp", "lmc_model.cpp", "lmc_capi.cpp", "lmc_config_io.cpp", "lmc_jump_kernels.hip",
+SOURCES = ["lmc_tables.cpp", "lmc_model.cpp", "lmc_pairs.cpp", "lmc_capi.cpp", "lmc_config_io.cpp", "lmc_jump_kernels.hip",
            "lmc_site_kernels.hip", "lmc_surrogate.hip", "lmc_surrogate_kmc.hip"]
 FLAGS = [
     "-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC",
@@ -24,9 +24,8 @@ FLAGS = [
 ]
 # Per-source instruction-scheduling strategies of LLVM's AMDGPU backend, each measured against
 # the default on its own workloads (results unchanged):
-# - KMC kernels, iterative ILP: 1 024 replicas of 20^3 cells, 1.336e8 against 1.298e8 steps/s
-#   on 20-step launches and 1.624e8 against 1.584e8 on 50 000-step runs; chain steps +1.7 %;
-#   the uneven batch unchanged.
+# - KMC kernels: the default. Their list batches are staged by hand, and on 1 024 replicas of 20^3
+#   cells every other strategy stays within 2 % of it (iterative min-register 40 % slower).
 # - canonical-MC kernels, iterative ILP: annealing +2.6 %, CMC beside the uneven KMC batch
 #   +0.9 %, CanonicalMcOmp rounds -0.25 %.
 # - surrogate KMC kernel, iterative max-occupancy: +6.2 % (iterative ILP 2.6x and iterative
@@ -34,7 +33,6 @@ FLAGS = [
 # The surrogate's training kernels keep the default: iterative ILP and max-memory-clause trained
 # within the run-to-run spread of 160 epochs (about 20 s), iterative max-occupancy 18 % slower.
 SOURCE_FLAGS = {
-    "lmc_jump_kernels.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
     "lmc_site_kernels.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
     "lmc_surrogate_kmc.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-maxocc"],
 }

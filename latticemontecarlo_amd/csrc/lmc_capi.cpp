@@ -22,6 +22,7 @@
 #include "lmc_element.h"
 #include "lmc_error.h"
 #include "lmc_model.h"
+#include "lmc_pairs.h"
 #include "lmc_rng.h"
 #include "lmc_surrogate.h"
 #include "lmc_tables.h"
@@ -168,100 +169,33 @@ Model::~Model() {
   }
 }
 
-// Solvent-baseline tables. With every non-endpoint site of a jump environment holding the
-// solvent s, the cluster sums of dE and of the barrier logits depend only on (s, M); a real
-// environment adds, for each cluster with a non-solvent site, value(cluster) - value(all s).
-// A cluster with several non-solvent sites is listed under each of them and evaluated only at
-// the lowest-numbered one (the kernel checks the entry's other slot).
-static void BuildSolventTables(const Model &m, const JumpTables &jt, const std::vector<int> &eb1,
-                               const std::vector<int> &eb2, std::vector<uint16_t> &off,
-                               std::vector<uint32_t> &inc, std::vector<double> &base) {
+// Sums (dE, MMM logit, MM2 logit) of a jump environment whose non-endpoint sites all hold element rank s,
+// by migrating rank M: base[s][M][3].
+static std::vector<double> BuildBaseSums(const Model &m, const JumpTables &jt, const std::vector<int> &code) {
   const int S = m.S;
-  // per slot j: the clusters containing j (j not a jump endpoint), by list type
-  std::vector<std::vector<uint32_t>> per[3];
-  for (auto &v : per) v.assign(kEnvSlots, {});
-  // state entry: reduced weight-block byte offset [0:13] (rank layout, positive rows) | j is the
-  // second other site [13] | the other site o [14:20] (63 = none) | neighbour-endpoint side [31]
-  auto add_state = [&](const std::vector<StateCluster> &cl, int endpoint, bool nside) {
-    for (const auto &c : cl) {
-      int others[2] = {-1, -1}, n = 0;
-      for (int i = 0; i < c.size; ++i)
-        if (c.slots[i] != endpoint) others[n++] = c.slots[i];
-      const int block = ReducedBlock(c.label, m.ne);
-      for (int i = 0; i < n; ++i) {
-        const int other = n == 2 ? others[1 - i] : 63;
-        per[0][others[i]].push_back(static_cast<uint32_t>(block * 8) | (static_cast<uint32_t>(i) << 13) |
-                                    (static_cast<uint32_t>(other) << 14) | (nside ? 0x80000000u : 0u));
-      }
-    }
-  };
-  add_state(jt.state_v_only, jt.v_slot, false);
-  add_state(jt.state_n_only, jt.n_slot, true);
-  // orbit entry: byte offset of the orbit's expanded weights [0:16] | j takes the rank*8 role
-  // (second site, or a singlet's site) [16] | the other site o [17:23] (63 = none); backward
-  // entries read canonical slot x at mirror[x]
-  auto add_orbits = [&](const OrbitTable &ot, const std::vector<int> &eb, int list, bool backward) {
-    for (const auto &c : ot.clusters) {
-      const uint32_t bse = static_cast<uint32_t>(eb[c.orbit]) * 8;
-      if (bse > 65535) throw std::invalid_argument("feature vector too long for the packed tables");
-      const int nsl = c.s1 < 0 ? 1 : 2;
-      for (int pos = 0; pos < nsl; ++pos) {
-        const int canon = pos == 0 ? c.s0 : c.s1;
-        const int canon_other = nsl == 1 ? -1 : (pos == 0 ? c.s1 : c.s0);
-        const int slot = backward ? jt.mirror[canon] : canon;
-        const int other = canon_other < 0 ? 63 : (backward ? jt.mirror[canon_other] : canon_other);
-        const uint32_t role = (nsl == 1 || pos == 1) ? 1u : 0u;
-        per[list][slot].push_back(bse | (role << 16) | (static_cast<uint32_t>(other) << 17));
-      }
-    }
-  };
-  if (m.kind == kE0 || m.kind == kQuartic) add_orbits(jt.mmm, eb1, 1, false);
-  if (m.kind == kQuartic) {
-    add_orbits(jt.mm2, eb2, 2, false);
-    add_orbits(jt.mm2, eb2, 2, true);
-  }
-  off.assign(3 * (kEnvSlots + 1), 0);
-  for (int t = 0; t < 3; ++t) {
-    for (int j = 0; j < kEnvSlots; ++j) {
-      off[t * (kEnvSlots + 1) + j] = static_cast<uint16_t>(inc.size());
-      inc.insert(inc.end(), per[t][j].begin(), per[t][j].end());
-    }
-    off[t * (kEnvSlots + 1) + kEnvSlots] = static_cast<uint16_t>(inc.size());
-  }
-  if (inc.size() > 65535) throw std::invalid_argument("incidence table too large");
-
-  const double nan = std::numeric_limits<double>::quiet_NaN();
-  base.assign(static_cast<size_t>(S) * S * 3, nan);
+  std::vector<double> base;
   auto w_of = [&](int label, int a, int s) -> long double {
     if (label == 0) return m.w[a];
     if (label < 4) return m.w[S + (label - 1) * S * S + a * S + s];
     return m.w[S + 3 * S * S + (label - 4) * S * S * S + (a * S + s) * S + s];
   };
   auto tt = [&](int kind, int a, int b) { return m.type_tab[(kind * S + a) * S + b]; };
-  for (int s = 0; s < S; ++s) {
-    if (s == m.x_code) continue;
-    for (int M = 0; M < S; ++M) {
-      if (M == m.x_code) continue;
+  for (int s : code)
+    for (int M : code) {
       long double de = 0, la = 0, lb = 0;
       for (const auto &c : jt.state_v_only) de += w_of(c.label, M, s) - w_of(c.label, m.x_code, s);
       for (const auto &c : jt.state_n_only) de -= w_of(c.label, M, s) - w_of(c.label, m.x_code, s);
       if (m.kind == kE0 || m.kind == kQuartic)
-        for (const auto &c : jt.mmm.clusters) {
-          const int kind = jt.mmm.orbit_kind[c.orbit];
-          la += m.b_mmm[static_cast<size_t>(M) * m.F_mmm + m.base_mmm[c.orbit] + tt(kind, s, s)];
-        }
+        for (const auto &c : jt.mmm.clusters)
+          la += m.b_mmm[static_cast<size_t>(M) * m.F_mmm + m.base_mmm[c.orbit] +
+                        tt(jt.mmm.orbit_kind[c.orbit], s, s)];
       if (m.kind == kQuartic)
-        for (const auto &c : jt.mm2.clusters) {
-          const int kind = jt.mm2.orbit_kind[c.orbit];
+        for (const auto &c : jt.mm2.clusters)
           lb += 2.0L * m.b_mm2[static_cast<size_t>(M) * m.F_mm2 + m.base_mm2[c.orbit] +
-                               tt(kind, s, s)];
-        }
-      double *o = &base[(static_cast<size_t>(s) * S + M) * 3];
-      o[0] = static_cast<double>(de);
-      o[1] = static_cast<double>(la);
-      o[2] = static_cast<double>(lb);
+                               tt(jt.mm2.orbit_kind[c.orbit], s, s)];
+      for (long double x : {de, la, lb}) base.push_back(static_cast<double>(x));
     }
-  }
+  return base;
 }
 
 // Models are shared by host threads (the reference's predictors are const objects called from
@@ -338,25 +272,18 @@ const KTables &Upload(Model &m) {
   // read the zero at the end of every weight row. Their sites are slot 63 (rank entries 0), in
   // each list's own byte roles: a state entry's byte 0 indexes the rank*8 bytes and byte 1 the
   // 16-bit rank*8*ne words (offset 2*63); an orbit entry the other way round.
-  // The wide kernel shape (64 lanes per event, 4 entries each) reads copies padded to multiples
-  // of kClusterPadWide.
   auto pad = [](std::vector<uint32_t> &v, int to, uint32_t roles, uint32_t zero_at) {
     if (zero_at > 65535) throw std::invalid_argument("weight table too large for the packed tables");
     while (v.size() % static_cast<size_t>(to)) v.push_back(roles | (zero_at << 16));
   };
   const uint32_t state_roles = 63u | (126u << 8), orbit_roles = 126u | (63u << 8);
-  std::vector<uint32_t> state_w = state, mmm_w = mmm, mm2_w = mm2;
   pad(state, kClusterPad, state_roles, static_cast<uint32_t>(nr * 8));
   pad(mmm, kClusterPad, orbit_roles, static_cast<uint32_t>(F1e * 8));
   pad(mm2, kClusterPad, orbit_roles, static_cast<uint32_t>(F2e * 8));
-  pad(state_w, kClusterPadWide, state_roles, static_cast<uint32_t>(nr * 8));
-  pad(mmm_w, kClusterPadWide, orbit_roles, static_cast<uint32_t>(F1e * 8));
-  pad(mm2_w, kClusterPadWide, orbit_roles, static_cast<uint32_t>(F2e * 8));
   // the 16-bit rank words are read at even byte offsets only
-  for (const auto *v : {&state, &state_w})
-    for (uint32_t e : *v)
+  for (uint32_t e : state)
       if ((e >> 8) & 1) throw std::logic_error("state entry with an odd rank-word offset");
-  for (const auto *v : {&mmm, &mm2, &mmm_w, &mm2_w})
+  for (const auto *v : {&mmm, &mm2})
     for (uint32_t e : *v)
       if (e & 1) throw std::logic_error("orbit entry with an odd rank-word offset");
   std::vector<uint32_t> site_cl;
@@ -387,9 +314,6 @@ const KTables &Upload(Model &m) {
   b.Add(state, &k.state);
   b.Add(mmm, &k.mmm);
   b.Add(mm2, &k.mm2);
-  b.Add(state_w, &k.state_w);
-  b.Add(mmm_w, &k.mmm_w);
-  b.Add(mm2_w, &k.mm2_w);
   b.Add(site_cl, &k.site_cl);
   b.Add(site_off, &k.site_off);
   b.Add(m.w, &k.w);
@@ -404,13 +328,38 @@ const KTables &Upload(Model &m) {
   b.Add(e1, &k.eci1);
   b.Add(e2, &k.eci2);
   b.Add(e3, &k.eci3);
-  std::vector<uint16_t> inc_off;
-  std::vector<uint32_t> inc;
-  std::vector<double> base;
-  BuildSolventTables(m, jt, eb1, eb2, inc_off, inc, base);
-  b.Add(inc_off, &k.inc_off);
-  b.Add(inc, &k.inc);
-  b.Add(base, &k.base);
+  const PairGeometry &pg = GetPairGeometry();
+  const PairTables pt = BuildPairTables(m);
+  std::vector<int32_t> site_pk;
+  for (const I3 &o : pg.site) site_pk.push_back(PackOff(o));
+  std::vector<uint8_t> slot, site_of;
+  for (int d = 0; d < 12; ++d) {
+    slot.insert(slot.end(), pg.slot[d].begin(), pg.slot[d].end());
+    site_of.insert(site_of.end(), pg.site_of[d].begin(), pg.site_of[d].end());
+  }
+  const std::vector<double> pbase = BuildBaseSums(m, jt, code);
+  b.Add(site_pk, &k.site_pk);
+  b.Add(slot, &k.slot);
+  std::vector<uint32_t> site3;
+  for (const auto &s : pg.site3) site3.insert(site3.end(), s.begin(), s.end());
+  b.Add(site_of, &k.site_of);
+  b.Add(site3, &k.site3);
+  b.Add(pt.cls, &k.cls);
+  b.Add(pt.clsb, &k.clsb);
+  b.Add(pt.dense, &k.dense);
+  b.Add(pt.denseb, &k.denseb);
+  b.Add(pt.one, &k.one);
+  b.Add(pt.oneb, &k.oneb);
+  std::vector<uint8_t> order;
+  for (const auto &o : pg.order) order.insert(order.end(), o.begin(), o.end());
+  b.Add(order, &k.order);
+  b.Add(pt.de, &k.de);
+  b.Add(pt.la, &k.la);
+  b.Add(pt.lb, &k.lb);
+  b.Add(pbase, &k.pbase);
+  k.de_row = pt.de_row;
+  k.la_row = pt.la_row;
+  k.lb_row = pt.lb_row;
   std::vector<int32_t> errflag(1, 0);
   const int32_t *err_ptr = nullptr;
   b.Add(errflag, &err_ptr);
@@ -426,9 +375,6 @@ const KTables &Upload(Model &m) {
   k.n_state = static_cast<int>(state.size());
   k.n_mmm = static_cast<int>(mmm.size());
   k.n_mm2 = static_cast<int>(mm2.size());
-  k.n_state_w = static_cast<int>(state_w.size());
-  k.n_mmm_w = static_cast<int>(mmm_w.size());
-  k.n_mm2_w = static_cast<int>(mm2_w.size());
   k.n_site = static_cast<int>(site_cl.size());
   k.n_eci = static_cast<int>(m.theta.size());
   k.v_slot = jt.v_slot;
@@ -443,8 +389,6 @@ const KTables &Upload(Model &m) {
   k.nwd = static_cast<int>(wd.size());
   k.wrow = wrow;
   k.rank_lut = rank_lut;
-  k.n_state_v = static_cast<int>(jt.state_v_only.size());
-  k.n_inc = static_cast<int>(inc.size());
   k.solvent_default = 0;
   for (int c = 0; c < m.S; ++c)
     if (m.eci.species[c] == "Al") k.solvent_default = c;
@@ -925,7 +869,7 @@ int lmc_eval_jumps(const lmc_model *m, const uint8_t *d_occ, const int64_t *d_of
     if (n_replicas == 0) return LMC_OK;
     const auto &t = lmc::Upload(*m->m);
     Check(lmc::LaunchEvalJumps(t, d_occ, d_offset, d_ncell, d_vac, n_replicas, d_nb, d_ea, d_de,
-                               m->m->dev_err, S(stream), m->m->formulation == 1),
+                               m->m->dev_err, S(stream)),
           "eval jumps kernel");
     return LMC_OK;
   });
@@ -989,7 +933,7 @@ int lmc_eval_pair(const lmc_model *m, const uint8_t *d_occ, int32_t ncell, int64
       Check(hipMemcpy(nc, &ncell, sizeof(ncell), hipMemcpyHostToDevice), "hipMemcpy");
       const auto &t = lmc::Upload(*m->m);
       Check(lmc::LaunchEvalJumps(t, d_occ, buf, nc, buf + 1, 1, buf + 2, fb, fb + 12,
-                                 m->m->dev_err, nullptr, m->m->formulation == 1),
+                                 m->m->dev_err, nullptr),
             "eval jumps kernel");
       int64_t nbs[12];
       double r[24];
@@ -1287,6 +1231,7 @@ int lmc_kmc_create(const lmc_model *barrier, const lmc_model *energy, int32_t R,
     d.cs = DevCopy(cs);
     d.solute_mass = DevCopy(smass);
     d.flags = DevCopy(flags);
+    for (int32_t f : flags) d.options |= f;
     d.solvent = DevCopy(solvent);
     d.escaped = DevCopy(std::vector<int32_t>(R, 0));
     d.esc_time = DevCopy(std::vector<double>(R, 0.0));
@@ -2342,7 +2287,7 @@ int lmc_jump_samples(const lmc_model *m, const uint8_t *d_occ, const int64_t *d_
     double *ea = DevAlloc<double>(12 * static_cast<size_t>(n_replicas));
     const hipError_t e = lmc::LaunchEvalJumps(t, d_occ, d_offset, d_ncell, d_vac, n_replicas, nb,
                                               ea, d_de, m->m->dev_err, S(stream),
-                                              m->m->formulation == 1, d_env, d_ekra);
+                                              d_env, d_ekra);
     (void)hipStreamSynchronize(S(stream));
     DevFree(nb);
     DevFree(ea);

@@ -25,6 +25,15 @@ __device__ __forceinline__ XYZ ToXYZ(int64_t id, int n) {
   const int Zh = static_cast<int>(r - static_cast<int64_t>(Y) * n);
   return {X, Y, 2 * Zh + ((X + Y) & 1)};
 }
+// ToXYZ with 32-bit divisions: every box has 4 n^3 <= 4e9 < 2^32 sites (n <= 1000).
+__device__ __forceinline__ XYZ ToXYZ32(uint32_t id, uint32_t n) {
+  const uint32_t plane = 2u * n * n;
+  const uint32_t X = id / plane;
+  const uint32_t rest = id - X * plane;
+  const uint32_t Y = rest / n;
+  const uint32_t Zh = rest - Y * n;
+  return {static_cast<int>(X), static_cast<int>(Y), static_cast<int>(2 * Zh + ((X + Y) & 1))};
+}
 __device__ __forceinline__ int Wrap(int v, int m) {  // |v| < 2m
   v += v < 0 ? m : 0;
   v -= v >= m ? m : 0;

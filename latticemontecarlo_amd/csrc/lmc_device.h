@@ -19,8 +19,6 @@ constexpr int kMaxStateClusters = 512;
 constexpr int kMaxOrbitClusters = 768;
 // Cluster lists are padded to multiples of this (4 entries per lane of an event's 21 lanes).
 constexpr int kClusterPad = 84;
-// Copies for the wide kernel shape: 4 entries per lane of an event's 64 lanes.
-constexpr int kClusterPadWide = 256;
 constexpr int kMaxSiteClusters = 256;
 constexpr int kMaxW = 1024;  // w1 | w2 | w3 for S <= 6
 
@@ -31,7 +29,6 @@ struct KTables {
   const uint32_t *state;    // one-endpoint state clusters
   const uint32_t *mmm;
   const uint32_t *mm2;
-  const uint32_t *state_w, *mmm_w, *mm2_w;  // the same lists padded to kClusterPadWide
   const uint32_t *site_cl;
   const int32_t *site_off;  // [43]
   const double *w;          // theta/N by (label, codes): w1[S] | w2[3][S][S] | w3[4][S][S][S]
@@ -46,23 +43,21 @@ struct KTables {
   const int32_t *eci1;      // [S]
   const int32_t *eci2;      // [3][S][S]
   const int32_t *eci3;      // [4][S][S][S]
-  // Solvent-baseline formulation: for every (solvent s, migrating species M), the sums (dE, MMM
-  // logit, MM2 logit) of an environment that is all solvent (base), and per environment slot j
-  // the clusters containing j (CSR inc_off[3][61] -> inc, lists: state, MMM, MM2 forward and
-  // backward); a real environment adds value - value(all solvent) for each cluster touching a
-  // non-solvent slot, once (at its lowest such slot).
-  //   state entry: reduced weight-block byte offset [0:13] | j is the second other site [13]
-  //                | other site [14:20] (63 = none) | neighbour-endpoint side [31]
-  //   orbit entry: expanded-weight byte offset [0:16] | j takes the rank*8 role [16]
-  //                | other site [17:23] (63 = none)
-  const uint16_t *inc_off;  // [3][61]
-  const uint32_t *inc;
-  const double *base;       // [S][S][3]
-  int n_inc, solvent_default;
+  // Quadratic form of the jump sums (lmc_pairs.h): geometry, class offsets, values by
+  // [reference rank][migrating rank][row], and the all-reference sums pbase (dE, MMM, MM2 logit)
+  // by [reference rank][migrating rank][3].
+  const int32_t *site_pk;   // [134] signed byte offsets x | y << 8 | z << 16
+  const uint8_t *slot;      // [12][136]
+  const uint8_t *site_of;   // [12][60]
+  const uint32_t *site3;    // [60][4]
+  const uint8_t *order;     // [27][16]
+  const uint32_t *cls, *one, *dense;
+  const uint16_t *clsb, *oneb, *denseb;
+  const double *de, *la, *lb, *pbase;
+  int de_row, la_row, lb_row;
+  int solvent_default;
   uint64_t vac_shell_mask;  // env slots within 3NN of the vacancy
   int n_state, n_mmm, n_mm2, n_site, n_eci;  // n_mm2 counts forward + backward entries
-  int n_state_v;            // state entries of the vacancy endpoint (the rest: neighbour's)
-  int n_state_w, n_mmm_w, n_mm2_w;
   int v_slot, n_slot;
   int kind, S, ne, x_code, F1, F2, nw;
   int nwd, wrow;
@@ -115,6 +110,7 @@ struct KmcDev {
   int64_t *esc_site = nullptr;
   int64_t *disp = nullptr;      // [R][3] vacancy displacement, a/2 units
   double *com = nullptr;        // [R][3] solute centre-of-mass trajectory
+  int32_t options = 0;          // any replica has a flag set
   int32_t *error = nullptr;     // [1] first error code
   int64_t *prev_j = nullptr;    // [R] chain steps: the site the vacancy came from
   // optional atom tracking: atom id on every site (ids local to the replica) and map_shift
@@ -193,7 +189,7 @@ struct CmcDev {
 // (optional): [12 R] kinetically resolved barrier (E0 model: E0; quartic: Ea - dE/2).
 hipError_t LaunchEvalJumps(const KTables &t, const uint8_t *occ, const int64_t *off,
                            const int32_t *ncell, const int64_t *vac, int32_t R, int64_t *nb,
-                           double *ea, double *de, int32_t *err, hipStream_t s, bool solvent,
+                           double *ea, double *de, int32_t *err, hipStream_t s,
                            uint8_t *env_out = nullptr, double *ekra_out = nullptr);
 // The 12 jumps of a vacancy placed at each of sites[K] in the single occupancy occ (n^3 cells),
 // with site sub_site holding species sub_code instead (the ExitTime analysis' configuration);
@@ -201,8 +197,8 @@ hipError_t LaunchEvalJumps(const KTables &t, const uint8_t *occ, const int64_t *
 hipError_t LaunchVacancyScan(const KTables &t, const uint8_t *occ, int32_t n, int64_t sub_site,
                              int sub_code, const int64_t *sites, int32_t K, int64_t *nb,
                              double *ea, double *de, int32_t *err, hipStream_t s);
-// form: 0 dense (256 threads per replica), 1 solvent baseline, 2 dense wide shape (768 threads
-// per replica, one workgroup per CU), 3 second-order chain steps (KineticMcChainOmpi).
+// form: 0 or 1 one wave per replica, 2 wide shape (four waves per replica), 3 second-order chain
+// steps (KineticMcChainOmpi).
 hipError_t LaunchKmc(const KTables &t, const KmcDev &k, uint64_t steps, uint64_t trace_base,
                      hipStream_t s, int form);
 // Everything LaunchKmc sets up outside the stream (LDS plan, kernel attributes), so that its

@@ -1,292 +1,521 @@
-// gfx950 kernels of the vacancy-jump evaluation and the KineticMcFirst step.
+// gfx950 kernels of the vacancy-jump evaluation and of the residence-time steps
+// (KineticMcFirst, KineticMcChain), on the quadratic form of lmc_pairs.h (lmc_pair_device.h).
 //
-// Work mapping: one 256-thread workgroup per replica. Per KMC step
-//   1. gather   : the 12 jump environments (12 x 60 sites) -> LDS (bytes, from HBM/L2);
-//   2. clusters : per-cluster weights of dE (one-endpoint state clusters,
-//                 VacancyMigrationPredictorQuartic.cpp:112-166), of the barrier logit (MMM
-//                 orbit clusters, VacancyMigrationPredictorE0.cpp:128-151) and of the Ks logit
-//                 (MM2 forward + backward, VacancyMigrationPredictorQuartic.cpp:167-215), in one
-//                 of two exact formulations:
-//                   dense   - 21 lanes per jump sum every cluster (4 accumulators per lane);
-//                   solvent - per (solvent, migrating species) sums of an all-solvent
-//                             environment are precomputed; 16 lanes per jump add, for each
-//                             environment site holding another species, the changes of the
-//                             clusters it touches;
-//   3. events   : 12 lanes form dE, Ea and the rate exp(-Ea beta) in a fixed order and store
-//                 them at the jump's rank (neighbour ids ascending);
-//   4. select   : the 12 event lanes form the ordered cumulative probabilities (FP64); the lane
-//                 holding the chosen event advances the residence-time clock (Philox u1/u2
-//                 drawn by an idle lane during the gather) and applies the jump
-//                 (KineticMcFirstOmp.cpp:52-82, KineticMcAbstract.cpp:106-182).
-// Clusters containing both jump endpoints have the same species multiset before and after the
-// jump and are skipped. Tables live in dynamic LDS; the barrier weight tables go there when they
-// fit the workgroup's share of the CU's LDS, otherwise they are read from global memory.
+// KMC step of one replica:
+//   1. gather : species of the 134 sites around the vacancy; the loads are issued as soon as the
+//               previous step has chosen its jump, ahead of its bookkeeping;
+//   2. sums   : terms of the non-reference sites and of their near pairs, per event;
+//   3. events : lane l finishes event l % 16 (neighbour ids ascending): Ea, dE and the rate
+//               exp(-Ea beta) (JumpEvent.cpp:6-13);
+//   4. select : cumulative rates by a scan within each row of 16 lanes against u2 times the total
+//               (KineticMcFirstOmp.cpp:52-82, KineticMcAbstract.cpp:106-123), residence time
+//               with u1, jump (KineticMcAbstract.cpp:140-182). Philox numbers are drawn 64 steps
+//               at a time, one step per lane.
+// One wave makes the whole step (its replica then needs no barrier), or it shares step 2 with three
+// helper waves. Tables are copied to LDS once per launch; the value tables are read from global memory
+// when they do not fit.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <type_traits>
 
-#include "lmc_jump_device.h"
+#include "lmc_pair_device.h"
+#include "lmc_replica.h"
+#include "lmc_rng.h"
 
 namespace lmc {
 namespace {
 
-// One workgroup per replica r (vacancy vac[r] in occupancy occ + off[r] of ncell[r]^3 cells).
-// kScan: one workgroup per scanned site vac[r] of the single occupancy occ (scan_n^3 cells), with
-// the gather substitution `sub`.
-template <bool kSolvent, bool kBL, bool kScan>
-__global__ __launch_bounds__(kThreads) void EvalJumpsKernel(KTables t, DynLayout lay,
-                                                            const uint8_t *occ,
-                                                            const int64_t *off,
-                                                            const int32_t *ncell,
-                                                            const int64_t *vac, int64_t *nb,
-                                                            double *ea, double *de, int32_t *err,
-                                                            uint8_t *env_out, double *ekra_out,
-                                                            int scan_n, GatherSub sub) {
-  __shared__ JumpLds L;
-  extern __shared__ char dyn[];
-  const int r = blockIdx.x;
-  const int n = kScan ? scan_n : ncell[r];
-  if (!ValidSite(n, vac[r])) {
-    if (threadIdx.x == 0) atomicOr(err, 8);
-    return;
-  }
-  const Tabs T =
-      LoadJumpTables<kSolvent, kBL>(t, L, dyn, lay, threadIdx.x, kThreads, threadIdx.x, kThreads);
+// Waves per SIMD that the scheduler aims at. Left to itself it keeps registers for more waves than the
+// LDS lets in and makes every list batch a chain of single loads (a wave has its SIMD almost alone).
+#define LMC_WAVES(lo, hi) __attribute__((amdgpu_waves_per_eu(lo, hi)))
+
+constexpr int kEvalWaves = 8;  // waves of an evaluation workgroup
+constexpr int kTeam = 4;       // waves of a replica in the team shape
+
+// Dynamic LDS of a workgroup (byte offsets): value tables, replicas' and waves' working sets.
+struct KmcLayout {
+  PairLayout tab;
+  int team, wave, extra, bytes;
+};
+
+__device__ __forceinline__ int WaveIndex() {
+  return __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+}
+
+// The 12 jumps of each replica r (vacancy vac[r] in occupancy occ + off[r] of ncell[r]^3 cells), or
+// with kScan of a vacancy placed at each site vac[r] of the single occupancy occ (scan_n^3 cells)
+// whose site sub_site holds sub_code. One wave per replica or site; the workgroups stride over
+// them, so that one copy of the tables serves many.
+template <bool kQ, bool kTab, bool kScan>
+__global__ __launch_bounds__(64 * kEvalWaves) LMC_WAVES(1, 2) void EvalJumpsKernel(
+    KTables t, KmcLayout lay, const uint8_t *occ, const int64_t *off, const int32_t *ncell,
+    const int64_t *vac, int32_t R, int64_t *nb, double *ea, double *de, int32_t *err,
+    uint8_t *env_out, double *ekra_out, int scan_n, int64_t sub_site, int sub_code) {
+  __shared__ PairShared<kQ> G;
+  extern __shared__ __align__(16) char dyn[];
+  const int lane = LaneId(), wave = WaveIndex();
+  const PairTab T =
+      LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, t.solvent_default, threadIdx.x, 64 * kEvalWaves);
   __syncthreads();
-  EvaluateJumps<kSolvent, kScan>(t, L, T, kScan ? occ : occ + off[r], n, ToXYZ(vac[r], n),
-                                 t.solvent_default, 0.0, err, threadIdx.x, nullptr, sub);
-  const int k = threadIdx.x;
-  if (k < 12) {
-    const int64_t o = static_cast<int64_t>(r) * 12 + k;
-    nb[o] = L.snb[k];
-    ea[o] = L.ea[k];
-    de[o] = L.de[k];
-    if (ekra_out) ekra_out[o] = L.ekra[k];
-  }
-  if (env_out) {  // environment rows of the events in rank order (60 slot codes, zero padded)
-    for (int i = threadIdx.x; i < 12 * 64; i += kThreads) {
-      const int q = i >> 6, j = i & 63;
-      env_out[(static_cast<int64_t>(r) * 12 + q) * 64 + j] = j < kEnvSlots ? L.env[L.dir[q]][j] : 0;
+  TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[wave];
+  WaveLds &W = reinterpret_cast<WaveLds *>(dyn + lay.wave)[wave];
+  const LaneSites ls = LoadSites(t, 0);
+  const ExpConst E = MakeExpConst();
+  for (int64_t r = static_cast<int64_t>(blockIdx.x) * kEvalWaves + wave; r < R;
+       r += static_cast<int64_t>(gridDim.x) * kEvalWaves) {
+    const int n = kScan ? scan_n : ncell[r];
+    const int64_t site = vac[r];
+    if (!ValidSite(n, site)) {
+      if (lane == 0) atomicOr(err, 8);
+      continue;
     }
-  }
-}
-
-// Replica r's state into LDS (one thread).
-__device__ void LoadReplica(const KmcDev &k, int r, int n, ReplicaLds &Q) {
-  Q.steps = k.steps[r];
-  Q.max_steps = k.max_steps[r];
-  Q.seed = k.seed[r];
-  Q.rid = k.rid[r];
-  Q.time = k.time[r];
-  Q.energy = k.energy[r];
-  Q.abse = k.abs_energy[r];
-  Q.T = k.temp[r];
-  Q.cv = k.cv[r];
-  Q.cs = k.cs[r];
-  Q.smass = k.solute_mass[r];
-  Q.vac = k.vac[r];
-  Q.flags = k.flags[r];
-  Q.esc = k.escaped[r];
-  Q.solvent = k.solvent[r];
-  for (int a = 0; a < 3; ++a) {
-    Q.disp[a] = k.disp[3 * r + a];
-    Q.com[a] = k.com[3 * r + a];
-  }
-  Q.done = (Q.steps > Q.max_steps || Q.esc || !ValidSite(n, Q.vac)) ? 1 : 0;
-  Q.beta = 1.0 / kBoltzmann / Q.T;
-  SetVacancyXYZ(Q, n);
-}
-
-// Replica r's state back to HBM (one thread).
-__device__ void StoreReplica(const KmcDev &k, int r, const ReplicaLds &Q) {
-  k.steps[r] = Q.steps;
-  k.time[r] = Q.time;
-  k.energy[r] = Q.energy;
-  k.abs_energy[r] = Q.abse;
-  k.temp[r] = Q.T;
-  k.vac[r] = Q.vac;
-  k.escaped[r] = Q.esc;
-  for (int a = 0; a < 3; ++a) {
-    k.disp[3 * r + a] = Q.disp[a];
-    k.com[3 * r + a] = Q.com[a];
-  }
-}
-
-// UpdateTemperature (KineticMcAbstract.cpp:45-50), before any lane reads beta.
-__device__ __forceinline__ void UpdateTemperature(const KmcDev &k, ReplicaLds &Q, int tid) {
-  if (k.n_tt > 0) {
-    if (tid == 0) {
-      Q.T = ScheduleTemperature(k.tt_time, k.tt_temp, k.n_tt, Q.time);
-      Q.beta = 1.0 / kBoltzmann / Q.T;
+    const uint8_t *o = kScan ? occ : occ + off[r];
+    const XYZ c = n <= 1000 ? ToXYZ32(static_cast<uint32_t>(site), static_cast<uint32_t>(n)) : ToXYZ(site, n);
+    Around<uint64_t> a;
+    GatherAround(ls, o, n, c, a);
+    if (kScan) Substitute(a, static_cast<uint64_t>(sub_site), sub_code);
+    const int dir = EventDirection(G, c, n);
+    const bool bad = CheckCodes(t, a, dir, err);
+    const int M = Bpermute(dir, a.code[0]);
+    const EventConst ec = LoadConst(t, G, M);
+    const int K = ListSites<kQ>(t, G, T, S, ls, a);
+    const PairSums s = PairTerms<kQ, 1>(G, T, S, W, ls, K, MakeRow<kQ>(t, T, dir, M), 0);
+    const EventValue e = FinishEvent<kQ>(E, ec, s, bad);
+    const uint64_t id = Bpermute64(dir, a.id[0]);
+    if (lane < 12) {
+      if (EventError(e)) atomicOr(err, 1);
+      const int64_t w = r * 12 + lane;
+      nb[w] = static_cast<int64_t>(id);
+      ea[w] = e.ea;
+      de[w] = e.de;
+      if (ekra_out) ekra_out[w] = e.ekra;
     }
-    __syncthreads();
-  }
-}
-
-// Persistent KMC: one 256-thread workgroup per replica, up to four per CU.
-template <bool kSolvent, bool kBL, bool kRecord>
-__global__ __launch_bounds__(kThreads, 4) void KmcKernel(KTables t, DynLayout lay, KmcDev k,
-                                                      uint64_t nsteps, uint64_t trace_base) {
-  __shared__ JumpLds L;
-  __shared__ ReplicaLds Q;
-  extern __shared__ char dyn[];
-  const int r = blockIdx.x;
-  const int tid = threadIdx.x;
-  const Tabs T = LoadJumpTables<kSolvent, kBL>(t, L, dyn, lay, tid, kThreads, tid, kThreads);
-  uint8_t *occ = k.occ + k.off[r];
-  const int n = k.ncell[r];
-  if (tid == 0) LoadReplica(k, r, n, Q);
-  __syncthreads();
-  const int sv = Q.solvent;
-  for (uint64_t it = 0; it < nsteps; ++it) {
-    if (Q.done) break;
-    RotatePriority(it);
-    UpdateTemperature(k, Q, tid);
-    // the selection reads the events in wave 0, which finished them (dense shape)
-    EvaluateJumps<kSolvent, false, false>(t, L, T, occ, n, VacancyXYZ(Q), sv, Q.beta, k.error,
-                                          tid, &Q);
-    SelectAndApply<kRecord>(t, k, L, Q, occ, r, trace_base + it, tid);
-    __syncthreads();
-  }
-  if (tid == 0) StoreReplica(k, r, Q);
-}
-
-// Persistent KMC, wide shape: one 768-thread workgroup per replica (wave k evaluates event k),
-// for batches of at most one replica per CU, where a step's latency sets the rate.
-template <bool kBL, bool kRecord>
-__global__ __launch_bounds__(kWideThreads, 1) void KmcWideKernel(KTables t, DynLayout lay,
-                                                                 KmcDev k, uint64_t nsteps,
-                                                                 uint64_t trace_base) {
-  __shared__ JumpLds L;
-  __shared__ ReplicaLds Q;
-  extern __shared__ char dyn[];
-  const int r = blockIdx.x;
-  const int tid = threadIdx.x;
-  const Tabs T =
-      LoadJumpTables<false, kBL, true>(t, L, dyn, lay, tid, kWideThreads, tid, kWideThreads);
-  uint8_t *occ = k.occ + k.off[r];
-  const int n = k.ncell[r];
-  if (tid == 0) LoadReplica(k, r, n, Q);
-  __syncthreads();
-  for (uint64_t it = 0; it < nsteps; ++it) {
-    if (Q.done) break;
-    UpdateTemperature(k, Q, tid);
-    {
-      Gathered<kWideThreads> G;
-      GatherIssue<kWideThreads>(L, occ, n, VacancyXYZ(Q), tid, G);
-      DrawSteps<kWideThreads>(L, Q, tid);
-      GatherStore<kWideThreads>(t, L, k.error, tid, G);
-    }
-    __syncthreads();
-    WideSums(t, L, T, tid);
-    __syncthreads();
-    if (tid < 64) {  // wave 0 finishes the 12 events, then selects
-      FinishFromSums(t, L, Q.beta, k.error, tid);
+    if (env_out) {  // environment rows of the events in rank order (60 slot codes, zero padded)
+      WaveFence();
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        if (lane + 64 * u < kPairSites) S.code[lane + 64 * u] = static_cast<uint16_t>(a.code[u]);
+      if (lane == 0) S.code[kPairSites] = static_cast<uint16_t>(t.x_code);
+      WaveFence();
+      for (int q = 0; q < 12; ++q) {
+        const int d = ReadLaneInt(dir, q);
+        env_out[(r * 12 + q) * 64 + lane] = lane < kEnvSlots ? static_cast<uint8_t>(S.code[t.site_of[d * kEnvSlots + lane]]) : 0;
+      }
       WaveFence();
     }
-    SelectAndApply<kRecord>(t, k, L, Q, occ, r, trace_base + it, tid);
-    __syncthreads();
   }
-  if (tid == 0) StoreReplica(k, r, Q);
 }
 
-// Persistent second-order (chain) KMC, KineticMcChainOmpi: one 256-thread workgroup per replica.
-// Each step evaluates the 12 jumps out of every first neighbour i of the vacancy k in the
-// configuration after the jump k -> i (12 passes of the dense evaluation: vacancy at i, site k
-// holding i's species), then lane 0 forms the second-order probabilities and time and jumps.
-template <bool kBL, bool kRecord>
-__global__ __launch_bounds__(kThreads, 4) void KmcChainKernel(KTables t, DynLayout lay, KmcDev k,
-                                                           uint64_t nsteps, uint64_t trace_base) {
-  __shared__ JumpLds L;
-  __shared__ ReplicaLds Q;
-  __shared__ ChainLds C;
-  extern __shared__ char dyn[];
-  const int r = blockIdx.x;
-  const int tid = threadIdx.x;
-  const Tabs T = LoadJumpTables<false, kBL>(t, L, dyn, lay, tid, kThreads, tid, kThreads);
+// Uniforms of the steps of one replica: lane l holds those of step base + l.
+struct StepDraws {
+  double u2, log_u1;
+  uint64_t base;
+  bool ok;
+};
+// u2 and log(u1) of step Q.steps; every 64 steps the wave draws the next 64.
+__device__ __forceinline__ void DrawStep(StepDraws &d, const ReplicaLds &Q, double &u2, double &log_u1) {
+  if (!d.ok || Q.steps - d.base >= 64) {  // uniform
+    const U4 u = Philox4x32_10(Q.seed, Q.steps + LaneId(), Q.rid, 0u);
+    d.u2 = UnitOpenRight(Join64(u.z, u.w));
+    d.log_u1 = log(UnitOpenLeft(Join64(u.x, u.y)));
+    d.base = Q.steps;
+    d.ok = true;
+  }
+  const int i = __builtin_amdgcn_readfirstlane(static_cast<int>(Q.steps - d.base));
+  u2 = ReadLane(d.u2, i);
+  log_u1 = ReadLane(d.log_u1, i);
+}
+
+// UpdateTemperature (KineticMcAbstract.cpp:45-50) and the RateCorrector factor at that temperature
+// (RateCorrector.hpp:17-24), formed again only when the temperature has changed.
+struct StepClock {
+  double corr, corr_T;
+};
+__device__ __forceinline__ void UpdateTemperature(const KmcDev &k, ReplicaLds &Q, StepClock &C) {
+  if (k.n_tt > 0) {
+    Q.T = ScheduleTemperature(k.tt_time, k.tt_temp, k.n_tt, Q.time);
+    Q.beta = 1.0 / kBoltzmann / Q.T;
+  }
+  if ((Q.flags & 1) && Q.T != C.corr_T) {
+    C.corr = Q.cv / (1.64 * exp(-(0.66 / kBoltzmann / Q.T - 0.7))) / (1 - 13 * Q.cs);
+    C.corr_T = Q.T;
+  }
+}
+
+// A chosen jump: target site and its coordinates, the move (a/2 units), migrating species, barrier,
+// energy change.
+struct Jump {
+  uint32_t site;
+  XYZ to, move;
+  int mig;
+  double ea, de;
+};
+
+// The jumps of the events as their lanes hold them, for one readlane each: x | y << 16, and
+// z | packed move << 16 (two bits per component, plus one).
+struct EventTargets {
+  uint32_t site, xy, zm;
+};
+__device__ __forceinline__ EventTargets MakeTargets(const LaneSites &ls, const Around<uint32_t> &a, int dir) {
+  return {static_cast<uint32_t>(Bpermute(dir, static_cast<int>(a.id[0]))),
+          static_cast<uint32_t>(Bpermute(dir, static_cast<int>(a.near.x | (a.near.y << 16)))),
+          static_cast<uint32_t>(Bpermute(dir, static_cast<int>(a.near.z | ls.move)))};
+}
+__device__ __forceinline__ Jump TakeJump(const EventTargets &e, int mig, double ea, double de, int sel) {
+  const uint32_t xy = static_cast<uint32_t>(ReadLaneInt(static_cast<int>(e.xy), sel));
+  const uint32_t zm = static_cast<uint32_t>(ReadLaneInt(static_cast<int>(e.zm), sel));
+  Jump j;
+  j.site = static_cast<uint32_t>(ReadLaneInt(static_cast<int>(e.site), sel));
+  j.to = {static_cast<int>(xy & 0xFFFFu), static_cast<int>(xy >> 16), static_cast<int>(zm & 0xFFFFu)};
+  j.move = {static_cast<int>((zm >> 16) & 3u) - 1, static_cast<int>((zm >> 18) & 3u) - 1,
+            static_cast<int>((zm >> 20) & 3u) - 1};
+  j.mig = ReadLaneInt(mig, sel);
+  j.ea = ea;
+  j.de = de;
+  return j;
+}
+
+// The first half of a step's end, before the next gather: what depends on the state before the jump
+// (escape record, log, atoms; kFull), then the occupancy (kStore) and the vacancy's new position. Every
+// lane holds Q; lane 0 keeps the records.
+template <bool kFull, bool kStore = true>
+__device__ __forceinline__ void ApplyJump(const KTables &t, const KmcDev &k, ReplicaLds &Q, uint8_t *occ,
+                                          int r, const Jump &j, bool escaped) {
+  if constexpr (kFull) {
+    const bool writer = kStore && LaneId() == 0;
+    if (escaped) {
+      if (writer && k.esc_time) {
+        k.esc_time[r] = Q.time;
+        k.esc_step[r] = Q.steps;
+        k.esc_site[r] = Q.vac;
+      }
+      Q.esc = 1;
+      Q.steps = Q.max_steps + 1;
+    }
+    if (writer && k.log_every && LogDue(Q.steps, k.log_every))
+      LogStep(k, Q, r, static_cast<int64_t>(j.site), j.ea, j.de);
+    if (writer && k.atom) {  // the vacancy at Q.vac is the lhs of the reference's jump pair
+      const int64_t o = k.off[r];
+      const int h = Q.m2 >> 1;
+      AtomJump(k.atom + o, k.shift + 3 * o, Q.vac, static_cast<int64_t>(j.site), ImageChange(j.to.X - Q.vx, h),
+               ImageChange(j.to.Y - Q.vy, h), ImageChange(j.to.Z - Q.vz, h));
+    }
+  }
+  if constexpr (kStore) {
+    // Config::LatticeJump (Config.cpp:431-456): the two bytes in one store of all lanes, without a
+    // branch
+    const bool odd = (LaneId() & 1) != 0;
+    occ[odd ? j.site : static_cast<uint32_t>(Q.vac)] = static_cast<uint8_t>(odd ? t.x_code : j.mig);
+  }
+  Q.vx = j.to.X;
+  Q.vy = j.to.Y;
+  Q.vz = j.to.Z;
+  Q.vac = static_cast<int64_t>(j.site);
+}
+
+// The second half, under the next gather's loads: clock, energies, trace, displacements
+// (KineticMcAbstract.cpp:147-181).
+template <bool kFull>
+__device__ __forceinline__ void FinishStep(const KmcDev &k, ReplicaLds &Q, int r, uint64_t trace_index,
+                                           const Jump &j, double dt, XYZ &moved) {
+  const XYZ &d = j.move;
+  if constexpr (kFull) {
+    if (trace_index < k.trace_cap && LaneId() == 0) {
+      const uint64_t o = static_cast<uint64_t>(r) * k.trace_cap + trace_index;
+      k.tr_sel[o] = static_cast<int64_t>(j.site);
+      k.tr_ea[o] = j.ea;
+      k.tr_de[o] = j.de;
+      k.tr_time[o] = Q.time + dt;
+    }
+    if ((Q.flags & 4) && j.mig != Q.solvent) {  // solute COM (KineticMcAbstract.cpp:163-177)
+      const double wgt = k.mass[j.mig] / Q.smass;
+      Q.com[0] -= d.X * kHalfLattice * wgt;
+      Q.com[1] -= d.Y * kHalfLattice * wgt;
+      Q.com[2] -= d.Z * kHalfLattice * wgt;
+    }
+  }
+  Q.time += dt;
+  Q.energy += j.de;
+  Q.abse += j.de;
+  moved.X += d.X;
+  moved.Y += d.Y;
+  moved.Z += d.Z;
+  Q.steps += 1;
+  if (Q.steps > Q.max_steps || (kFull && Q.esc)) Q.done = 1;
+}
+
+// IsEscaped (KineticMcAbstract.cpp:192-223): the 42 sites of the vacancy's three shells (sites
+// 0 .. 41) hold the solvent.
+__device__ __forceinline__ bool Escaped(const ReplicaLds &Q, int code0) {
+  return (Q.flags & 2) && __ballot(LaneId() < 42 && code0 != Q.solvent) == 0;
+}
+
+// Event of the ordered cumulative probabilities: the first one whose sum reaches u2 of the total,
+// else the last (`cum` on lanes 0 .. 10 of a row).
+__device__ __forceinline__ int SelectEvent(double cum, double goal) {
+  const uint64_t below = __ballot(LaneId() < 11 && cum < goal);
+  return __builtin_ctzll(~below);
+}
+
+// Exchange area of a team: events' direction and migrating species, listed sites, partial sums.
+struct TeamExchange {
+  double part[kTeam][16][3];
+  int info[16];
+  int K;
+};
+
+// Persistent KMC. kWaves 1: `group` replicas per workgroup, one wave each; the waves never meet after
+// the table copy. kWaves kTeam: one replica per workgroup, a leading wave makes the step and three
+// helpers share its sums, with two barriers per step.
+// kFull: options, schedule, trace, log and atoms are compiled in.
+template <bool kQ, bool kTab, int kWaves, bool kFull>
+__global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) void KmcKernel(
+    KTables t, KmcLayout lay, KmcDev k, int group, int nsteps, uint64_t trace_base) {
+  __shared__ PairShared<kQ> G;
+  extern __shared__ __align__(16) char dyn[];
+  const int lane = LaneId(), wave = WaveIndex();
+  const int first = blockIdx.x * group, mine = kWaves == 1 ? wave : 0, wv = kWaves == 1 ? 0 : wave;
+  const PairTab T =
+      LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, k.solvent[first], threadIdx.x, blockDim.x);
+  TeamExchange &X = *reinterpret_cast<TeamExchange *>(dyn + lay.extra);
+  __syncthreads();
+  const int r = first + mine;
+  if (mine >= group || r >= k.R) return;
+  TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[mine];
+  WaveLds &W = reinterpret_cast<WaveLds *>(dyn + lay.wave)[wave];
+  const LaneSites ls = LoadSites(t, wv);
+  const ExpConst E = MakeExpConst();
   uint8_t *occ = k.occ + k.off[r];
   const int n = k.ncell[r];
-  if (tid == 0) {
-    LoadReplica(k, r, n, Q);
-    C.prev = k.prev_j[r];
-    L.bad = 0;
+  ReplicaLds Q;
+  LoadReplica(k, r, n, Q);
+  StepDraws draws{0.0, 0.0, 0, false};
+  XYZ moved{0, 0, 0};  // displacement of this launch
+  StepClock clock{1.0, 0.0};
+  Around<uint32_t> a;
+  double u2 = 0.0, log_u1 = 0.0;
+  int dir = 0;
+  bool error = false;
+  if (wv == 0 && !Q.done) {
+    GatherAround(ls, occ, n, VacancyXYZ(Q), a);
+    dir = EventDirection(G, VacancyXYZ(Q), n);
+    DrawStep(draws, Q, u2, log_u1);
   }
-  __syncthreads();
-  const int sv = Q.solvent;
-  for (uint64_t it = 0; it < nsteps; ++it) {
-    if (Q.done) break;
-    RotatePriority(it);
-    UpdateTemperature(k, Q, tid);
-    ChainNeighbours(t, L, C, Q, occ, n, tid);
-    if (tid == kThreads - 1) DrawStep(L, Q);
-    __syncthreads();
-    for (int i = 0; i < 12; ++i) {
-      int dx, dy, dz;
-      Unpack16(C.soff[i], dx, dy, dz);
-      const XYZ vi{Wrap(Q.vx + dx, Q.m2), Wrap(Q.vy + dy, Q.m2), Wrap(Q.vz + dz, Q.m2)};
-      EvaluateJumps<false, true>(t, L, T, occ, n, vi, sv, Q.beta, k.error, tid, nullptr,
-                                 GatherSub{Q.vac, C.sm[i]});
-      if (tid == 0) ChainPass(L, C, Q, i);
-      __syncthreads();
+  for (int it = 0; it < nsteps; ++it) {
+    if (wv == 0 && Q.done && kWaves == 1) break;
+    EventConst ec;
+    EventRow row;
+    EventTargets to;
+    bool bad = false;
+    int K = -1;  // team: the replica has ended
+    if (wv == 0 && !Q.done) {
+      if (kFull) UpdateTemperature(k, Q, clock);
+      bad = CheckCodes(t, a, dir, k.error);
+      const int M = Bpermute(dir, a.code[0]);
+      to = MakeTargets(ls, a, dir);
+      row = MakeRow<kQ>(t, T, dir, M);
+      ec = LoadConst(t, G, M);
+      K = ListSites<kQ>(t, G, T, S, ls, a);
     }
-    if (tid == 0) ChainSelectAndApply<kRecord>(t, k, L, C, Q, occ, n, r, trace_base + it);
-    __syncthreads();
+    PairSums s;
+    if constexpr (kWaves == 1) {
+      s = PairTerms<kQ, 1>(G, T, S, W, ls, K, row, 0);
+    } else {
+      if (wv == 0) {
+        if (lane < 16) X.info[lane] = row.dir | (row.M << 8);
+        if (lane == 0) X.K = K;
+      }
+      __syncthreads();
+      K = __builtin_amdgcn_readfirstlane(X.K);
+      if (K < 0) break;  // uniform over the workgroup
+      if (wv != 0) {
+        const int i = X.info[lane & 15];
+        row = MakeRow<kQ>(t, T, i & 255, i >> 8);
+      }
+      s = PairTerms<kQ, kWaves>(G, T, S, W, ls, K, row, wv);
+      if (lane < 16) {
+        double *p = X.part[wv][lane];
+        p[0] = s.de;
+        p[1] = s.la;
+        if (kQ) p[2] = s.lb;
+      }
+      __syncthreads();
+      if (wv != 0) continue;
+      const double *p = X.part[0][lane & 15];
+      s = {p[0], p[1], kQ ? p[2] : 0.0};
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) {
+        s.de += p[48 * w];
+        s.la += p[48 * w + 1];
+        if (kQ) s.lb += p[48 * w + 2];
+      }
+    }
+    const EventValue e = FinishEvent<kQ>(E, ec, s, bad);
+    error = error || EventError(e);
+    const double cum = RowScan((lane & 15) < 12 ? Exp(E, -e.ea * Q.beta) : 0.0);
+    const double total = ReadLane(cum, 11);
+    const int sel = SelectEvent(cum, u2 * total);
+    const Jump j = TakeJump(to, row.M, kFull ? ReadLane(e.ea, sel) : 0.0, ReadLane(e.de, sel), sel);
+    ApplyJump<kFull>(t, k, Q, occ, r, j, kFull && Escaped(Q, a.code[0]));
+    WaveFence();
+    GatherAround(ls, occ, n, VacancyXYZ(Q), a);
+    dir = EventDirection(G, VacancyXYZ(Q), n);
+    double dt = -log_u1 / (total * kPrefactor);
+    if (kFull && (Q.flags & 1)) dt *= clock.corr;
+    FinishStep<kFull>(k, Q, r, trace_base + it, j, dt, moved);
+    DrawStep(draws, Q, u2, log_u1);
   }
-  if (tid == 0) {
-    StoreReplica(k, r, Q);
-    k.prev_j[r] = C.prev;
+  if (wv != 0) return;
+  if (__ballot(error) && lane == 0) atomicOr(k.error, 1);
+  if (lane == 0) StoreReplica<kFull>(k, r, Q, moved);
+}
+
+// Persistent second-order (chain) KMC, KineticMcChainOmpi (KineticMcChainOmpi.cpp:56-151). Each step
+// evaluates the 12 jumps out of every first neighbour i of the vacancy k in the configuration after
+// the jump k -> i (12 passes: the vacancy at i, site k holding i's species), takes k -> i as the
+// reverse of i -> k, and forms the second-order probabilities and the time with lane r on neighbour
+// r (id order). kWaves 1: one wave makes all passes of a replica. kWaves kTeam: four waves hold the
+// replica's state and make every fourth pass; one barrier per step exchanges their results, wave 0
+// writes.
+template <bool kQ, bool kTab, int kWaves, bool kFull>
+__global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) void KmcChainKernel(
+    KTables t, KmcLayout lay, KmcDev k, int group, int nsteps, uint64_t trace_base) {
+  __shared__ PairShared<kQ> G;
+  extern __shared__ __align__(16) char dyn[];
+  const int lane = LaneId(), wave = WaveIndex();
+  const int first = blockIdx.x * group;
+  const PairTab T =
+      LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, k.solvent[first], threadIdx.x, blockDim.x);
+  __syncthreads();
+  const int r = kWaves == 1 ? first + wave : first;
+  if (kWaves == 1 && (wave >= group || r >= k.R)) return;
+  const int wv = kWaves == 1 ? 0 : wave;
+  TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[wave];
+  WaveLds &W = reinterpret_cast<WaveLds *>(dyn + lay.wave)[wave];
+  // results of the passes, [step parity][neighbour rank][total rate, Ea, dE]
+  double *res = reinterpret_cast<double *>(dyn + lay.extra) + (kWaves == 1 ? wave * 72 : 0);
+  const LaneSites ls = LoadSites(t, 0);
+  const ExpConst E = MakeExpConst();
+  uint8_t *occ = k.occ + k.off[r];
+  const int n = k.ncell[r];
+  ReplicaLds Q;
+  LoadReplica(k, r, n, Q);
+  uint32_t prev = static_cast<uint32_t>(k.prev_j[r]);
+  int prev_mig = -1;  // species the last jump left at prev
+  bool error = false;
+  StepDraws draws{0.0, 0.0, 0, false};
+  XYZ moved{0, 0, 0};  // displacement of this launch
+  StepClock clock{1.0, 0.0};
+  for (int it = 0; it < nsteps; ++it) {
+    if (Q.done) break;
+    if (kFull) UpdateTemperature(k, Q, clock);
+    const XYZ c = VacancyXYZ(Q);
+    Around<uint32_t> a;
+    GatherAround(ls, occ, n, c, a);
+    // the other waves may read before wave 0 has stored the jump
+    if (kWaves > 1 && prev_mig >= 0) Substitute(a, prev, prev_mig);
+    double u2, log_u1;
+    DrawStep(draws, Q, u2, log_u1);
+    const int dir = EventDirection(G, c, n);
+    (void)CheckCodes(t, a, dir, k.error);
+    double *x = res + (it & 1) * 36;
+    for (int i = wv; i < 12; i += kWaves) {
+      const int di = ReadLaneInt(dir, i);
+      const XYZ ci = WrapAdd(c, PackedXYZ(ReadLaneInt(ls.pk[0], di)), Q.m2);
+      Around<uint32_t> b;
+      GatherAround(ls, occ, n, ci, b);
+      if (kWaves > 1 && prev_mig >= 0) Substitute(b, prev, prev_mig);
+      Substitute(b, static_cast<uint32_t>(Q.vac), ReadLaneInt(a.code[0], di));
+      const int dirb = EventDirection(G, ci, n);
+      const bool bad = CheckCodes(t, b, dirb, k.error);
+      const int M = Bpermute(dirb, b.code[0]);
+      const EventConst ec = LoadConst(t, G, M);
+      const int K = ListSites<kQ>(t, G, T, S, ls, b);
+      const PairSums s = PairTerms<kQ, 1>(G, T, S, W, ls, K, MakeRow<kQ>(t, T, dirb, M), 0);
+      const EventValue e = FinishEvent<kQ>(E, ec, s, bad);
+      error = error || EventError(e);
+      const double cum = RowScan((lane & 15) < 12 ? Exp(E, -e.ea * Q.beta) : 0.0);
+      // the jump back to k has the opposite direction, 11 - di
+      const int back = __builtin_ctzll(__ballot(lane < 12 && dirb == 11 - di));
+      const double ea = ReadLane(e.ea, back), de = ReadLane(e.de, back), tot = ReadLane(cum, 11);
+      if (lane == 0) {
+        x[3 * i] = tot;
+        x[3 * i + 1] = ea;
+        x[3 * i + 2] = de;
+      }
+    }
+    if (kWaves > 1) __syncthreads();
+    else WaveFence();
+    // lane i: the event k -> i as the reverse of i -> k (KineticMcChainOmpi.cpp:56-91,
+    // JumpEvent.cpp:25-30,51-54)
+    const int ev = (lane & 15) < 12 ? lane & 15 : 11;
+    const bool on = (lane & 15) < 12;
+    const double total_i = x[3 * ev], barrier = x[3 * ev + 1] - x[3 * ev + 2], de = -x[3 * ev + 2];
+    const double rate = on ? Exp(E, -barrier * Q.beta) : 0.0;
+    const double p_ik = Exp(E, (de - barrier) * Q.beta) / total_i;
+    const uint32_t sid = static_cast<uint32_t>(Bpermute(dir, static_cast<int>(a.id[0])));
+    const double total = ReadLane(RowScan(rate), 11);
+    const double t1 = 1 / total / kPrefactor, ti = 1 / total_i / kPrefactor;
+    const double p_ki = rate / total;
+    const double bb = on ? p_ki * p_ik : 0.0, b1 = on ? p_ki * (1 - p_ik) : 0.0;
+    const bool was = on && sid == prev;
+    auto row_total = [](double v) { return ReadLane(RowScan(v), 11); };
+    const double g = row_total(bb), gb = row_total(b1);
+    const double og = row_total(was ? 0.0 : bb), ob = row_total(was ? 0.0 : b1);
+    const double al = row_total(was ? b1 : 0.0), ga = row_total(was ? p_ki : 0.0);
+    const double tb = on ? (t1 + ti) * bb : 0.0;
+    const double ts = row_total(tb) / g, ts_j = row_total(was ? 0.0 : tb) / og;
+    const double inv = 1 / (1 - ga);
+    double dt = inv * (ob * t1 + og * (ts_j + t1 + g / gb * ts));
+    const double prob = was ? inv * (og / gb) * al : inv * (1 + og / gb) * b1;
+    const double cum = RowScan(prob);
+    const int sel = SelectEvent(cum, u2);
+    const Jump j = TakeJump(MakeTargets(ls, a, dir), Bpermute(dir, a.code[0]), ReadLane(barrier, sel),
+                            ReadLane(de, sel), sel);
+    prev = static_cast<uint32_t>(Q.vac);
+    prev_mig = j.mig;
+    const bool escaped = kFull && Escaped(Q, a.code[0]);
+    if (wv == 0) ApplyJump<kFull>(t, k, Q, occ, r, j, escaped);
+    else ApplyJump<kFull, false>(t, k, Q, occ, r, j, escaped);
+    WaveFence();
+    if (kFull && (Q.flags & 1)) dt *= clock.corr;
+    if (wv == 0) FinishStep<kFull>(k, Q, r, trace_base + it, j, dt, moved);
+    else FinishStep<kFull>(k, Q, r, ~0ull, j, dt, moved);
+  }
+  if (wv != 0) return;
+  if (__ballot(error) && lane == 0) atomicOr(k.error, 1);
+  if (lane == 0) {
+    StoreReplica<kFull>(k, r, Q, moved);
+    k.prev_j[r] = static_cast<int64_t>(prev);
   }
 }
 
-// Dynamic LDS plan: weight tables go to LDS while the workgroup stays within its share of the
-// CU's LDS (up to 4 resident workgroups per CU when the batch fills the chip).
-// form: 0 dense, 1 solvent baseline, 2 dense wide shape (one workgroup per CU), 3 chain steps.
-DynLayout PlanLds(const KTables &t, int32_t R, int form) {
-  const bool solvent = form == 1;
+// Dynamic LDS plan for workgroups of `teams` replicas and `waves` waves: the value tables go to LDS
+// when per_cu workgroups then still fit a CU.
+KmcLayout PlanLds(const KTables &t, int teams, int waves, size_t extra, int per_cu) {
   const DeviceLimits &dl = CurrentDeviceLimits();
-  const int cus = dl.cus;
-  const size_t lds_cu = dl.lds_cu, lds_block = dl.lds_block;
-  const int per_cu = form == 2 ? 1 : std::min(4, std::max(1, (R + cus - 1) / cus));
-  const size_t stat = sizeof(JumpLds) + sizeof(ReplicaLds) + (form == 3 ? sizeof(ChainLds) : 0) + 256;
-  const size_t share = std::min(lds_block, lds_cu / per_cu);
-  auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
-  DynLayout lay{};
+  const bool quartic = t.kind == kQuartic;
+  const size_t fixed = quartic ? sizeof(PairShared<true>) : sizeof(PairShared<false>);
+  const size_t share = std::min(dl.lds_block, dl.lds_cu / std::max(1, per_cu));
+  KmcLayout lay{};
   size_t at = 0;
-  lay.w = static_cast<int>(at);
-  at = al(at + sizeof(double) * t.nwd);
-  if (solvent) {
-    lay.base = static_cast<int>(at);
-    at = al(at + sizeof(double) * 3 * t.S * t.S);
-    lay.lists = static_cast<int>(at);
-    at = al(at + sizeof(uint32_t) * t.n_inc);
-    lay.offs = static_cast<int>(at);
-    at = al(at + sizeof(uint16_t) * 3 * (kEnvSlots + 1));
-  } else {
-    lay.lists = static_cast<int>(at);
-    if (form == 2)
-      at = al(at + sizeof(uint32_t) * (t.n_state_w + t.n_mmm_w + (t.kind == kQuartic ? t.n_mm2_w : 0)));
-    else
-      at = al(at + sizeof(uint32_t) * (t.n_state + t.n_mmm + (t.kind == kQuartic ? t.n_mm2 : 0)));
-    // (n_mm2 counts the forward and the backward entries)
-  }
-  const size_t b1 = sizeof(double) * static_cast<size_t>(t.ne) * t.F1;
-  const size_t b2 = sizeof(double) * static_cast<size_t>(t.ne) * t.F2;
-  if ((t.kind == kE0 || t.kind == kQuartic) && stat + at + b1 <= share) {
-    lay.b1_lds = 1;
-    lay.b1 = static_cast<int>(at);
-    at = al(at + b1);
-  }
-  if (t.kind == kQuartic && lay.b1_lds) {
-    if (stat + at + b2 <= share) {
-      lay.b2_lds = 1;
-      lay.b2 = static_cast<int>(at);
-      at = al(at + b2);
-    } else {  // both barrier tables in LDS or neither
-      at = lay.b1;
-      lay.b1_lds = 0;
-    }
+  auto add = [&](int &where, size_t bytes) {
+    where = static_cast<int>(at);
+    at = (at + bytes + 15) & ~size_t(15);
+  };
+  add(lay.team, teams * sizeof(TeamLds));
+  add(lay.wave, waves * sizeof(WaveLds));
+  add(lay.extra, extra);
+  const size_t row = 8 * static_cast<size_t>(t.ne);
+  const size_t tabs = row * (t.de_row + t.la_row + (quartic ? t.lb_row : 0)) + 48;
+  if (fixed + at + tabs <= share) {
+    lay.tab.tab_lds = 1;
+    add(lay.tab.de, row * t.de_row);
+    add(lay.tab.la, row * t.la_row);
+    if (quartic) add(lay.tab.lb, row * t.lb_row);
   }
   lay.bytes = static_cast<int>(at);
   return lay;
@@ -294,81 +523,112 @@ DynLayout PlanLds(const KTables &t, int32_t R, int form) {
 
 template <typename K>
 hipError_t AllowLds(K kernel, size_t bytes) {
-  if (bytes <= 65536) return hipSuccess;
   return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+}
+
+// f(quartic, tables in LDS) with compile-time arguments.
+template <typename F>
+hipError_t WithModel(const KTables &t, const KmcLayout &lay, F &&f) {
+  if (t.kind == kQuartic)
+    return lay.tab.tab_lds ? f(std::true_type{}, std::true_type{}) : f(std::true_type{}, std::false_type{});
+  return lay.tab.tab_lds ? f(std::false_type{}, std::true_type{}) : f(std::false_type{}, std::false_type{});
+}
+
+template <bool kScan>
+hipError_t LaunchEval(const KTables &t, const uint8_t *occ, const int64_t *off, const int32_t *ncell,
+                      const int64_t *vac, int32_t R, int64_t *nb, double *ea, double *de, int32_t *err,
+                      hipStream_t s, uint8_t *env_out, double *ekra_out, int n, int64_t sub_site,
+                      int sub_code) {
+  if (R <= 0) return hipSuccess;
+  // two workgroups per CU is what the LDS of a ternary model holds
+  const int cus = CurrentDeviceLimits().cus;
+  const int blocks = std::min((R + kEvalWaves - 1) / kEvalWaves, 2 * cus);
+  const KmcLayout lay = PlanLds(t, kEvalWaves, kEvalWaves, 0, 1);
+  return WithModel(t, lay, [&](auto q, auto tab) {
+    auto kernel = EvalJumpsKernel<decltype(q)::value, decltype(tab)::value, kScan>;
+    const hipError_t e = AllowLds(kernel, lay.bytes);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kEvalWaves), lay.bytes, s, t, lay, occ, off, ncell,
+                       vac, R, nb, ea, de, err, env_out, ekra_out, n, sub_site, sub_code);
+    return hipGetLastError();
+  });
+}
+
+// How a KMC batch is laid over the chip. form: 0, 1 one wave per replica; 2 a team of four waves per
+// replica; 3 chain steps.
+struct KmcPlan {
+  KmcLayout lay;
+  int group, blocks, threads;
+  bool chain, team;
+};
+KmcPlan PlanKmc(const KTables &t, int32_t R, int form) {
+  const int cus = CurrentDeviceLimits().cus;
+  KmcPlan p;
+  p.chain = form == 3;
+  p.team = form == 2 || R <= cus || (p.chain && R <= 2 * cus);
+  // one-wave replicas: as many per workgroup as it takes to give every CU one workgroup, up to eight
+  p.group = p.team ? 1 : std::min(8, std::max(1, (R + cus - 1) / cus));
+  p.blocks = (R + p.group - 1) / p.group;
+  const int waves = std::max(kTeam, p.group);
+  p.threads = 64 * waves;
+  const size_t extra = p.chain ? waves * 72 * sizeof(double) : p.team ? sizeof(TeamExchange) : 0;
+  p.lay = PlanLds(t, p.chain ? waves : p.group, waves, extra, p.blocks > cus ? 2 : 1);
+  return p;
+}
+
+// f(kernel) of the plan's instantiation.
+template <typename F>
+hipError_t WithKmcKernel(const KTables &t, const KmcPlan &p, bool full, F &&f) {
+  return WithModel(t, p.lay, [&](auto q, auto tab) {
+    constexpr bool kQ = decltype(q)::value, kT = decltype(tab)::value;
+    auto pick = [&](auto all) {
+      constexpr bool kF = decltype(all)::value;
+      if (p.chain) return p.team ? f(KmcChainKernel<kQ, kT, kTeam, kF>) : f(KmcChainKernel<kQ, kT, 1, kF>);
+      return p.team ? f(KmcKernel<kQ, kT, kTeam, kF>) : f(KmcKernel<kQ, kT, 1, kF>);
+    };
+    return full ? pick(std::true_type{}) : pick(std::false_type{});
+  });
 }
 
 }  // namespace
 
 hipError_t LaunchEvalJumps(const KTables &t, const uint8_t *occ, const int64_t *off,
                            const int32_t *ncell, const int64_t *vac, int32_t R, int64_t *nb,
-                           double *ea, double *de, int32_t *err, hipStream_t s, bool solvent,
-                           uint8_t *env_out, double *ekra_out) {
-  if (R <= 0) return hipSuccess;
-  const DynLayout lay = PlanLds(t, R, solvent ? 1 : 0);
-  auto go = [&](auto kernel) {
-    hipError_t e = AllowLds(kernel, lay.bytes);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, dim3(R), dim3(kThreads), lay.bytes, s, t, lay, occ, off, ncell,
-                       vac, nb, ea, de, err, env_out, ekra_out, 0, GatherSub{-1, 0});
-    return hipGetLastError();
-  };
-  if (lay.b1_lds)
-    return solvent ? go(EvalJumpsKernel<true, true, false>) : go(EvalJumpsKernel<false, true, false>);
-  return solvent ? go(EvalJumpsKernel<true, false, false>) : go(EvalJumpsKernel<false, false, false>);
+                           double *ea, double *de, int32_t *err, hipStream_t s, uint8_t *env_out,
+                           double *ekra_out) {
+  return LaunchEval<false>(t, occ, off, ncell, vac, R, nb, ea, de, err, s, env_out, ekra_out, 0, -1, 0);
 }
 
 hipError_t LaunchVacancyScan(const KTables &t, const uint8_t *occ, int32_t n, int64_t sub_site,
                              int sub_code, const int64_t *sites, int32_t K, int64_t *nb,
                              double *ea, double *de, int32_t *err, hipStream_t s) {
-  if (K <= 0) return hipSuccess;
-  const DynLayout lay = PlanLds(t, K, 0);
-  auto go = [&](auto kernel) {
-    hipError_t e = AllowLds(kernel, lay.bytes);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, dim3(K), dim3(kThreads), lay.bytes, s, t, lay, occ, nullptr,
-                       nullptr, sites, nb, ea, de, err, nullptr, nullptr, n,
-                       GatherSub{sub_site, sub_code});
-    return hipGetLastError();
-  };
-  return lay.b1_lds ? go(EvalJumpsKernel<false, true, true>) : go(EvalJumpsKernel<false, false, true>);
-}
-
-// The instantiation of form (0 dense, 1 solvent baseline, 2 dense wide, 3 second-order chain
-// steps) and LDS placement, with its block size; f(kernel, threads).
-template <typename F>
-hipError_t WithKmcKernel(int form, bool b1_lds, bool record, F &&f) {
-  auto pick = [&](auto rec) {
-    constexpr bool kR = decltype(rec)::value;
-    if (form == 3)
-      return b1_lds ? f(KmcChainKernel<true, kR>, kThreads) : f(KmcChainKernel<false, kR>, kThreads);
-    if (form == 2)
-      return b1_lds ? f(KmcWideKernel<true, kR>, kWideThreads) : f(KmcWideKernel<false, kR>, kWideThreads);
-    if (form == 1)
-      return b1_lds ? f(KmcKernel<true, true, kR>, kThreads) : f(KmcKernel<true, false, kR>, kThreads);
-    return b1_lds ? f(KmcKernel<false, true, kR>, kThreads) : f(KmcKernel<false, false, kR>, kThreads);
-  };
-  return record ? pick(std::true_type{}) : pick(std::false_type{});
+  return LaunchEval<true>(t, occ, nullptr, nullptr, sites, K, nb, ea, de, err, s, nullptr, nullptr, n,
+                          sub_site, sub_code);
 }
 
 hipError_t PrepareKmc(const KTables &t, int32_t R, int form) {
   if (R <= 0) return hipSuccess;
-  const DynLayout lay = PlanLds(t, R, form);
-  auto allow = [&](auto kernel, int) { return AllowLds(kernel, lay.bytes); };
-  const hipError_t e = WithKmcKernel(form, lay.b1_lds != 0, false, allow);
-  return e != hipSuccess ? e : WithKmcKernel(form, lay.b1_lds != 0, true, allow);
+  const KmcPlan p = PlanKmc(t, R, form);
+  auto allow = [&](auto kernel) { return AllowLds(kernel, p.lay.bytes); };
+  const hipError_t e = WithKmcKernel(t, p, false, allow);
+  return e != hipSuccess ? e : WithKmcKernel(t, p, true, allow);
 }
 
 hipError_t LaunchKmc(const KTables &t, const KmcDev &k, uint64_t steps, uint64_t trace_base,
                      hipStream_t s, int form) {
   if (k.R <= 0 || steps == 0) return hipSuccess;
-  const DynLayout lay = PlanLds(t, k.R, form);
-  const bool record = k.atom != nullptr || k.log_every != 0;
-  return WithKmcKernel(form, lay.b1_lds != 0, record, [&](auto kernel, int threads) {
-    hipError_t e = AllowLds(kernel, lay.bytes);
+  // a launch counts its steps and displacements in 32 bits
+  for (constexpr uint64_t kMost = 1u << 30; steps > kMost; steps -= kMost, trace_base += kMost) {
+    const hipError_t e = LaunchKmc(t, k, kMost, trace_base, s, form);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, dim3(k.R), dim3(threads), lay.bytes, s, t, lay, k, steps,
+  }
+  const KmcPlan p = PlanKmc(t, k.R, form);
+  const bool full = k.options || k.n_tt > 0 || k.trace_cap || k.atom || k.log_every;
+  return WithKmcKernel(t, p, full, [&](auto kernel) {
+    const hipError_t e = AllowLds(kernel, p.lay.bytes);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, dim3(p.blocks), dim3(p.threads), p.lay.bytes, s, t, p.lay, k, p.group, static_cast<int>(steps),
                        trace_base);
     return hipGetLastError();
   });

@@ -230,16 +230,6 @@ __device__ __forceinline__ XYZ ReadLaneXYZ(const XYZ &v, int lane) {
           __builtin_amdgcn_readlane(v.Z, lane)};
 }
 
-// ToXYZ with 32-bit divisions: every box has 4 n^3 <= 4e9 < 2^32 sites (n <= 1000).
-__device__ __forceinline__ XYZ ToXYZ32(uint32_t id, uint32_t n) {
-  const uint32_t plane = 2u * n * n;
-  const uint32_t X = id / plane;
-  const uint32_t rest = id - X * plane;
-  const uint32_t Y = rest / n;
-  const uint32_t Zh = rest - Y * n;
-  return {static_cast<int>(X), static_cast<int>(Y), static_cast<int>(2 * Zh + ((X + Y) & 1))};
-}
-
 // Draw attempt att of step `steps` (Philox counter 2 att + 1): the two sites and their
 // coordinates. CanonicalMcAbstract.cpp:43-101 redraws until the species differ; lane l of a
 // wave holds attempt base + l, so the lowest lane of the first round with a hit is the

@@ -404,7 +404,7 @@ __global__ __launch_bounds__(G * kSub) void SurrogateKernel(KTables t, DynLayout
   const bool live = r < k.R;
   JumpLds &L = Ls[g];
   ReplicaLds &Q = Qs[g];
-  const Tabs T = LoadJumpTables<false, kBL>(t, L, dyn, lay, lt, kSub, tid, kBlock);
+  const Tabs T = LoadJumpTables<kBL>(t, L, dyn, lay, lt, kSub, tid, kBlock);
   uint8_t *occ = live ? k.occ + k.off[r] : nullptr;
   const int n = live ? k.ncell[r] : 0;
   if (tid < kEnvRow) S.none[tid] = 0xFF;

@@ -464,8 +464,8 @@ Batch Layout(int32_t R, const int32_t *ncell) {
 void ComputeTotalEnergy(const lmc_model *em, const uint8_t *d_occ, const int64_t *d_off,
                         const int32_t *d_ncell, int32_t R, double *d_energy, hipStream_t s) {
   const auto &t = lmc::Upload(*em->m);
-  unsigned long long *counts = DevAlloc<unsigned long long>(static_cast<size_t>(R) * t.n_eci);
-  const hipError_t e = lmc::LaunchTotalEnergy(t, d_occ, d_off, d_ncell, R, counts, d_energy, s);
+  unsigned long long *counts = DevAlloc<unsigned long long>(static_cast<size_t>(R) * lmc::TotalCountRow(t));
+  const hipError_t e = lmc::LaunchTotalEncode(t, d_occ, d_off, d_ncell, R, counts, nullptr, d_energy, s);
   (void)hipStreamSynchronize(s);
   (void)hipFree(counts);
   Check(e, "total energy kernel");
@@ -1040,7 +1040,7 @@ int lmc_total_energy_noalloc(const lmc_model *m, const uint8_t *d_occ, const int
     if (n_replicas == 0) return LMC_OK;
     unsigned long long *counts = nullptr;
     Check(lmc::TotalEnergyScratch(&counts), "scratch address");
-    Check(lmc::LaunchTotalEnergy(t, d_occ, d_offset, d_ncell, n_replicas, counts, d_energy,
+    Check(lmc::LaunchTotalEncode(t, d_occ, d_offset, d_ncell, n_replicas, counts, nullptr, d_energy,
                                  S(stream)),
           "total energy kernel");
     return LMC_OK;
@@ -1055,7 +1055,7 @@ int lmc_total_encode(const lmc_model *m, const uint8_t *d_occ, const int64_t *d_
     RequireBuffers("lmc_total_encode", n_replicas, {d_occ, d_offset, d_ncell, d_encode});
     const auto &t = lmc::Upload(*m->m);
     unsigned long long *counts =
-        DevAlloc<unsigned long long>(static_cast<size_t>(n_replicas) * t.n_eci);
+        DevAlloc<unsigned long long>(static_cast<size_t>(n_replicas) * lmc::TotalCountRow(t));
     const hipError_t e = lmc::LaunchTotalEncode(t, d_occ, d_offset, d_ncell, n_replicas, counts,
                                                 d_encode, nullptr, S(stream));
     (void)hipStreamSynchronize(S(stream));

@@ -216,7 +216,10 @@ hipError_t LaunchSiteDe(const KTables &t, const uint8_t *occ, const int64_t *off
 hipError_t LaunchCmcAverage(const CmcDev &c, hipStream_t s);
 hipError_t LaunchCmc(const KTables &t, const CmcDev &c, uint64_t trials, uint64_t trace_base,
                      hipStream_t s);
-// GetEncode of every replica: encode[R][n_eci] and energy[R] (either may be null).
+// Counts per replica that LaunchTotalEncode works on: the ECIs and the clusters that have none.
+int TotalCountRow(const KTables &t);
+// GetEncode of every replica: encode[R][n_eci] and energy[R] (either may be null); counts holds
+// R * TotalCountRow entries.
 hipError_t LaunchTotalEncode(const KTables &t, const uint8_t *occ, const int64_t *off,
                              const int32_t *ncell, int32_t R, unsigned long long *counts,
                              double *encode, double *energy, hipStream_t s);
@@ -224,9 +227,6 @@ hipError_t LaunchTotalEncode(const KTables &t, const uint8_t *occ, const int64_t
 hipError_t LaunchClusterEncode(const KTables &t, const uint8_t *occ, int32_t n, const int64_t *set,
                                int32_t m, unsigned long long *counts, double *encode,
                                double *energy, hipStream_t s);
-hipError_t LaunchTotalEnergy(const KTables &t, const uint8_t *occ, const int64_t *off,
-                             const int32_t *ncell, int32_t R, unsigned long long *counts,
-                             double *energy, hipStream_t s);
 // The per-device address of the fixed cluster-count scratch array of lmc_total_energy_noalloc
 // (looked up once per device) and its capacity in counts.
 hipError_t TotalEnergyScratch(unsigned long long **ptr);

@@ -1143,53 +1143,203 @@ __device__ __forceinline__ int Shell(int x, int y, int z) {
   return r2 == 2 ? 1 : r2 == 4 ? 2 : r2 == 6 ? 3 : 0;
 }
 
+// Index of a pair (shell 1..3) or triplet (label 4..7) of species in a count row: its ECI, or past the
+// ECIs for clusters with two or more vacancies, which have none.
+__device__ __forceinline__ int PairIndex(const KTables &t, int shell, int a, int b) {
+  if (a == t.x_code && b == t.x_code) return t.n_eci + shell - 1;
+  return t.eci2[((shell - 1) * t.S + a) * t.S + b];
+}
+__device__ __forceinline__ int TripletIndex(const KTables &t, int label, int a, int b, int c) {
+  const int x = (a == t.x_code) + (b == t.x_code) + (c == t.x_code);
+  if (x >= 2) {  // the third species
+    const int other = a != t.x_code ? a : b != t.x_code ? b : c;
+    return t.n_eci + 3 + (label - 4) * t.S + other;
+  }
+  return t.eci3[(label - 4) * t.S * t.S * t.S + (a * t.S + b) * t.S + c];
+}
+// a count row: at most 561 ECIs (8 species), 3 pairs and 4 * 8 triplets without one
+constexpr int kMaxCountRow = 640;
+
+// The species that the counts leave out: the most frequent one of 64 sites spread over the box (any
+// choice is exact). Called by a whole wave.
+__device__ __forceinline__ int ReferenceSpecies(const uint8_t *o, uint64_t N, int S) {
+  const int v = Code(o[(static_cast<uint64_t>(threadIdx.x & 63) * N) >> 6], S);
+  int ref = 0, most = -1;
+  for (int c = 0; c < S; ++c) {
+    const int n = __builtin_popcountll(__ballot(v == c));
+    if (n > most) {
+      most = n;
+      ref = c;
+    }
+  }
+  return ref;
+}
+
+// The 21 neighbour offsets that follow the site in (x, y, z) order: each pair and each triplet of the box
+// is seen once, from its first member. label[a][c]: the label of the triplet (site, a, c > a), 0 for none.
+// The ordered enumeration meets a pair twice, a triplet of label 4 six times, of 5 and 6 twice (from
+// either end of its two first-neighbour bonds), of 7 once.
+constexpr int kHalf = 21;
+struct NeighbourTables {
+  int8_t off[kHalf][3], shell[kHalf];
+  uint8_t label[kHalf][kHalf];
+  uint32_t with[kHalf];  // the c with a label
+};
+__host__ __device__ constexpr int ShellOfOffset(int x, int y, int z) {
+  const int r2 = x * x + y * y + z * z;
+  return r2 == 2 ? 1 : r2 == 4 ? 2 : r2 == 6 ? 3 : 0;
+}
+constexpr NeighbourTables MakeNeighbourTables() {
+  NeighbourTables n{};
+  int at = 0;
+  for (int x = 0; x <= 2; ++x)
+    for (int y = -2; y <= 2; ++y)
+      for (int z = -2; z <= 2; ++z)
+        if (ShellOfOffset(x, y, z) && (x > 0 || y > 0 || (y == 0 && z > 0))) {
+          n.off[at][0] = static_cast<int8_t>(x);
+          n.off[at][1] = static_cast<int8_t>(y);
+          n.off[at][2] = static_cast<int8_t>(z);
+          n.shell[at++] = static_cast<int8_t>(ShellOfOffset(x, y, z));
+        }
+  for (int a = 0; a < kHalf; ++a)
+    for (int c = a + 1; c < kHalf; ++c) {
+      const int third = ShellOfOffset(n.off[c][0] - n.off[a][0], n.off[c][1] - n.off[a][1], n.off[c][2] - n.off[a][2]);
+      int times[4] = {0, 0, 0, 0};
+      ++times[n.shell[a]];
+      ++times[n.shell[c]];
+      ++times[third];
+      const int label = times[0] ? 0 : times[1] == 3 ? 4 : times[1] == 2 ? (times[2] ? 5 : 6)
+                        : times[1] == 1 && times[2] == 1 ? 7 : 0;
+      n.label[a][c] = static_cast<uint8_t>(label);
+      if (label) n.with[a] |= 1u << c;
+    }
+  return n;
+}
+__constant__ NeighbourTables c_nb = MakeNeighbourTables();
+
+// Ordered cluster counts of the clusters without the reference species (EnergyPredictor.cpp:40-96);
+// EncodeKernel derives the others. A workgroup lists the non-reference sites of 4 096 at a time, then a
+// thread takes a listed site: the species of the neighbours that follow it (21 independent byte loads),
+// then the pairs and triplets of non-reference ones through bit masks. The histogram has a copy per
+// lane (as many as fit), a copy to a bank: atomics of a wave on one counter do not queue.
+// Bound by the LDS atomics and the gathers of the listed sites. 64 boxes of 28^3-32^3 cells, the whole
+// call: 4 720 -> 84 us at 5 at.% solute, 2 580 -> 480 us at 75 % (LDS atomics of all 187 ordered clusters
+// of every site, on a few hot counters, before).
+constexpr int kCountChunk = 4096, kHistWords = 8192;
 __global__ __launch_bounds__(kThreads) void TotalCountsKernel(KTables t, const uint8_t *occ,
                                                               const int64_t *off,
                                                               const int32_t *ncell,
-                                                              unsigned long long *counts) {
-  __shared__ unsigned int hist[512];
-  const int r = blockIdx.x;  // grid (R, 64): x the replica, y a slice of its sites
+                                                              unsigned long long *counts, int row) {
+  __shared__ unsigned int hist[kHistWords];
+  __shared__ uint16_t list[kCountChunk];
+  __shared__ uint16_t eci2[3 * kMaxSpecies * kMaxSpecies], eci3[4 * kMaxSpecies * kMaxSpecies * kMaxSpecies];
+  __shared__ uint8_t label[kHalf][kHalf];
+  __shared__ uint32_t with[kHalf];
+  __shared__ int s_len;
+  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63;  // grid (R, slices of the box)
   const int n = ncell[r];
-  const int64_t N = 4ll * n * n * n;
+  const uint64_t N = 4ull * n * n * n;
+  if (blockIdx.y * static_cast<uint64_t>(kCountChunk) >= N) return;
   const uint8_t *o = occ + off[r];
-  for (int i = threadIdx.x; i < t.n_eci; i += blockDim.x) hist[i] = 0;
-  __syncthreads();
   const int S = t.S;
-  for (int64_t s = static_cast<int64_t>(blockIdx.y) * blockDim.x + threadIdx.x; s < N;
-       s += static_cast<int64_t>(gridDim.y) * blockDim.x) {
-    const XYZ c = ToXYZ(s, n);
-    const int e1 = Code(o[s], S);
-    atomicAdd(&hist[t.eci1[e1]], 1u);
-    for (int a = 0; a < 12; ++a) {
-      const int ax = c_nn1[a][0], ay = c_nn1[a][1], az = c_nn1[a][2];
-      const int e2 = Code(o[SiteAt(c, n, ax, ay, az)], S);
-      atomicAdd(&hist[t.eci2[(0 * S + e1) * S + e2]], 1u);
-      for (int b = 0; b < 12; ++b) {
-        const int x = ax + c_nn1[b][0], y = ay + c_nn1[b][1], z = az + c_nn1[b][2];
-        const int sh = Shell(x, y, z);
-        if (!sh) continue;
-        const int e3 = Code(o[SiteAt(c, n, x, y, z)], S);
-        atomicAdd(&hist[t.eci3[(((3 + sh) - 4) * S * S * S) + (e1 * S + e2) * S + e3]], 1u);
+  const int copies = row <= kHistWords / 32 ? 32 : row <= kHistWords / 16 ? 16 : 8;  // row <= 640
+  for (int i = tid; i < row * copies; i += kThreads) hist[i] = 0;
+  for (int i = tid; i < 3 * S * S; i += kThreads)
+    eci2[i] = static_cast<uint16_t>(PairIndex(t, i / (S * S) + 1, i / S % S, i % S) * copies);
+  for (int i = tid; i < 4 * S * S * S; i += kThreads)
+    eci3[i] = static_cast<uint16_t>(TripletIndex(t, i / (S * S * S) + 4, i / (S * S) % S, i / S % S, i % S) * copies);
+  for (int i = tid; i < kHalf * kHalf; i += kThreads) label[i / kHalf][i % kHalf] = c_nb.label[i / kHalf][i % kHalf];
+  if (tid < kHalf) with[tid] = c_nb.with[tid];
+  unsigned int *mine = hist + (lane & (copies - 1));
+  const int ref = ReferenceSpecies(o, N, S);
+  const int64_t plane = 2ll * n * n;
+  for (uint64_t base = blockIdx.y * static_cast<uint64_t>(kCountChunk); base < N;
+       base += gridDim.y * static_cast<uint64_t>(kCountChunk)) {
+    if (tid == 0) s_len = 0;
+    __syncthreads();
+    uint8_t v[kCountChunk / kThreads];
+#pragma unroll
+    for (int u = 0; u < kCountChunk / kThreads; ++u) {
+      const uint64_t s = base + u * kThreads + tid;
+      v[u] = o[s < N ? s : N - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < kCountChunk / kThreads; ++u) {
+      const bool on = base + u * kThreads + tid < N && Code(v[u], S) != ref;
+      const uint64_t m = __ballot(on);
+      int at = 0;
+      if (lane == 0 && m) at = atomicAdd(&s_len, __builtin_popcountll(m));
+      at = __builtin_amdgcn_readfirstlane(at);
+      if (on) list[at + __builtin_popcountll(m & ((1ull << lane) - 1))] = static_cast<uint16_t>(u * kThreads + tid);
+    }
+    __syncthreads();
+    for (int i = tid; i < s_len; i += kThreads) {
+      const uint64_t s = base + list[i];
+      uint32_t X, Y, Zh;
+      if (N <= 0xFFFFFFFFull) {  // 32-bit divisions but for boxes past 1 023 cells
+        const uint32_t p = static_cast<uint32_t>(plane), u = static_cast<uint32_t>(s);
+        X = u / p;
+        Y = (u - X * p) / n;
+        Zh = u - X * p - Y * n;
+      } else {
+        X = static_cast<uint32_t>(s / plane);
+        const uint64_t rest = s - X * plane;
+        Y = static_cast<uint32_t>(rest / n);
+        Zh = static_cast<uint32_t>(rest - static_cast<uint64_t>(Y) * n);
       }
-      for (int b = 0; b < 6; ++b) {
-        const int x = ax + c_nn2[b][0], y = ay + c_nn2[b][1], z = az + c_nn2[b][2];
-        if (Shell(x, y, z) != 3) continue;
-        const int e3 = Code(o[SiteAt(c, n, x, y, z)], S);
-        atomicAdd(&hist[t.eci3[3 * S * S * S + (e1 * S + e2) * S + e3]], 1u);
+      const uint32_t m = 2 * n, Z = 2 * Zh + ((X + Y) & 1);
+      int64_t xs[3];
+      uint32_t ys[5], zs[5];  // within a plane
+      auto wrap = [&](uint32_t w) { return min(min(w, w + m), w - m); };
+#pragma unroll
+      for (int d = 0; d < 5; ++d) {
+        if (d < 3) xs[d] = wrap(X + d) * plane;
+        ys[d] = wrap(Y + d - 2) * n;
+        zs[d] = wrap(Z + d - 2) >> 1;
+      }
+      constexpr NeighbourTables nb = MakeNeighbourTables();
+      uint8_t e[kHalf];
+#pragma unroll
+      for (int j = 0; j < kHalf; ++j) e[j] = o[xs[nb.off[j][0]] + (ys[nb.off[j][1] + 2] + zs[nb.off[j][2] + 2])];
+      const int e1 = Code(o[s], S);
+      uint32_t other = 0, code[3] = {0, 0, 0};  // the non-reference neighbours; species, 4 bits each
+#pragma unroll
+      for (int j = 0; j < kHalf; ++j) {
+        const uint32_t c = Code(e[j], S);
+        other |= static_cast<uint32_t>(c != static_cast<uint32_t>(ref)) << j;
+        code[j >> 3] |= c << (4 * (j & 7));
+      }
+      constexpr uint32_t second = [] {  // bit masks of the shells
+        uint32_t w = 0;
+        for (int j = 0; j < kHalf; ++j) w |= static_cast<uint32_t>(nb.shell[j] == 2) << j;
+        return w;
+      }();
+      constexpr uint32_t third = [] {
+        uint32_t w = 0;
+        for (int j = 0; j < kHalf; ++j) w |= static_cast<uint32_t>(nb.shell[j] == 3) << j;
+        return w;
+      }();
+      auto species = [&](int j) {
+        const uint32_t w = j < 8 ? code[0] : j < 16 ? code[1] : code[2];
+        return static_cast<int>((w >> (4 * (j & 7))) & 15u);
+      };
+      atomicAdd(&mine[t.eci1[e1] * copies], 1u);
+      for (uint32_t b = other; b; b &= b - 1) {
+        const int a = __builtin_ctz(b), sh = ((second >> a) & 1) + 2 * ((third >> a) & 1), e2 = species(a);
+        atomicAdd(&mine[eci2[(sh * S + e1) * S + e2]], 2u);
+        for (uint32_t c = other & with[a]; c; c &= c - 1) {
+          const int j = __builtin_ctz(c), l = label[a][j] - 4;
+          atomicAdd(&mine[eci3[((l * S + e1) * S + e2) * S + species(j)]], l == 0 ? 6u : l == 3 ? 1u : 2u);
+        }
       }
     }
-    for (int a = 0; a < 6; ++a) {
-      const int e2 = o[SiteAt(c, n, c_nn2[a][0], c_nn2[a][1], c_nn2[a][2])];
-      atomicAdd(&hist[t.eci2[(1 * S + e1) * S + e2]], 1u);
-    }
-    for (int a = 0; a < 24; ++a) {
-      const int e2 = o[SiteAt(c, n, c_nn3[a][0], c_nn3[a][1], c_nn3[a][2])];
-      atomicAdd(&hist[t.eci2[(2 * S + e1) * S + e2]], 1u);
-    }
+    __syncthreads();
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < t.n_eci; i += blockDim.x)
-    if (hist[i]) atomicAdd(&counts[static_cast<int64_t>(r) * t.n_eci + i], hist[i]);
+  for (int i = tid; i < row; i += kThreads) {
+    unsigned long long sum = 0;
+    for (int k = 0; k < copies; ++k) sum += hist[i * copies + ((k + tid) & (copies - 1))];
+    if (sum) atomicAdd(&counts[static_cast<int64_t>(r) * row + i], sum);
+  }
 }
 
 // Membership of site s in the sorted list set[m].
@@ -1210,7 +1360,7 @@ __device__ __forceinline__ bool InSet(const int64_t *set, int m, int64_t s) {
 __global__ __launch_bounds__(kThreads) void ClusterCountsKernel(KTables t, const uint8_t *occ, int n,
                                                                 const int64_t *set, int m,
                                                                 unsigned long long *counts) {
-  __shared__ unsigned int hist[512];
+  __shared__ unsigned int hist[kMaxCountRow];
   for (int i = threadIdx.x; i < t.n_eci; i += blockDim.x) hist[i] = 0;
   __syncthreads();
   const int S = t.S;
@@ -1257,29 +1407,112 @@ __global__ __launch_bounds__(kThreads) void ClusterCountsKernel(KTables t, const
     if (hist[i]) atomicAdd(&counts[i], hist[i]);
 }
 
-// The encode count / N_label of each replica (EnergyPredictor.cpp:89-95) and theta . encode.
-__global__ void EncodeKernel(KTables t, const unsigned long long *counts, int32_t R,
-                             double *encode, double *energy) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= R) return;
-  double e = 0.0;
-  for (int i = 0; i < t.n_eci; ++i) {
-    const double x = static_cast<double>(counts[static_cast<int64_t>(r) * t.n_eci + i]) / t.norm_tot[i];
-    if (encode) encode[static_cast<int64_t>(r) * t.n_eci + i] = x;
-    e += t.theta[i] * x;
+// Number of x in the multiset {a, b} or {a, b, c}.
+__device__ __forceinline__ int Times(int x, int a, int b) { return (x == a) + (x == b); }
+__device__ __forceinline__ int Times(int x, int a, int b, int c) { return (x == a) + (x == b) + (x == c); }
+
+// The counts with the reference species s from those without it (one wave, c the count row in LDS). Every
+// site takes part in the same number of ordered clusters at every position, so with C{..} the ordered
+// count of a multiset of species, N sites, z neighbours, and m triplets per site and position:
+//   C{s} = N - sum C{a}
+//   sum over all pairs of (number of a's) C = 2 z C{a}, which gives C{a, s}; C{s, s} from z N
+//   sum over c of (number of c's in {a, b, c}) C{a, b, c} = sum over the position left out of k C{a, b} of
+//   the shell between the other two, with k third sites per such pair; this gives C{a, b, s}
+//   sum of (number of a's) C = 3 m C{a} gives C{a, s, s}; C{s, s, s} from m N.
+__device__ void CompleteCounts(const KTables &t, unsigned long long *c, int s, unsigned long long N) {
+  const int S = t.S, lane = threadIdx.x & 63;
+  const int z[3] = {12, 6, 24}, m[4] = {48, 24, 48, 24};
+  // third sites per pair of positions (1, 2), (2, 3), (1, 3) of a triplet, and the pair's shell
+  const int k[4][3] = {{4, 4, 4}, {2, 2, 4}, {4, 4, 2}, {2, 4, 1}};
+  const int shell[4][3] = {{1, 1, 1}, {1, 1, 2}, {1, 1, 3}, {1, 2, 3}};
+  auto one = [&](int a) -> unsigned long long & { return c[t.eci1[a]]; };
+  auto two = [&](int sh, int a, int b) -> unsigned long long & { return c[PairIndex(t, sh, a, b)]; };
+  auto three = [&](int l, int a, int b, int d) -> unsigned long long & { return c[TripletIndex(t, 4 + l, a, b, d)]; };
+  if (lane == 0) {
+    unsigned long long rest = N;
+    for (int a = 0; a < S; ++a)
+      if (a != s) rest -= one(a);
+    one(s) = rest;
   }
-  if (energy) energy[r] = e;
+  __syncthreads();
+  for (int i = lane; i < 3 * S; i += 64) {
+    const int sh = i / S + 1, a = i % S;
+    if (a == s) continue;
+    unsigned long long rest = 2ull * z[sh - 1] * one(a);
+    for (int b = 0; b < S; ++b)
+      if (b != s) rest -= Times(a, a, b) * two(sh, a, b);
+    two(sh, a, s) = rest;
+  }
+  __syncthreads();
+  if (lane < 3) {
+    unsigned long long rest = z[lane] * N;
+    for (int a = 0; a < S; ++a)
+      for (int b = a; b < S; ++b)
+        if (!(a == s && b == s)) rest -= two(lane + 1, a, b);
+    two(lane + 1, s, s) = rest;
+  }
+  __syncthreads();
+  for (int i = lane; i < 4 * S * S; i += 64) {
+    const int l = i / (S * S), a = i / S % S, b = i % S;
+    if (a > b || a == s || b == s) continue;
+    unsigned long long rest = 0;
+    for (int p = 0; p < 3; ++p) rest += k[l][p] * two(shell[l][p], a, b);
+    for (int d = 0; d < S; ++d)
+      if (d != s) rest -= Times(d, a, b, d) * three(l, a, b, d);
+    three(l, a, b, s) = rest;
+  }
+  __syncthreads();
+  for (int i = lane; i < 4 * S; i += 64) {
+    const int l = i / S, a = i % S;
+    if (a == s) continue;
+    unsigned long long rest = 3ull * m[l] * one(a);
+    for (int b = 0; b < S; ++b)
+      for (int d = b; d < S; ++d)
+        if (!(b == s && d == s)) rest -= Times(a, a, b, d) * three(l, a, b, d);
+    three(l, a, s, s) = rest;
+  }
+  __syncthreads();
+  if (lane < 4) {
+    unsigned long long rest = m[lane] * N;
+    for (int a = 0; a < S; ++a)
+      for (int b = a; b < S; ++b)
+        for (int d = b; d < S; ++d)
+          if (!(a == s && b == s && d == s)) rest -= three(lane, a, b, d);
+    three(lane, s, s, s) = rest;
+  }
+  __syncthreads();
 }
 
-__global__ void TotalEnergyKernel(KTables t, const unsigned long long *counts, int32_t R,
-                                  double *energy) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= R) return;
-  double e = 0.0;
-  for (int i = 0; i < t.n_eci; ++i)
-    e += t.theta[i] * (static_cast<double>(counts[static_cast<int64_t>(r) * t.n_eci + i]) /
-                       t.norm_tot[i]);
-  energy[r] = e;
+// The encode count / N_label of each replica (EnergyPredictor.cpp:89-95) and theta . encode; one wave per
+// replica, counts in rows of `row`. occ: the counts lack the reference species (null: they are whole).
+// Clusters with two vacancies have no ECI and count for the first one.
+__global__ __launch_bounds__(64) void EncodeKernel(KTables t, const unsigned long long *counts, int row,
+                                                   const uint8_t *occ, const int64_t *off,
+                                                   const int32_t *ncell, double *encode, double *energy) {
+  __shared__ unsigned long long c[kMaxCountRow];
+  __shared__ double x[kMaxCountRow], w[kMaxCountRow];
+  const int r = blockIdx.x, lane = threadIdx.x;
+  for (int i = lane; i < row; i += 64) c[i] = counts[static_cast<int64_t>(r) * row + i];
+  __syncthreads();
+  if (occ) {
+    const int n = ncell[r];
+    const unsigned long long N = 4ull * n * n * n;
+    if (n > 0) CompleteCounts(t, c, ReferenceSpecies(occ + off[r], N, t.S), N);
+    if (lane == 0)
+      for (int i = t.n_eci; i < row; ++i) c[0] += c[i];
+    __syncthreads();
+  }
+  for (int i = lane; i < t.n_eci; i += 64) {
+    x[i] = static_cast<double>(c[i]) / t.norm_tot[i];
+    w[i] = t.theta[i];
+    if (encode) encode[static_cast<int64_t>(r) * t.n_eci + i] = x[i];
+  }
+  __syncthreads();
+  if (energy && lane == 0) {
+    double e = 0.0;
+    for (int i = 0; i < t.n_eci; ++i) e += w[i] * x[i];
+    energy[r] = e;
+  }
 }
 
 __global__ void ZeroKernel(unsigned long long *p, int64_t n) {
@@ -1363,19 +1596,24 @@ hipError_t LaunchCmcAverage(const CmcDev &c, hipStream_t s) {
   return hipGetLastError();
 }
 
+int TotalCountRow(const KTables &t) { return t.n_eci + 3 + 4 * t.S; }
+
 hipError_t LaunchTotalEncode(const KTables &t, const uint8_t *occ, const int64_t *off,
                              const int32_t *ncell, int32_t R, unsigned long long *counts,
                              double *encode, double *energy, hipStream_t s) {
   if (R <= 0) return hipSuccess;
-  const int64_t nc = static_cast<int64_t>(R) * t.n_eci;
+  const int row = TotalCountRow(t);
+  if (row > kMaxCountRow) return hipErrorInvalidValue;
+  const int64_t nc = static_cast<int64_t>(R) * row;
   hipLaunchKernelGGL(ZeroKernel, dim3((nc + 255) / 256), dim3(256), 0, s, counts, nc);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(TotalCountsKernel, dim3(R, 64), dim3(kThreads), 0, s, t, occ, off, ncell,
-                     counts);
+  // slices of a box: enough workgroups for the chip when there are few boxes
+  const int slices = std::max(64, std::min(1024, 4096 / R));
+  hipLaunchKernelGGL(TotalCountsKernel, dim3(R, slices), dim3(kThreads), 0, s, t, occ, off, ncell, counts, row);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(EncodeKernel, dim3((R + 63) / 64), dim3(64), 0, s, t, counts, R, encode, energy);
+  hipLaunchKernelGGL(EncodeKernel, dim3(R), dim3(64), 0, s, t, counts, row, occ, off, ncell, encode, energy);
   return hipGetLastError();
 }
 
@@ -1391,15 +1629,17 @@ hipError_t LaunchClusterEncode(const KTables &t, const uint8_t *occ, int32_t n, 
                      counts);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(EncodeKernel, dim3(1), dim3(64), 0, s, t, counts, 1, encode, energy);
+  hipLaunchKernelGGL(EncodeKernel, dim3(1), dim3(64), 0, s, t, counts, t.n_eci, nullptr, nullptr, nullptr, encode,
+                     energy);
   return hipGetLastError();
 }
 
 // The cluster-count scratch of lmc_total_energy_noalloc: one copy per device, held until the
 // process ends. Host code never passes `scratch` itself (its host-side name is not a device
 // address); it passes the address TotalEnergyScratch looked up on the current device.
-constexpr size_t kScratchCounts = size_t{1} << 19;  // 4 MiB of 64-bit counts
-static __device__ __align__(256) unsigned long long scratch[kScratchCounts];
+constexpr size_t kScratchCounts = size_t{1} << 19;  // 64-bit counts of ECIs
+// a count row holds up to as many entries again for clusters without an ECI
+static __device__ __align__(256) unsigned long long scratch[2 * kScratchCounts];
 
 constexpr int kMaxScratchDevices = 64;
 std::mutex g_scratch_mu;
@@ -1421,22 +1661,6 @@ hipError_t TotalEnergyScratch(unsigned long long **ptr) {
   }
   *ptr = g_scratch_ptr[dev];
   return hipSuccess;
-}
-
-hipError_t LaunchTotalEnergy(const KTables &t, const uint8_t *occ, const int64_t *off,
-                             const int32_t *ncell, int32_t R, unsigned long long *counts,
-                             double *energy, hipStream_t s) {
-  if (R <= 0) return hipSuccess;
-  const int64_t nc = static_cast<int64_t>(R) * t.n_eci;
-  hipLaunchKernelGGL(ZeroKernel, dim3((nc + 255) / 256), dim3(256), 0, s, counts, nc);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(TotalCountsKernel, dim3(R, 64), dim3(kThreads), 0, s, t, occ, off, ncell,
-                     counts);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(TotalEnergyKernel, dim3((R + 63) / 64), dim3(64), 0, s, t, counts, R, energy);
-  return hipGetLastError();
 }
 
 }  // namespace lmc

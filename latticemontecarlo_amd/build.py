@@ -26,14 +26,12 @@ FLAGS = [
 # the default on its own workloads (results unchanged):
 # - KMC kernels: the default. Their list batches are staged by hand, and on 1 024 replicas of 20^3
 #   cells every other strategy stays within 2 % of it (iterative min-register 40 % slower).
-# - canonical-MC kernels, iterative ILP: annealing +2.6 %, CMC beside the uneven KMC batch
-#   +0.9 %, CanonicalMcOmp rounds -0.25 %.
+# - canonical-MC kernels: the default (iterative ILP 8 % slower on serial trials, 6 % on annealing).
 # - surrogate KMC kernel, iterative max-occupancy: +6.2 % (iterative ILP 2.6x and iterative
 #   min-register 2.8x slower, max-ILP -34 %, max-memory-clause -4 %).
 # The surrogate's training kernels keep the default: iterative ILP and max-memory-clause trained
 # within the run-to-run spread of 160 epochs (about 20 s), iterative max-occupancy 18 % slower.
 SOURCE_FLAGS = {
-    "lmc_site_kernels.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
     "lmc_surrogate_kmc.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-maxocc"],
 }
 

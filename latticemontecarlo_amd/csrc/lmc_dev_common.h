@@ -104,6 +104,17 @@ __device__ __forceinline__ void AtomJump(int32_t *atom, int32_t *shift, int64_t 
   }
 }
 
+// Orders the LDS traffic of one wave around a point (its lanes then see each other's writes).
+__device__ __forceinline__ void WaveFence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Keeps the loads of a stage together: left to itself the scheduler pairs every load with its use
+// and waits for each one alone.
+__device__ __forceinline__ void Stage() { __builtin_amdgcn_sched_barrier(0); }
+
 // v of lane l - kShift within the lane's row of 16 (0 past the row start): DPP row_shr on both
 // halves of the double.
 template <int kShift>

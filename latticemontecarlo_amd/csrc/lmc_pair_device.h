@@ -284,10 +284,6 @@ struct PairSums {
   double de, la, lb;
 };
 
-// Keeps the loads of a stage together: left to itself the scheduler pairs every load with its use
-// and waits for each one alone.
-__device__ __forceinline__ void Stage() { __builtin_amdgcn_sched_barrier(0); }
-
 // Values of one batch: the loads of all its terms, then the additions.
 template <bool kQ, int kN>
 struct Values {

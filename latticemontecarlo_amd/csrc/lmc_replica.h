@@ -30,13 +30,6 @@ __device__ __forceinline__ void SetVacancyXYZ(ReplicaLds &Q, int n) {
 }
 __device__ __forceinline__ XYZ VacancyXYZ(const ReplicaLds &Q) { return {Q.vx, Q.vy, Q.vz}; }
 
-// Orders the LDS traffic of one wave around a point (its lanes then see each other's writes).
-__device__ __forceinline__ void WaveFence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // TimeTemperatureInterpolator::GetTemperature (TimeTemperatureInterpolator.cpp:44-65)
 __device__ double ScheduleTemperature(const double *tt, const double *tv, int n, double time) {
   int i = 0;

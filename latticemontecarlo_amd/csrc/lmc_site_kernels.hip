@@ -18,10 +18,9 @@ struct SiteLds {
   uint32_t cl[kMaxSiteClusters];
   int32_t off[kSiteSlots];
   double w[kMaxW];
-  uint8_t env[4][48];           // environments of up to two swaps (p, q of each)
-  int slot[4];                  // partner slots (q around p, p around q) of each swap
+  uint8_t env[2][48];           // environments of the swap's sites
+  int slot[2];                  // partner slots (q around p, p around q)
   double part[kThreads / 64];   // per-wave partial sums
-  double part2[kThreads / 64];  // the same for the second swap
 };
 
 __device__ void LoadSiteTables(const KTables &t, SiteLds &L) {
@@ -219,17 +218,6 @@ __device__ void AnnealUpdate(CmcAnneal &A, const AnnealSchedule &s, bool accepte
 
 constexpr uint32_t kMaxPairAttempts = 1u << 20;
 
-__device__ __forceinline__ int64_t ReadLane64(int64_t v, int lane) {
-  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), lane));
-  const uint32_t hi =
-      static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), lane));
-  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
-}
-__device__ __forceinline__ XYZ ReadLaneXYZ(const XYZ &v, int lane) {
-  return {__builtin_amdgcn_readlane(v.X, lane), __builtin_amdgcn_readlane(v.Y, lane),
-          __builtin_amdgcn_readlane(v.Z, lane)};
-}
-
 // Draw attempt att of step `steps` (Philox counter 2 att + 1): the two sites and their
 // coordinates. CanonicalMcAbstract.cpp:43-101 redraws until the species differ; lane l of a
 // wave holds attempt base + l, so the lowest lane of the first round with a hit is the
@@ -255,7 +243,7 @@ __device__ __forceinline__ double TrialUniform(const CmcDev &c, int r, uint64_t 
   return UnitOpenRight(Join64(u.x, u.y));
 }
 
-// Cluster `tid` of the site table, decoded once: the weight index of centre species x with the
+// Cluster i of the site table, decoded once: the weight index of centre species x with the
 // other sites' species e1, e2 is base + x kx + e1 k1 + e2 k2 (SiteWeight's three cases).
 struct SiteCluster {
   int base, kx, k1, k2;
@@ -263,11 +251,11 @@ struct SiteCluster {
   int r1, r2;      // raw slots (63 = none), for the partner test
   bool live;
 };
-__device__ SiteCluster DecodeSiteCluster(const KTables &t, const SiteLds &L, int i) {
+__device__ SiteCluster DecodeSiteCluster(const KTables &t, const uint32_t *cl, int i) {
   SiteCluster q{};
   q.live = i < t.n_site;
   if (!q.live) return q;
-  const uint32_t d = L.cl[i];
+  const uint32_t d = cl[i];
   const int S = t.S, label = d & 7;
   q.r1 = (d >> 4) & 63;
   q.r2 = (d >> 10) & 63;
@@ -287,68 +275,6 @@ __device__ SiteCluster DecodeSiteCluster(const KTables &t, const SiteLds &L, int
     q.o2 = q.r2;
   }
   return q;
-}
-// w(x -> en) - w(x -> eo) of the cluster in environment `which`, 0 when it contains slot skip.
-__device__ __forceinline__ double ClusterDelta(const SiteLds &L, const SiteCluster &q, int which,
-                                               int eo, int en, int skip) {
-  if (!q.live || (skip >= 0 && (q.r1 == skip || q.r2 == skip))) return 0.0;
-  const uint8_t *e = L.env[which];
-  const int rest = q.base + e[q.o1] * q.k1 + e[q.o2] * q.k2;
-  return L.w[rest + en * q.kx] - L.w[rest + eo * q.kx];
-}
-
-// One trial's pair as found by its wave: sites, coordinates, species, and the winning lane of
-// the first draw round (-1: found in a later round; -2: none within kMaxPairAttempts).
-struct TrialLds {
-  int64_t p, q;
-  XYZ xp, xq;
-  int ep, eq, win;
-};
-
-// Finds the trial's pair among the wave's draw attempts (cand: attempts lane of step `step`,
-// further rounds drawn here), gathers both environments into L.env[e0], L.env[e0 + 1] and both
-// partner slots, and leaves the result in T (lane 0 writes). Called by a whole wave.
-__device__ void FindTrial(const CmcDev &c, int r, uint64_t step, const uint8_t *occ, uint64_t N,
-                          int n, int S, int lane, int ox, int oy, int oz, PairDraw &cand,
-                          SiteLds &L, int e0, TrialLds &T) {
-  uint64_t m = __ballot(occ[cand.a] != occ[cand.b]);
-  const bool first = m != 0;
-  for (uint32_t base = 64; !m && base < kMaxPairAttempts; base += 64) {
-    cand = DrawAttempt(c, r, step, base + static_cast<uint32_t>(lane), N, n);
-    m = __ballot(occ[cand.a] != occ[cand.b]);
-  }
-  if (!m) {
-    if (lane == 0) T.win = -2;
-    return;
-  }
-  const int w = __builtin_ctzll(m);
-  const int64_t p = ReadLane64(cand.a, w), q = ReadLane64(cand.b, w);
-  const XYZ xp = ReadLaneXYZ(cand.xa, w), xq = ReadLaneXYZ(cand.xb, w);
-  bool hq = false, hp = false;
-  if (lane < kSiteSlots) {
-    const uint8_t vp = occ[SiteAt(xp, n, ox, oy, oz)];
-    const uint8_t vq = occ[SiteAt(xq, n, ox, oy, oz)];
-    L.env[e0][lane] = vp < S ? vp : 0;  // codes are validated at creation
-    L.env[e0 + 1][lane] = vq < S ? vq : 0;
-    if (lane >= 1) {  // partner slots: the first offset equal to the minimum image
-      hq = ox == MinImage(xq.X - xp.X, n) && oy == MinImage(xq.Y - xp.Y, n) &&
-           oz == MinImage(xq.Z - xp.Z, n);
-      hp = ox == MinImage(xp.X - xq.X, n) && oy == MinImage(xp.Y - xq.Y, n) &&
-           oz == MinImage(xp.Z - xq.Z, n);
-    }
-  }
-  const uint64_t mq = __ballot(hq), mp = __ballot(hp);
-  if (lane == 0) {
-    L.slot[e0] = mq ? __builtin_ctzll(mq) : -1;
-    L.slot[e0 + 1] = mp ? __builtin_ctzll(mp) : -1;
-    T.p = p;
-    T.q = q;
-    T.xp = xp;
-    T.xq = xq;
-    T.ep = occ[p];
-    T.eq = occ[q];
-    T.win = first ? w : -1;
-  }
 }
 
 // The dump cadence, evaluated for consecutive steps with one division per change of cadence.
@@ -383,85 +309,124 @@ struct LogClock {
 // optional linear temperature ramp t0 -> t1 over maximum_steps, or the adaptive annealing
 // schedule. One workgroup per replica. kLdsOcc: the replica's occupancy (N bytes, N a multiple
 // of 4) lives in dynamic LDS for the launch and is written back at its end.
-// Two trials per round of three barriers: trial A (step s) and, speculatively, trial B (step
-// s + 1) on the same occupancy.
-//   1. wave 0 finds A's pair among its 64 precomputed draw attempts (ballot) and gathers both
-//      environments and partner slots; wave 1 does the same for B;
-//   2. every thread adds its cluster's change for both swaps (DPP wave sums); wave 1 checks
-//      whether A's two sites lie among B's draw attempts up to its winning one or in B's
-//      environments;
-//   3. lane 0 of wave 3 accepts or rejects A, then B unless A was accepted and touched B (B is
-//      then redone as the next round's A, so the trajectory is the sequential one); meanwhile
-//      waves 0 and 1 draw the attempts of steps s + 2 and s + 3 and lane 0 of wave 2 their
-//      Metropolis uniforms.
+//
+// Bound by the latency of one trial's chain (draw, species, environments, weights, Metropolis), so
+// kCmcWaves trials run side by side on the same occupancy and are taken in order up to the first that
+// an accepted one before it would have changed: the trajectory is the sequential one. A round:
+//   1. wave w finds the pair of step s + w among the 63 attempts that it drew ahead (lane 63 drew the
+//      Metropolis uniform), gathers both environments, adds the change of the site clusters (four to a
+//      lane) for both sites and tests the step;
+//   2. an accepted trial has marked its two sites in the occupancy (top bit); the later waves look at
+//      the sites that they read (attempts up to the winning one, environments) again, and the first
+//      that read a site of an accepted trial before it ends the round;
+//   3. the commit wave swaps, records, adds the energies in order, and sets the next round's betas,
+//      while the other waves draw the attempts of the next round's steps.
+// 64 replicas of 30^3 cells at 5 at.% solute, 2 000 trials: 2 760 -> 820 us (two trials to a round, each
+// by a whole workgroup of four waves, before); 6^3 cells 2 940 -> 1 800, 1 at.% 3 990 -> 2 500, annealing
+// 2 920 -> 1 170.
+// In a small box accepted trials often end a round early: the next rounds then try fewer, and more again
+// after one that was taken whole (8 waves instead of 15: 15 % slower at 30^3 cells, 28 % faster at
+// 6^3). A wave that missed its pair in the first 63 attempts draws 127 ahead
+// until one of the first eight wins.
 // kLog: the log records and the averaging ring are compiled in (taken when c.log_every is set).
+constexpr int kCmcWaves = 15;
+constexpr int kCmcRing = 32;  // at least two rounds, a power of two
+constexpr int kCmcThreads = (kCmcWaves + 1) * 64;
+constexpr int kCmcFirst = 63;  // attempts of a trial's first draw; lane 63 draws its uniform
+constexpr int kClustersPerLane = kMaxSiteClusters / 64;
+
+struct CmcLds {
+  double w[kMaxW];
+  uint16_t env[kCmcWaves][64];  // species around p (low byte) and q of each trial
+  double de[kCmcWaves];
+  double beta[kCmcRing], T[kCmcRing];  // by step modulo kCmcRing; annealing: by wave
+  uint32_t p[kCmcWaves], q[kCmcWaves];
+  uint8_t ep[kCmcWaves], eq[kCmcWaves];
+  uint8_t flag[kCmcWaves], conflict[kCmcWaves];
+  int limit;  // annealing: trials of the next round whose temperatures are known
+};
+constexpr uint8_t kMark = 0x80;  // species codes are below it
+enum : uint8_t { kTrialAccepted = 1, kTrialLost = 2 };  // lost: no pair within kMaxPairAttempts
+
 template <bool kLdsOcc, bool kLog>
-__global__ __launch_bounds__(kThreads) void CmcKernel(KTables t, CmcDev c, uint64_t ntrials,
-                                                      uint64_t trace_base) {
-  __shared__ SiteLds L;
-  __shared__ TrialLds s_tr[2];
-  __shared__ int s_done, s_adv, s_conf;
-  __shared__ double s_u[4], s_beta[4];  // by step & 3; s_beta: the ramp's beta
-  // annealing: T at the start of the round and the betas of A (that T) and B (after A's decay)
-  __shared__ double s_T, s_bA, s_bB;
+__global__ __launch_bounds__(kCmcThreads) void CmcKernel(KTables t, CmcDev c, uint64_t ntrials,
+                                                         uint64_t trace_base) {
+  __shared__ CmcLds L;
   extern __shared__ uint32_t occ_words[];
-  constexpr int kAcceptThread = 3 * 64;
   const int r = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  LoadSiteTables(t, L);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool commit = wave == kCmcWaves;
+  for (int i = tid; i < t.nw; i += kCmcThreads) L.w[i] = t.w[i];
   const int n = c.ncell[r];
   const uint64_t N = 4ull * n * n * n;
   uint8_t *occ = c.occ + c.off[r];
   if constexpr (kLdsOcc) {
     const uint32_t *src = reinterpret_cast<const uint32_t *>(occ);
-    for (uint64_t i = tid; i < N / 4; i += kThreads) occ_words[i] = src[i];
+    for (uint64_t i = tid; i < N / 4; i += kCmcThreads) occ_words[i] = src[i];
     occ = reinterpret_cast<uint8_t *>(occ_words);
   }
   uint64_t steps = c.steps[r];
-  const uint64_t maxs = c.max_steps[r];
+  const uint64_t maxs = c.max_steps[r], seed = c.seed[r];
+  const uint32_t rid = c.rid[r];
   uint64_t acc = 0;
   double energy = 0, abse = 0;
   CmcAnneal A{};
   AnnealSchedule sched{};
   LogClock clk;
   uint64_t log_i = 0, ring_i = 0, ring_at = 0;  // records, energies added, ring slot
-  if (tid == kAcceptThread) {
+  if (commit) {
     acc = c.accepted[r];
     energy = c.energy[r];
     abse = c.abs_energy[r];
     if (c.anneal) {
       A = c.anneal[r];
       sched = MakeAnnealSchedule(maxs);
-      s_T = A.T;
     }
     if constexpr (kLog) {
       clk.L = c.log_every;
       clk.plain = c.anneal != nullptr;
       clk.Reset(steps);
       log_i = c.log_n[r];
-      c.log_lo[r] = log_i;
+      if (lane == 0) c.log_lo[r] = log_i;
       if (c.avg_m) {
         ring_i = c.ring_n[r];
         ring_at = ring_i % c.ring_cap;
       }
     }
   }
-  const double decay = c.anneal ? MakeAnnealSchedule(maxs).decay : 1.0;
-  if (tid == 0) s_done = steps > maxs ? 1 : 0;
-  PairDraw cand{};
-  int ox = 0, oy = 0, oz = 0;  // waves 0 and 1: the lane's environment offset
-  if (wave < 2) {
-    cand = DrawAttempt(c, r, steps + wave, static_cast<uint32_t>(lane), N, n);
-    if (lane < kSiteSlots) Unpack(t.site_off[lane], ox, oy, oz);
-  }
-  // the ramp's temperature and beta of a step (CanonicalMcAbstract: beta = 1 / kB / T)
+  // the ramp's temperature of a step (CanonicalMcAbstract: beta = 1 / kB / T)
   auto ramp_T = [&](uint64_t step) {
     return c.t0[r] + (c.t1[r] - c.t0[r]) * (static_cast<double>(step) / static_cast<double>(maxs));
   };
-  auto ramp_beta = [&](uint64_t step) { return 1.0 / kBoltzmann / ramp_T(step); };
-  // a log record of the step about to be tried (accept thread)
+  // Temperatures and betas of kCmcWaves steps from `step` on (commit wave). Annealing: the temperatures
+  // are those of the decay alone, so the round ends with the trial that closes an acceptance window or
+  // may reheat.
+  auto set_betas = [&](uint64_t step) {
+    double T;
+    if (c.anneal) {
+      T = A.T;
+      for (int k = 1; k < kCmcWaves; ++k)
+        if (lane >= k) T *= sched.decay;
+      const uint64_t trials = A.window_trials + static_cast<uint64_t>(lane) + 1;  // once lane's trial is done
+      const uint64_t at = step + static_cast<uint64_t>(lane);
+      const bool reheat = A.reheats < 5 && at - A.last_improvement >= sched.trigger &&
+                          at - A.last_reheat >= sched.cooldown &&
+                          static_cast<double>(A.window_accepts) / static_cast<double>(trials) < 0.05;
+      const uint64_t stop = __ballot(lane < kCmcWaves && (trials >= sched.window || reheat));
+      if (lane == 0) L.limit = stop ? __builtin_ctzll(stop) + 1 : kCmcWaves;
+    } else {
+      T = ramp_T(step + static_cast<uint64_t>(lane));
+    }
+    if (lane < kCmcWaves) {
+      const int at = c.anneal ? lane : static_cast<int>((step + lane) & (kCmcRing - 1));
+      L.T[at] = T;
+      L.beta[at] = 1.0 / kBoltzmann / (c.anneal ? fmax(T, 1e-12) : T);
+    }
+  };
+  // a log record of the step about to be tried (commit wave)
   auto put_log = [&](uint64_t step, double T, double second) {
-    if (log_i < c.log_cap) {
+    if (log_i < c.log_cap && lane == 0) {
       CmcLogRecord &rec = c.log[static_cast<uint64_t>(r) * c.log_cap + log_i];
       rec.steps = step;
       rec.temperature = T;
@@ -472,148 +437,303 @@ __global__ __launch_bounds__(kThreads) void CmcKernel(KTables t, CmcDev c, uint6
     }
     ++log_i;  // counts past the capacity too, so the host can report the loss
   };
-  // lane 0 of wave 2: the Metropolis uniforms (and ramp betas) of steps s and s + 1
-  auto draw_ahead = [&](uint64_t step) {
-    s_u[step & 3] = TrialUniform(c, r, step);
-    if (!c.anneal) s_beta[step & 3] = ramp_beta(step);
+  // attempts (and the uniform, in lane 63 of the first draw) of a step; their coordinates X, Y < 2^11
+  // and Z / 2 < 2^10 in one word
+  uint32_t a = 0, b = 0, xa = 0, xb = 0, a2 = 0, b2 = 0;
+  bool dilute = false, second = false;  // second: a2, b2 hold the 64 attempts after the first 63
+  double uni = 0.0;
+  auto pack = [&](uint32_t site) {
+    const uint32_t plane = 2u * n * n, X = site / plane, rest = site - X * plane, Y = rest / n;
+    return X | Y << 11 | (rest - Y * n) << 22;
   };
-  if (tid == 128) {
-    draw_ahead(steps);
-    draw_ahead(steps + 1);
+  auto unpack = [](uint32_t v) -> XYZ {
+    const int X = v & 2047, Y = (v >> 11) & 2047;
+    return {X, Y, static_cast<int>(v >> 22) * 2 + ((X + Y) & 1)};
+  };
+  auto draw = [&](uint64_t step) {
+    const U4 u = Philox4x32_10(seed, step, rid, lane == kCmcFirst ? 0xFFFFFFFEu : 2u * lane + 1u);
+    second = dilute;
+    if (second) {
+      const U4 v = Philox4x32_10(seed, step, rid, 2u * (kCmcFirst + lane) + 1u);
+      a2 = static_cast<uint32_t>(MulHi64(Join64(v.x, v.y), N));
+      b2 = static_cast<uint32_t>(MulHi64(Join64(v.z, v.w), N));
+    }
+    a = static_cast<uint32_t>(MulHi64(Join64(u.x, u.y), N));
+    b = static_cast<uint32_t>(MulHi64(Join64(u.z, u.w), N));
+    xa = pack(a);
+    xb = pack(b);
+    uni = UnitOpenRight(Join64(u.x, u.y));
+  };
+  SiteCluster cl[kClustersPerLane];
+  int ox = 0, oy = 0, oz = 0;  // the lane's environment offset
+  if (commit) {
+    set_betas(steps);
+  } else {
+    draw(steps + wave);
+#pragma unroll
+    for (int k = 0; k < kClustersPerLane; ++k) cl[k] = DecodeSiteCluster(t, t.site_cl, lane + 64 * k);
+    if (lane < kSiteSlots) Unpack(t.site_off[lane], ox, oy, oz);
   }
   __syncthreads();
-  const SiteCluster cl = DecodeSiteCluster(t, L, tid);
-  // Metropolis step of the trial at `step` (accept thread): accept, trace, swap, anneal.
-  // pre_T, pre_beta: a temperature and its beta computed ahead (used when A.T equals pre_T).
-  auto metropolis = [&](uint64_t step, uint64_t trace_index, const TrialLds &T, double de,
-                        double pre_T, double pre_beta) {
-    if constexpr (kLog) {
-      if (c.avg_m) {  // ThermodynamicAveraging::AddEnergy before Dump (CanonicalMcSerial.cpp:45)
-        c.ring[static_cast<uint64_t>(r) * c.ring_cap + ring_at] = energy;
-        if (++ring_at == c.ring_cap) ring_at = 0;
-        ++ring_i;
-      }
-    }
-    double beta;
-    if (c.anneal) {
-      const bool lower = energy < A.lowest - 1e-4;  // Dump (SimulatedAnnealing.cpp:80-97)
-      if (lower) A.lowest = energy;
-      if constexpr (kLog) {
-        if (lower) put_log(step, A.T, A.lowest);
-        if (clk.Due(step)) put_log(step, A.T, A.lowest);
-      }
-      beta = A.T == pre_T ? pre_beta : 1.0 / kBoltzmann / fmax(A.T, 1e-12);
-    } else {
-      beta = s_beta[step & 3];
-      if constexpr (kLog) {
-        if (clk.Due(step)) put_log(step, ramp_T(step), 0.0);
-      }
-    }
-    const bool accept = de < 0 || s_u[step & 3] < exp(-de * beta);
-    if (trace_index < c.trace_cap) {
-      const uint64_t o = static_cast<uint64_t>(r) * c.trace_cap + trace_index;
-      c.tr_p[o] = T.p;
-      c.tr_q[o] = T.q;
-      c.tr_de[o] = de;
-      c.tr_acc[o] = accept ? 1 : 0;
-    }
-    if (accept) {
-      if (c.atom) {
-        const int64_t o = c.off[r];
-        AtomJump(c.atom + o, c.shift + 3 * o, T.p, T.q, ImageChange(T.xq.X - T.xp.X, n),
-                 ImageChange(T.xq.Y - T.xp.Y, n), ImageChange(T.xq.Z - T.xp.Z, n));
-      }
-      occ[T.p] = static_cast<uint8_t>(T.eq);
-      occ[T.q] = static_cast<uint8_t>(T.ep);
-      energy += de;
-      abse += de;
-      ++acc;
-    }
-    if (c.anneal) AnnealUpdate(A, sched, accept, step, energy);
-    return accept;
-  };
-  bool fresh = true;  // waves 0 and 1 hold the attempts of steps and steps + 1
   uint64_t it = 0;
-  while (it < ntrials) {
-    if (s_done) break;
-    if (wave < 2) {
-      if (!fresh) cand = DrawAttempt(c, r, steps + wave, static_cast<uint32_t>(lane), N, n);
-      FindTrial(c, r, steps + wave, occ, N, n, t.S, lane, ox, oy, oz, cand, L, 2 * wave,
-                s_tr[wave]);
-      if (wave == 0 && lane == 0 && s_tr[0].win == -2) {
-        atomicOr(c.error, 2);
-        s_done = 1;
+  bool lost = false;
+  int active = kCmcWaves;  // trials of a round
+  while (it < ntrials && steps <= maxs) {
+    int limit = c.anneal ? L.limit : kCmcWaves;  // read before the commit wave sets the next one
+    int win = -1;           // winning attempt of the first draw, -1: of a later one
+    uint32_t sp = 0, sq = 0;  // the lane's sites of both environments
+    uint64_t seen = 0;        // the lanes whose second attempts were looked at
+    if (commit) {
+      if (!c.anneal) set_betas(steps + kCmcWaves);  // the next round may start anywhere up to there
+    } else if (wave < active) {
+      // another wave of the round may have marked a site by now
+      uint64_t m = __ballot(lane < kCmcFirst && ((occ[a] ^ occ[b]) & ~kMark) != 0);
+      if (m) win = __builtin_ctzll(m);
+      uint32_t base = kCmcFirst;
+      dilute = !m || (dilute && win >= 8);
+      uint32_t ta = a, tb = b, txa = xa, txb = xb;
+      if (!m && second) {
+        ta = a2;
+        tb = b2;
+        m = __ballot(((occ[ta] ^ occ[tb]) & ~kMark) != 0);
+        base += 64;
+        if (m) {
+          txa = pack(ta);
+          txb = pack(tb);
+          seen = (m ^ (m - 1));
+          win = kCmcFirst;  // all of the first
+        }
       }
+      for (; !m && base < kMaxPairAttempts; base += 128) {  // two draws side by side
+        uint32_t more[2][2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const U4 u = Philox4x32_10(seed, steps + wave, rid, 2u * (base + 64u * k + lane) + 1u);
+          more[k][0] = static_cast<uint32_t>(MulHi64(Join64(u.x, u.y), N));
+          more[k][1] = static_cast<uint32_t>(MulHi64(Join64(u.z, u.w), N));
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          if (m) continue;
+          ta = more[k][0];
+          tb = more[k][1];
+          m = __ballot(base + 64u * k + lane < kMaxPairAttempts && ((occ[ta] ^ occ[tb]) & ~kMark) != 0);
+        }
+        txa = pack(ta);
+        txb = pack(tb);
+      }
+      uint8_t flag = kTrialLost;
+      if (m) {
+        const int at = __builtin_ctzll(m);
+        auto lane_of = [&](uint32_t v) {
+          return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), at));
+        };
+        const uint32_t p = lane_of(ta), q = lane_of(tb);
+        const XYZ xp = unpack(lane_of(txa)), xq = unpack(lane_of(txb));
+        sp = static_cast<uint32_t>(SiteAt(xp, n, ox, oy, oz));
+        sq = static_cast<uint32_t>(SiteAt(xq, n, ox, oy, oz));
+        const int vp = occ[sp] & ~kMark, vq = occ[sq] & ~kMark;
+        // lane 0 is the site itself; codes are validated at creation
+        const int ep = __builtin_amdgcn_readlane(vp, 0), eq = __builtin_amdgcn_readlane(vq, 0);
+        const int S = t.S;
+        L.env[wave][lane] = static_cast<uint16_t>((vp < S ? vp : 0) | (vq < S ? vq : 0) << 8);
+        // partner slots: the first offset equal to the minimum image
+        int slot_p = 64, slot_q = 64;
+        const int dx = MinImage(xq.X - xp.X, n), dy = MinImage(xq.Y - xp.Y, n), dz = MinImage(xq.Z - xp.Z, n);
+        const int nx = MinImage(xp.X - xq.X, n), ny = MinImage(xp.Y - xq.Y, n), nz = MinImage(xp.Z - xq.Z, n);
+        if (dx * dx + dy * dy + dz * dz <= 6) {
+          const bool in = lane >= 1 && lane < kSiteSlots;
+          const uint64_t mq = __ballot(in && ox == dx && oy == dy && oz == dz);
+          const uint64_t mp = __ballot(in && ox == nx && oy == ny && oz == nz);
+          if (mq) slot_p = __builtin_ctzll(mq);
+          if (mp) slot_q = __builtin_ctzll(mp);
+        }
+        WaveFence();
+        uint32_t e1[kClustersPerLane], e2[kClustersPerLane];
+#pragma unroll
+        for (int k = 0; k < kClustersPerLane; ++k) {
+          e1[k] = L.env[wave][cl[k].o1];
+          e2[k] = L.env[wave][cl[k].o2];
+        }
+        Stage();
+        double w[kClustersPerLane][4];  // p's cluster after and before, q's
+#pragma unroll
+        for (int k = 0; k < kClustersPerLane; ++k) {
+          const int rest_p = cl[k].base + (e1[k] & 255) * cl[k].k1 + (e2[k] & 255) * cl[k].k2;
+          const int rest_q = cl[k].base + (e1[k] >> 8) * cl[k].k1 + (e2[k] >> 8) * cl[k].k2;
+          const int at_p = ep * cl[k].kx, at_q = eq * cl[k].kx;
+          w[k][0] = L.w[rest_p + at_q];
+          w[k][1] = L.w[rest_p + at_p];
+          w[k][2] = L.w[rest_q + at_p];
+          w[k][3] = L.w[rest_q + at_q];
+        }
+        Stage();
+        double de = 0.0;
+        if (slot_p < 64 || slot_q < 64) {  // clusters with both sites keep their species
+#pragma unroll
+          for (int k = 0; k < kClustersPerLane; ++k) {
+            if (cl[k].r1 == slot_p || cl[k].r2 == slot_p) w[k][0] = w[k][1] = 0.0;
+            if (cl[k].r1 == slot_q || cl[k].r2 == slot_q) w[k][2] = w[k][3] = 0.0;
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < kClustersPerLane; ++k)  // lanes past the last cluster add w - w
+          de += (w[k][0] - w[k][1]) + (w[k][2] - w[k][3]);
+        de = WaveSum(de);
+        const double u = ReadLane(uni, kCmcFirst);
+        const bool accept = de < 0 || u < exp(-de * L.beta[c.anneal ? wave : (steps + wave) & (kCmcRing - 1)]);
+        flag = accept ? kTrialAccepted : 0;
+        if (lane == 0) {
+          L.de[wave] = de;
+          L.p[wave] = p;
+          L.q[wave] = q;
+          L.ep[wave] = static_cast<uint8_t>(ep);
+          L.eq[wave] = static_cast<uint8_t>(eq);
+          if (accept) {
+            occ[p] = static_cast<uint8_t>(ep) | kMark;
+            occ[q] = static_cast<uint8_t>(eq) | kMark;
+          }
+        }
+      }
+      if (lane == 0) L.flag[wave] = flag;
     }
     __syncthreads();
-    if (s_done) break;
-    {
-      const TrialLds &TA = s_tr[0], &TB = s_tr[1];
-      const bool hasB = TB.win != -2;
-      double va = ClusterDelta(L, cl, 0, TA.ep, TA.eq, L.slot[0]) +
-                  ClusterDelta(L, cl, 1, TA.eq, TA.ep, L.slot[1]);
-      double vb = hasB ? ClusterDelta(L, cl, 2, TB.ep, TB.eq, L.slot[2]) +
-                             ClusterDelta(L, cl, 3, TB.eq, TB.ep, L.slot[3])
-                       : 0.0;
-      va = WaveSum(va);
-      vb = WaveSum(vb);
-      if (lane == 0) {
-        L.part[wave] = va;
-        L.part2[wave] = vb;
+    const int slot = lane < kCmcWaves ? lane : 0;
+    const uint8_t flag = L.flag[slot];
+    const uint32_t tp = L.p[slot], tq = L.q[slot];
+    const bool swap = lane < active && (flag & kTrialAccepted);
+    const uint64_t accepted = __ballot(swap);
+    const uint64_t lost_at = __ballot(lane < active && (flag & kTrialLost));
+    if (lost_at & 1) {  // every thread sees the same flags
+      lost = true;
+      if (commit && swap) {
+        occ[tp] = L.ep[slot];
+        occ[tq] = L.eq[slot];
       }
-      if (c.anneal && tid == 128) {  // both betas of the round, off the Metropolis lane's path
-        const double T = s_T, Tb = T * decay;
-        s_bA = 1.0 / kBoltzmann / fmax(T, 1e-12);
-        s_bB = 1.0 / kBoltzmann / fmax(Tb, 1e-12);
-      }
-      if (wave == 1) {  // does A's swap touch B's draw or environments?
-        bool hit = false;
-        if (TB.win >= 0 && lane <= TB.win)
-          hit = cand.a == TA.p || cand.a == TA.q || cand.b == TA.p || cand.b == TA.q;
-        if (hasB && lane < kSiteSlots) {
-          const int64_t s1 = SiteAt(TB.xp, n, ox, oy, oz), s2 = SiteAt(TB.xq, n, ox, oy, oz);
-          hit = hit || s1 == TA.p || s1 == TA.q || s2 == TA.p || s2 == TA.q;
+      break;
+    }
+    limit = min(limit, active);
+    if (ntrials - it < static_cast<uint64_t>(limit)) limit = static_cast<int>(ntrials - it);
+    if (maxs - steps < static_cast<uint64_t>(limit)) limit = static_cast<int>(maxs - steps) + 1;
+    if (lost_at) limit = min(limit, __builtin_ctzll(lost_at));  // tried again as a round's first
+    int adv = limit;
+    if (accepted & ((1ull << (limit - 1)) - 1)) {  // one before the last: what did the later trials read?
+      if (!commit && wave < limit) {
+        const uint64_t before = accepted & ((1ull << wave) - 1);
+        const uint32_t p = L.p[wave], q = L.q[wave];
+        const bool drew = lane <= win, in = lane < kSiteSlots;
+        const bool drew2 = (seen >> lane) & 1;
+        constexpr int kReads = 6;
+        const uint32_t read[kReads] = {drew ? a : p, drew ? b : p, drew2 ? a2 : p, drew2 ? b2 : p, in ? sp : p, in ? sq : p};
+        uint8_t v[kReads];
+#pragma unroll
+        for (int k = 0; k < kReads; ++k) v[k] = occ[read[k]];
+        // its own two sites against theirs, its other sites through the marks
+        bool hit = lane < wave && swap && (tp == p || tp == q || tq == p || tq == q);
+        bool marked = false;
+#pragma unroll
+        for (int k = 0; k < kReads; ++k) marked |= (v[k] & kMark) != 0 && read[k] != p && read[k] != q;
+        if (win < 0 && before) hit = true;
+        if (__ballot(marked)) {  // by one of the trials before it?
+          for (uint64_t e = before; e; e &= e - 1) {
+            const int i = __builtin_ctzll(e);
+            const uint32_t pi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(tp), i));
+            const uint32_t qi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(tq), i));
+#pragma unroll
+            for (int k = 0; k < kReads; ++k) hit |= read[k] == pi || read[k] == qi;
+          }
         }
         const uint64_t mh = __ballot(hit);
-        if (lane == 0) s_conf = (!hasB || TB.win < 0 || mh) ? 1 : 0;
+        if (lane == 0) L.conflict[wave] = mh ? 1 : 0;
       }
+      __syncthreads();
+      const uint64_t stop = __ballot(lane < limit && L.conflict[slot]);
+      if (stop) adv = __builtin_ctzll(stop);
     }
-    __syncthreads();
-    if (tid == kAcceptThread) {
-      double de = 0.0;
-      for (int w = 0; w < kThreads / 64; ++w) de += L.part[w];
-      const double T = c.anneal ? s_T : 0.0;
-      const bool acc_a = metropolis(steps, trace_base + it, s_tr[0], de, T, c.anneal ? s_bA : 0.0);
-      int adv = 1;
-      const bool b_ok = s_tr[1].win != -2 && !(acc_a && s_conf);
-      if (steps + 1 <= maxs && it + 1 < ntrials && b_ok) {
-        double deb = 0.0;
-        for (int w = 0; w < kThreads / 64; ++w) deb += L.part2[w];
-        (void)metropolis(steps + 1, trace_base + it + 1, s_tr[1], deb, T * decay,
-                         c.anneal ? s_bB : 0.0);
-        adv = 2;
+    active = min(adv == limit ? active + 2 : max(max(adv + 3, active - 2), 4), kCmcWaves);
+    if (commit) {
+      const double tde = L.de[slot];
+      const bool mine = lane < adv && swap;
+      if (swap && !mine) {  // not taken this round: the marks go
+        occ[tp] = L.ep[slot];
+        occ[tq] = L.eq[slot];
       }
-      s_adv = adv;
-      if (c.anneal) s_T = A.T;
-      if (steps + adv > maxs) s_done = 1;
-    } else if (wave < 2) {
-      cand = DrawAttempt(c, r, steps + 2 + wave, static_cast<uint32_t>(lane), N, n);
-    } else if (tid == 128) {
-      draw_ahead(steps + 2);
-      draw_ahead(steps + 3);
+      if (lane < adv) {
+        const uint64_t index = trace_base + it + static_cast<uint64_t>(lane);
+        if (index < c.trace_cap) {
+          const uint64_t o = static_cast<uint64_t>(r) * c.trace_cap + index;
+          c.tr_p[o] = tp;
+          c.tr_q[o] = tq;
+          c.tr_de[o] = tde;
+          c.tr_acc[o] = mine ? 1 : 0;
+        }
+      }
+      if (mine) {  // the accepted trials' sites are disjoint
+        if (c.atom) {
+          const int64_t o = c.off[r];
+          const XYZ xp = ToXYZ32(tp, n), xq = ToXYZ32(tq, n);
+          AtomJump(c.atom + o, c.shift + 3 * o, tp, tq, ImageChange(xq.X - xp.X, n),
+                   ImageChange(xq.Y - xp.Y, n), ImageChange(xq.Z - xp.Z, n));
+        }
+        occ[tp] = L.eq[slot];
+        occ[tq] = L.ep[slot];
+      }
+      // energies, records and the schedule in trial order
+      const int at0 = static_cast<int>(steps & (kCmcRing - 1));
+      if (kLog || c.anneal) {
+        for (int j = 0; j < adv; ++j) {
+          const uint64_t step = steps + static_cast<uint64_t>(j);
+          const bool on = (accepted >> j) & 1;
+          if constexpr (kLog) {
+            if (c.avg_m) {  // ThermodynamicAveraging::AddEnergy before Dump (CanonicalMcSerial.cpp:45)
+              if (lane == 0) c.ring[static_cast<uint64_t>(r) * c.ring_cap + ring_at] = energy;
+              if (++ring_at == c.ring_cap) ring_at = 0;
+              ++ring_i;
+            }
+          }
+          if (c.anneal) {
+            const bool lower = energy < A.lowest - 1e-4;  // Dump (SimulatedAnnealing.cpp:80-97)
+            if (lower) A.lowest = energy;
+            if constexpr (kLog) {
+              if (lower) put_log(step, A.T, A.lowest);
+              if (clk.Due(step)) put_log(step, A.T, A.lowest);
+            }
+          } else if constexpr (kLog) {
+            if (clk.Due(step)) put_log(step, L.T[(at0 + j) & (kCmcRing - 1)], 0.0);
+          }
+          if (on) {
+            const double de = ReadLane(tde, j);
+            energy += de;
+            abse += de;
+            ++acc;
+          }
+          if (c.anneal) AnnealUpdate(A, sched, on, step, energy);
+        }
+      } else {
+        const double taken = mine ? tde : 0.0;
+#pragma unroll
+        for (int j = 0; j < kCmcWaves; ++j) {
+          const double de = ReadLane(taken, j);
+          energy += de;
+          abse += de;
+        }
+        acc += __builtin_popcountll(__ballot(mine));
+      }
+      if (c.anneal) set_betas(steps + static_cast<uint64_t>(adv));
+    } else if (wave < active) {
+      draw(steps + static_cast<uint64_t>(adv + wave));
     }
+    steps += static_cast<uint64_t>(adv);
+    it += static_cast<uint64_t>(adv);
     __syncthreads();
-    const int adv = s_adv;
-    fresh = adv == 2;
-    steps += adv;
-    it += adv;
   }
   if constexpr (kLdsOcc) {
     __syncthreads();
     uint32_t *dst = reinterpret_cast<uint32_t *>(c.occ + c.off[r]);
-    for (uint64_t i = tid; i < N / 4; i += kThreads) dst[i] = occ_words[i];
+    for (uint64_t i = tid; i < N / 4; i += kCmcThreads) dst[i] = occ_words[i];
   }
-  if (tid == kAcceptThread) {
+  if (commit && lane == 0) {
+    if (lost) atomicOr(c.error, 2);
     c.steps[r] = steps;
     c.accepted[r] = acc;
     c.energy[r] = energy;
@@ -890,7 +1010,7 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, SiteLds &L, Omp
       double v = 0.0;
 #pragma unroll 4
       for (int i = 0; i < kOmpChunkLen; ++i) {
-        const SiteCluster q = DecodeSiteCluster(t, L, ch * kOmpChunkLen + i);
+        const SiteCluster q = DecodeSiteCluster(t, L.cl, ch * kOmpChunkLen + i);
         v += ClusterDeltaAt(L, q, ea, ep, eq, sa) + ClusterDeltaAt(L, q, eb, eq, ep, sb);
       }
       O.u.part[ch][e] = v;
@@ -1586,8 +1706,8 @@ hipError_t LaunchCmc(const KTables &t, const CmcDev &c, uint64_t trials, uint64_
     return c.log_every
                ? launch(CmcOmpKernel<true, true>, CmcOmpKernel<false, true>, st_omp, kOmpThreads)
                : launch(CmcOmpKernel<true, false>, CmcOmpKernel<false, false>, st_omp, kOmpThreads);
-  return c.log_every ? launch(CmcKernel<true, true>, CmcKernel<false, true>, st_serial, kThreads)
-                     : launch(CmcKernel<true, false>, CmcKernel<false, false>, st_serial, kThreads);
+  return c.log_every ? launch(CmcKernel<true, true>, CmcKernel<false, true>, st_serial, kCmcThreads)
+                     : launch(CmcKernel<true, false>, CmcKernel<false, false>, st_serial, kCmcThreads);
 }
 
 hipError_t LaunchCmcAverage(const CmcDev &c, hipStream_t s) {

@@ -623,6 +623,7 @@ struct lmc_cmc {
     DevFree(d.omp_de);
     DevFree(d.omp_len);
     DevFree(d.omp_pos);
+    DevFree(d.omp_ref);
     DevFree(d.anneal);
     DevFree(d.atom);
     DevFree(d.shift);
@@ -1844,6 +1845,7 @@ int lmc_cmc_set_parallel_trials(lmc_cmc *c, int32_t trials_per_round) {
     DevFree(c->d.omp_de);
     DevFree(c->d.omp_len);
     DevFree(c->d.omp_pos);
+    DevFree(c->d.omp_ref);
     c->d.omp_k = trials_per_round;
     if (!trials_per_round) return LMC_OK;
     const size_t R = static_cast<size_t>(c->d.R), n = R * static_cast<size_t>(trials_per_round);
@@ -1852,6 +1854,9 @@ int lmc_cmc_set_parallel_trials(lmc_cmc *c, int32_t trials_per_round) {
     c->d.omp_de = DevAlloc<double>(n);
     c->d.omp_len = DevCopy(std::vector<int32_t>(R, 0));
     c->d.omp_pos = DevCopy(std::vector<int32_t>(R, 0));
+    c->d.omp_ref = DevAlloc<uint8_t>(R);
+    Check(lmc::LaunchCmcReference(lmc::Upload(*c->pm->m), c->d, c->d.omp_ref, nullptr), "species kernel");
+    Check(hipDeviceSynchronize(), "hipDeviceSynchronize");
     return LMC_OK;
   });
 }

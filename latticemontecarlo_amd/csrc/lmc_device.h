@@ -183,6 +183,7 @@ struct CmcDev {
   int64_t *omp_p = nullptr, *omp_q = nullptr;
   double *omp_de = nullptr;
   int32_t *omp_len = nullptr, *omp_pos = nullptr;
+  uint8_t *omp_ref = nullptr;  // [R] the most frequent species
 };
 
 // env_out (optional): [12 R][64] environment rows of the events in rank order; ekra_out
@@ -211,6 +212,8 @@ hipError_t LaunchSwapDe(const KTables &t, const uint8_t *occ, const int64_t *off
 hipError_t LaunchSiteDe(const KTables &t, const uint8_t *occ, const int64_t *off,
                         const int32_t *ncell, const int64_t *sites, const uint8_t *from,
                         const uint8_t *codes, int32_t R, double *de, hipStream_t s);
+// The most frequent species of each replica into ref[R].
+hipError_t LaunchCmcReference(const KTables &t, const CmcDev &c, uint8_t *ref, hipStream_t s);
 // The thermodynamic averages of the canonical-MC log records of the last launch
 // (ThermodynamicAveraging::GetThermodynamicAverage, ThermodynamicAveraging.cpp:25-40).
 hipError_t LaunchCmcAverage(const CmcDev &c, hipStream_t s);

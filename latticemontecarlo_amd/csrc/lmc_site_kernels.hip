@@ -218,23 +218,18 @@ __device__ void AnnealUpdate(CmcAnneal &A, const AnnealSchedule &s, bool accepte
 
 constexpr uint32_t kMaxPairAttempts = 1u << 20;
 
-// Draw attempt att of step `steps` (Philox counter 2 att + 1): the two sites and their
-// coordinates. CanonicalMcAbstract.cpp:43-101 redraws until the species differ; lane l of a
-// wave holds attempt base + l, so the lowest lane of the first round with a hit is the
-// sequential answer.
-struct PairDraw {
-  int64_t a, b;
-  XYZ xa, xb;
-};
-__device__ __forceinline__ PairDraw DrawAttempt(const CmcDev &c, int r, uint64_t steps,
-                                                uint32_t att, uint64_t N, int n) {
-  const U4 u = Philox4x32_10(c.seed[r], steps, c.rid[r], 2u * att + 1u);
-  PairDraw d;
-  d.a = static_cast<int64_t>(MulHi64(Join64(u.x, u.y), N));
-  d.b = static_cast<int64_t>(MulHi64(Join64(u.z, u.w), N));
-  d.xa = ToXYZ32(static_cast<uint32_t>(d.a), static_cast<uint32_t>(n));
-  d.xb = ToXYZ32(static_cast<uint32_t>(d.b), static_cast<uint32_t>(n));
-  return d;
+// A pair draw attempt is Philox counter 2 attempt + 1 of the trial's (the round's) first step;
+// CanonicalMcAbstract.cpp:43-101 redraws until the species differ, so the lowest attempt with different
+// species is the sequential answer.
+
+// Site coordinates X, Y < 2^11 and Z / 2 < 2^10 in one word (every box has n <= 1000).
+__device__ __forceinline__ uint32_t PackSiteXYZ(uint32_t site, uint32_t n) {
+  const uint32_t plane = 2u * n * n, X = site / plane, rest = site - X * plane, Y = rest / n;
+  return X | Y << 11 | (rest - Y * n) << 22;
+}
+__device__ __forceinline__ XYZ UnpackSiteXYZ(uint32_t v) {
+  const int X = v & 2047, Y = (v >> 11) & 2047;
+  return {X, Y, static_cast<int>(v >> 22) * 2 + ((X + Y) & 1)};
 }
 
 // Metropolis uniform of step `steps`.
@@ -437,19 +432,11 @@ __global__ __launch_bounds__(kCmcThreads) void CmcKernel(KTables t, CmcDev c, ui
     }
     ++log_i;  // counts past the capacity too, so the host can report the loss
   };
-  // attempts (and the uniform, in lane 63 of the first draw) of a step; their coordinates X, Y < 2^11
-  // and Z / 2 < 2^10 in one word
+  // attempts (and the uniform, in lane 63 of the first draw) of a step, and their coordinates
   uint32_t a = 0, b = 0, xa = 0, xb = 0, a2 = 0, b2 = 0;
   bool dilute = false, second = false;  // second: a2, b2 hold the 64 attempts after the first 63
   double uni = 0.0;
-  auto pack = [&](uint32_t site) {
-    const uint32_t plane = 2u * n * n, X = site / plane, rest = site - X * plane, Y = rest / n;
-    return X | Y << 11 | (rest - Y * n) << 22;
-  };
-  auto unpack = [](uint32_t v) -> XYZ {
-    const int X = v & 2047, Y = (v >> 11) & 2047;
-    return {X, Y, static_cast<int>(v >> 22) * 2 + ((X + Y) & 1)};
-  };
+  auto pack = [&](uint32_t site) { return PackSiteXYZ(site, n); };
   auto draw = [&](uint64_t step) {
     const U4 u = Philox4x32_10(seed, step, rid, lane == kCmcFirst ? 0xFFFFFFFEu : 2u * lane + 1u);
     second = dilute;
@@ -529,7 +516,7 @@ __global__ __launch_bounds__(kCmcThreads) void CmcKernel(KTables t, CmcDev c, ui
           return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), at));
         };
         const uint32_t p = lane_of(ta), q = lane_of(tb);
-        const XYZ xp = unpack(lane_of(txa)), xq = unpack(lane_of(txb));
+        const XYZ xp = UnpackSiteXYZ(lane_of(txa)), xq = UnpackSiteXYZ(lane_of(txb));
         sp = static_cast<uint32_t>(SiteAt(xp, n, ox, oy, oz));
         sq = static_cast<uint32_t>(SiteAt(xq, n, ox, oy, oz));
         const int vp = occ[sp] & ~kMark, vq = occ[sq] & ~kMark;
@@ -759,45 +746,59 @@ __global__ __launch_bounds__(kCmcThreads) void CmcKernel(KTables t, CmcDev c, ui
 //
 // One 1024-thread workgroup per replica (the canonical workloads have few replicas, so a CU
 // each; 16 waves hide the phases' latencies). Per round:
-//   draw   : passes of 1024 attempts, one per thread, species checked in parallel; the first 128
-//            valid attempts of a pass ranked by ballots; their exclusion by the round's earlier
-//            events and their pairwise conflicts checked by 8 threads each (LDS atomics); then
-//            one lane walks them in order (the reference's do/while with its draw count);
-//   dE     : both 43-site environments of every event gathered at once; thread (chunk, event)
-//            adds the changes of 16 site clusters for both swapped sites, and the 16 chunk sums
-//            of an event are added in chunk order;
-//   trials : event lanes test their Metropolis steps in parallel and apply the accepted swaps;
-//            one lane adds the energies in trial order (and takes the log records).
+//   draw   : passes of 1024 attempts, one per thread, species checked in parallel; the first valid
+//            attempts of a pass (24 more than events are wanted: a few meet another one) ranked by
+//            ballots; their pairs, spread evenly over the threads, tested for conflicts; then wave 0
+//            takes them in order by ballots (the reference's do/while with its draw count), while wave 1
+//            draws the round's Metropolis uniforms;
+//   dE     : a wave gathers an environment at a time and notes which sites are not of the replica's
+//            most frequent species; eight threads to an environment add those sites' terms and their
+//            pairs' (see OmpTables);
+//   trials : event lanes test their Metropolis steps in parallel; the accepted swaps are applied while
+//            wave 0 adds the energies in trial order (and takes the log records).
+// Bound by the latency of these phases. 64 replicas of 30^3 cells, 5 at.% solute, 20 000 trials in
+// rounds of 64: 15.2 -> 7.6 ms (all site clusters of both sites for every event, conflicts by rows and one
+// lane walking the draws and the energies, before); 6^3 cells, 2 000 trials: 12.1 -> 6.9 ms.
 constexpr int kOmpThreads = 1024;
 constexpr int kOmpMaxK = 64;
 constexpr int kOmpPass = kOmpThreads;          // attempts per draw pass
 constexpr int kOmpMaxValid = 128;              // valid attempts resolved per pass
-constexpr int kOmpGroups = kOmpThreads / kOmpMaxValid;  // checking threads per valid attempt
-constexpr int kOmpChunks = kOmpThreads / kOmpMaxK;      // cluster chunks per event
-constexpr int kOmpChunkLen = kMaxSiteClusters / kOmpChunks;
-static_assert(kOmpChunks * kOmpChunkLen == kMaxSiteClusters, "chunks cover the site clusters");
+constexpr int kOmpSpare = 24;
+constexpr int kOmpShare = kOmpThreads / (2 * kOmpMaxK);  // threads per environment
+static_assert(kOmpShare == 8 && kOmpMaxK + kOmpSpare <= kOmpMaxValid, "");
 
 struct OmpDraw {  // one draw pass: its valid attempts in attempt order
-  int64_t va[kOmpMaxValid], vb[kOmpMaxValid];
-  XYZ vxa[kOmpMaxValid], vxb[kOmpMaxValid];
+  uint32_t va[kOmpMaxValid], vb[kOmpMaxValid], xa[kOmpMaxValid], xb[kOmpMaxValid];
   uint32_t conf[kOmpMaxValid][kOmpMaxValid / 32];  // bit j: conflicts with valid attempt j
   uint32_t excl[kOmpMaxValid];                     // meets an earlier pass's event
   int vidx[kOmpMaxValid];
 };
 
+// The cluster sum of a centre species x over an environment, over the sites that are not of the
+// reference species r only: E(x) = base(x) + sum f1[shell][x][c] + sum over their pairs of
+// f2[label][x][c][c'], with g[label][x][c] = w3(x, c, r) - w3(x, r, r),
+//   f2 = (w3(x, c, c') - w3(x, c, r)) - g(x, c'), f1 = w2(x, c) - w2(x, r) + sum of g over the sites that
+// form a triplet with it. Exact for every composition; the bases of a swap's two sites cancel.
+struct OmpTables {
+  double f[kMaxW];  // as w: f1 at S, f2 at S + 3 S S
+  double g[kMaxW / 4];
+  uint64_t with[kSiteSlots];               // the slots that form a triplet with a slot and the centre
+  uint8_t label[kSiteSlots][kSiteSlots];   // its label 1..4, 0 for none
+  uint8_t shell[kSiteSlots];               // 0..2
+};
+
 struct OmpLds {
+  OmpTables t;
+  int32_t off[kSiteSlots];
   uint8_t env[2 * kOmpMaxK][48];
+  uint64_t other[2 * kOmpMaxK];  // slots not of the reference species
   int slot[2 * kOmpMaxK];
-  XYZ ch[2 * kOmpMaxK];  // sites of the round's events so far
-  int64_t p[kOmpMaxK], q[kOmpMaxK];
-  XYZ xp[kOmpMaxK], xq[kOmpMaxK];
-  int ep[kOmpMaxK], eq[kOmpMaxK];
-  double de[kOmpMaxK];
+  uint32_t ch[2 * kOmpMaxK];  // sites of the round's events so far
+  uint32_t p[kOmpMaxK], q[kOmpMaxK], xp[kOmpMaxK], xq[kOmpMaxK];
+  uint8_t ep[kOmpMaxK], eq[kOmpMaxK];
+  double de[kOmpMaxK], uni[kOmpMaxK], beta[kOmpMaxK];
   int8_t acc[kOmpMaxK];
-  union {
-    OmpDraw d;                          // draw phase
-    double part[kOmpChunks][kOmpMaxK];  // dE phase
-  } u;
+  OmpDraw d;
   int wave_valid[kOmpThreads / 64];
   int8_t slot_lut[125];  // env slot of offset (dx, dy, dz) in [-2, 2]^3, -1 beyond the 3rd shell
   // round control
@@ -805,26 +806,82 @@ struct OmpLds {
   uint32_t att0;
 };
 
+// Tables of reference species ref (all threads; a barrier follows).
+__device__ void LoadOmpTables(const KTables &t, OmpLds &O, int ref) {
+  const int tid = threadIdx.x, S = t.S, SS = S * S, w3 = S + 3 * SS;
+  OmpTables &T = O.t;
+  for (int i = tid; i < kSiteSlots * kSiteSlots; i += kOmpThreads) T.label[i / kSiteSlots][i % kSiteSlots] = 0;
+  if (tid < kSiteSlots) {
+    T.with[tid] = 0;
+    T.shell[tid] = 0;
+    O.off[tid] = t.site_off[tid];
+  }
+  if (tid < 125) O.slot_lut[tid] = -1;
+  for (int i = tid; i < 4 * SS; i += kOmpThreads) {
+    const int at = w3 + (i / SS) * SS * S + (i % SS) * S + ref, x = i / S % S;
+    T.g[i] = t.w[at] - t.w[w3 + (i / SS) * SS * S + (x * S + ref) * S + ref];
+  }
+  __syncthreads();
+  for (int i = tid; i < t.n_site; i += kOmpThreads) {
+    const uint32_t d = t.site_cl[i];
+    const int label = d & 7, a = (d >> 4) & 63, b = (d >> 10) & 63;
+    if (label >= 4) {
+      T.label[a][b] = T.label[b][a] = static_cast<uint8_t>(label - 3);
+      atomicOr(reinterpret_cast<unsigned long long *>(&T.with[a]), 1ull << b);
+      atomicOr(reinterpret_cast<unsigned long long *>(&T.with[b]), 1ull << a);
+    } else if (label) {
+      T.shell[a] = static_cast<uint8_t>(label - 1);
+    }
+  }
+  for (int i = tid; i < 4 * SS * S; i += kOmpThreads) {
+    const int l = i / (SS * S), x = i / SS % S, c = i / S % S, e = i % S;
+    const double *w = t.w + w3 + l * SS * S;
+    T.f[w3 + i] = c == ref || e == ref ? 0.0
+                                       : (w[(x * S + c) * S + e] - w[(x * S + c) * S + ref]) -
+                                             T.g[l * SS + x * S + e];
+  }
+  if (tid >= 1 && tid < kSiteSlots) {
+    int x, y, z;
+    Unpack(O.off[tid], x, y, z);
+    O.slot_lut[(x + 2) * 25 + (y + 2) * 5 + (z + 2)] = static_cast<int8_t>(tid);
+  }
+  __syncthreads();
+  for (int i = tid; i < 3 * SS; i += kOmpThreads) {
+    const int sh = i / SS;
+    int at = 1;  // a slot of that shell; all of them have the same triplets
+    while (T.shell[at] != sh) ++at;
+    double v = t.w[S + i] - t.w[S + sh * SS + (i / S % S) * S + ref];
+    for (int b = 1; b < kSiteSlots; ++b)
+      if (T.label[at][b]) v += T.g[(T.label[at][b] - 1) * SS + i % SS];
+    T.f[S + i] = v;
+  }
+  __syncthreads();
+}
+
 // Whether site b lies on site a or in its 1st-3rd neighbour shells (squared minimum-image
 // distance at most 6 in (a/2)^2; FCC distances are even).
 __device__ __forceinline__ bool Near(const XYZ &a, const XYZ &b, int n) {
-  const int dx = MinImage(b.X - a.X, n), dy = MinImage(b.Y - a.Y, n), dz = MinImage(b.Z - a.Z, n);
-  return dx * dx + dy * dy + dz * dz <= 6;
+  const int m = 2 * n;
+  const int dx = abs(b.X - a.X), dy = abs(b.Y - a.Y), dz = abs(b.Z - a.Z);
+  const int x = min(dx, m - dx), y = min(dy, m - dy), z = min(dz, m - dz);
+  return x * x + y * y + z * z <= 6;
 }
 
-// w(x -> en) - w(x -> eo) of cluster q in environment e, 0 when it contains slot skip.
-__device__ __forceinline__ double ClusterDeltaAt(const SiteLds &L, const SiteCluster &q,
-                                                 const uint8_t *e, int eo, int en, int skip) {
-  if (!q.live || (skip >= 0 && (q.r1 == skip || q.r2 == skip))) return 0.0;
-  const int rest = q.base + e[q.o1] * q.k1 + e[q.o2] * q.k2;
-  return L.w[rest + en * q.kx] - L.w[rest + eo * q.kx];
+// Metropolis uniforms and ramp betas of the round's events, the first at step s0 (one wave).
+__device__ __forceinline__ void OmpDrawTests(const CmcDev &c, OmpLds &O, int r, uint64_t s0, uint64_t maxs, int K) {
+  const int e = threadIdx.x & 63;
+  if (e >= K) return;
+  const uint64_t step = s0 + static_cast<uint64_t>(e);
+  O.uni[e] = TrialUniform(c, r, step);
+  const double T = c.t0[r] + (c.t1[r] - c.t0[r]) * (static_cast<double>(step) / static_cast<double>(maxs));
+  O.beta[e] = 1.0 / kBoltzmann / T;
 }
 
 // The round starting at step s0: pairs, environments, partner slots and dE into O (all threads).
-__device__ void BuildOmpRound(const KTables &t, const CmcDev &c, SiteLds &L, OmpLds &O, int r,
-                              uint64_t s0, const uint8_t *occ, uint64_t N, int n, int K) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  OmpDraw &D = O.u.d;
+__device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int r, uint64_t s0, uint64_t maxs,
+                              const uint8_t *occ, uint64_t N, int n, int K, int ref) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  OmpDraw &D = O.d;
   if (tid == 0) {
     O.len = 0;
     O.nch = 0;
@@ -832,51 +889,57 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, SiteLds &L, Omp
     O.finished = 0;
     O.att0 = 0;
   }
+  if (tid < kOmpMaxValid) {
+    D.excl[tid] = 0;
+    for (int w = 0; w < kOmpMaxValid / 32; ++w) D.conf[tid][w] = 0;
+  }
   __syncthreads();
+  bool first = true;
   while (!O.finished) {
-    const PairDraw d = DrawAttempt(c, r, s0, O.att0 + static_cast<uint32_t>(tid), N, n);
-    const bool valid = occ[d.a] != occ[d.b];
+    const U4 u4 = Philox4x32_10(c.seed[r], s0, c.rid[r], 2u * (O.att0 + static_cast<uint32_t>(tid)) + 1u);
+    const uint32_t a = static_cast<uint32_t>(MulHi64(Join64(u4.x, u4.y), N));
+    const uint32_t b = static_cast<uint32_t>(MulHi64(Join64(u4.z, u4.w), N));
+    const bool valid = occ[a] != occ[b];
     const uint64_t m = __ballot(valid);
     if (lane == 0) O.wave_valid[wave] = __builtin_popcountll(m);
     __syncthreads();
-    int u = __builtin_popcountll(m & ((1ull << lane) - 1));
-    for (int w = 0; w < wave; ++w) u += O.wave_valid[w];
-    int total = 0;
-    for (int w = 0; w < kOmpThreads / 64; ++w) total += O.wave_valid[w];
-    const int nv = total < kOmpMaxValid ? total : kOmpMaxValid;
-    if (valid && u < kOmpMaxValid) {
-      D.va[u] = d.a;
-      D.vb[u] = d.b;
-      D.vxa[u] = d.xa;
-      D.vxb[u] = d.xb;
+    // valid attempts of the waves before this one, and in all (a running sum over each row of 16 lanes)
+    int run = O.wave_valid[lane & 15];
+    run += __builtin_amdgcn_update_dpp(0, run, 0x111, 0xF, 0xF, true);
+    run += __builtin_amdgcn_update_dpp(0, run, 0x112, 0xF, 0xF, true);
+    run += __builtin_amdgcn_update_dpp(0, run, 0x114, 0xF, 0xF, true);
+    run += __builtin_amdgcn_update_dpp(0, run, 0x118, 0xF, 0xF, true);
+    const int total = __builtin_amdgcn_readlane(run, 15);
+    const int u = (wave ? __builtin_amdgcn_readlane(run, wave - 1) : 0) +
+                  __builtin_popcountll(m & ((1ull << lane) - 1));
+    const int len0 = O.len, nch0 = O.nch;
+    const int cap = K - len0 + kOmpSpare;  // at most kOmpMaxValid
+    const int nv = total < cap ? total : cap;
+    if (valid && u < nv) {
+      D.va[u] = a;
+      D.vb[u] = b;
+      D.xa[u] = PackSiteXYZ(a, n);
+      D.xb[u] = PackSiteXYZ(b, n);
       D.vidx[u] = tid;
     }
-    if (tid < kOmpMaxValid) {
-      D.excl[tid] = 0;
-      for (int w = 0; w < kOmpMaxValid / 32; ++w) D.conf[tid][w] = 0;
-    }
     __syncthreads();
-    {  // thread (g, v): the g-th share of valid attempt v's checks
-      const int v = tid % kOmpMaxValid, g = tid / kOmpMaxValid;
-      if (v < nv) {
-        const XYZ a = D.vxa[v], b = D.vxb[v];
-        bool ex = false;
-        for (int j = g; j < O.nch; j += kOmpGroups) ex = ex || Near(O.ch[j], a, n) || Near(O.ch[j], b, n);
-        if (ex) atomicOr(&D.excl[v], 1u);
-        static_assert(kOmpMaxValid == 128, "conflict masks are two 64-bit words");
-        uint64_t lo = 0, hi = 0;  // registers, not a run-time indexed array
-        for (int j = g; j < v; j += kOmpGroups) {
-          const bool hit = Near(D.vxa[j], a, n) || Near(D.vxa[j], b, n) || Near(D.vxb[j], a, n) ||
-                           Near(D.vxb[j], b, n);
-          if (hit) {
-            if (j < 64) lo |= 1ull << j;
-            else hi |= 1ull << (j - 64);
-          }
+    if (nv > 0) {
+      const float per = 1.0f / static_cast<float>(nv);
+      auto meet = [&](const XYZ &s, int v) {
+        return Near(s, UnpackSiteXYZ(D.xa[v]), n) || Near(s, UnpackSiteXYZ(D.xb[v]), n);
+      };
+      // every pair of attempts once: (v, v + d mod nv) for d up to half way round
+      for (int i = tid; i < nv * (nv / 2); i += kOmpThreads) {
+        const int d = static_cast<int>((i + 0.5f) * per), v = i - d * nv;  // i < 2^13: exact
+        const int w = v + d + 1 >= nv ? v + d + 1 - nv : v + d + 1;
+        if (meet(UnpackSiteXYZ(D.xa[v]), w) || meet(UnpackSiteXYZ(D.xb[v]), w)) {
+          const int lo = min(v, w);
+          atomicOr(&D.conf[max(v, w)][lo >> 5], 1u << (lo & 31));
         }
-        if (lo & 0xFFFFFFFFull) atomicOr(&D.conf[v][0], static_cast<uint32_t>(lo));
-        if (lo >> 32) atomicOr(&D.conf[v][1], static_cast<uint32_t>(lo >> 32));
-        if (hi & 0xFFFFFFFFull) atomicOr(&D.conf[v][2], static_cast<uint32_t>(hi));
-        if (hi >> 32) atomicOr(&D.conf[v][3], static_cast<uint32_t>(hi >> 32));
+      }
+      for (int i = tid; i < nv * nch0; i += kOmpThreads) {  // against the events of earlier passes
+        const int j = static_cast<int>((i + 0.5f) * per), v = i - j * nv;  // i < 2^14: exact
+        if (meet(UnpackSiteXYZ(O.ch[j]), v)) D.excl[v] = 1;
       }
     }
     __syncthreads();
@@ -885,7 +948,7 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, SiteLds &L, Omp
       // unless it meets an earlier pass's event or conflicts with an attempt taken before it.
       // Lane l decides attempts l and l + 64 as soon as every earlier attempt it conflicts with
       // is decided (ballots; the chains of conflicts are short), then the draw count and K cut
-      // the taken set (a wave-uniform scan), and the taken attempts become the next events.
+      // the taken set, and the taken attempts become the next events.
       const int v0 = lane, v1 = lane + 64;
       const uint64_t c0 = v0 < nv ? D.conf[v0][0] | (static_cast<uint64_t>(D.conf[v0][1]) << 32) : 0;
       const uint64_t c1lo = v1 < nv ? D.conf[v1][0] | (static_cast<uint64_t>(D.conf[v1][1]) << 32) : 0;
@@ -907,124 +970,115 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, SiteLds &L, Omp
         alo = __ballot(a0);
         ahi = __ballot(a1);
       }
-      // draw count and K (wave-uniform): draw v of the current event has count base + v - last
-      const int len0 = O.len, nch0 = O.nch;
-      int base = O.ct, last = -1, len = len0;
-      bool fin = false;
-      uint64_t tlo = 0, thi = 0, rlo = alo, rhi = ahi;
-      while (true) {
-        const int p = rlo ? __builtin_ctzll(rlo) : (rhi ? 64 + __builtin_ctzll(rhi) : nv);
-        if (p >= nv) {  // no further taken attempt in this pass
-          if (base + (nv - 1 - last) >= 50) fin = true;
-          else base += nv - 1 - last;
-          break;
-        }
-        if (base + (p - last) >= 50) {  // the 50th draw of the event comes first
-          fin = true;
-          break;
-        }
-        if (p < 64) {
-          tlo |= 1ull << p;
-          rlo &= rlo - 1;
-        } else {
-          thi |= 1ull << (p - 64);
-          rhi &= rhi - 1;
-        }
-        ++len;
-        base = 0;
-        last = p;
-        if (len == K) {
-          fin = true;
-          break;
-        }
-      }
-      const bool t0 = (tlo >> v0) & 1, t1 = (thi >> v0) & 1;
-      if (t0 || t1) {
-        const int v = t0 ? v0 : v1;
-        const int e = len0 + (t0 ? __builtin_popcountll(tlo & ((1ull << v0) - 1))
-                                 : __builtin_popcountll(tlo) +
-                                       __builtin_popcountll(thi & ((1ull << v0) - 1)));
+      // An event's draws: from the taken attempt before it (the first one's go on from the pass before).
+      // The 50th draw of an event ends the round, and so does event K.
+      const uint64_t below = (1ull << lane) - 1, b0 = alo & below, b1 = ahi & below;
+      auto top = [](uint64_t v) { return 63 - __builtin_clzll(v); };
+      const int ct = O.ct;
+      const int n0 = b0 ? v0 - top(b0) : ct + v0 + 1;
+      const int n1 = b1 ? lane - top(b1) : alo ? v1 - top(alo) : ct + v1 + 1;
+      const uint64_t late0 = __ballot(a0 && n0 >= 50), late1 = __ballot(a1 && n1 >= 50);
+      const int cut = late0 ? __builtin_ctzll(late0) : late1 ? 64 + __builtin_ctzll(late1) : kOmpMaxValid;
+      const int e0 = len0 + __builtin_popcountll(b0);
+      const int e1 = len0 + __builtin_popcountll(alo) + __builtin_popcountll(b1);
+      const bool t0 = a0 && v0 < cut && e0 < K, t1 = a1 && v1 < cut && e1 < K;
+      auto take = [&](int v, int e) {
         O.p[e] = D.va[v];
         O.q[e] = D.vb[v];
-        O.xp[e] = D.vxa[v];
-        O.xq[e] = D.vxb[v];
-        O.ch[nch0 + 2 * (e - len0)] = D.vxa[v];
-        O.ch[nch0 + 2 * (e - len0) + 1] = D.vxb[v];
-      }
-      if (t0 && t1) {  // the lane's second taken attempt
-        const int e = len0 + __builtin_popcountll(tlo) + __builtin_popcountll(thi & ((1ull << v0) - 1));
-        O.p[e] = D.va[v1];
-        O.q[e] = D.vb[v1];
-        O.xp[e] = D.vxa[v1];
-        O.xq[e] = D.vxb[v1];
-        O.ch[nch0 + 2 * (e - len0)] = D.vxa[v1];
-        O.ch[nch0 + 2 * (e - len0) + 1] = D.vxb[v1];
-      }
+        O.xp[e] = O.ch[2 * e] = D.xa[v];
+        O.xq[e] = O.ch[2 * e + 1] = D.xb[v];
+      };
+      if (t0) take(v0, e0);
+      if (t1) take(v1, e1);
+      const uint64_t tlo = __ballot(t0), thi = __ballot(t1);
       if (lane == 0) {
-        O.ct = base;
+        const int len = len0 + __builtin_popcountll(tlo) + __builtin_popcountll(thi);
+        const int last = thi ? 64 + top(thi) : tlo ? top(tlo) : -1;
+        const int open = last < 0 ? ct + nv : nv - 1 - last;  // draws of the event to come
+        bool fin = len == K || cut < kOmpMaxValid || open >= 50;
+        O.ct = open;
         O.len = len;
-        O.nch = nch0 + 2 * (len - len0);
+        O.nch = 2 * len;
         // the next pass starts after the last attempt looked at
-        const uint32_t adv = total > kOmpMaxValid ? static_cast<uint32_t>(D.vidx[nv - 1] + 1)
-                                                  : static_cast<uint32_t>(kOmpPass);
-        O.att0 += adv;
+        O.att0 += total > cap ? static_cast<uint32_t>(D.vidx[nv - 1] + 1) : static_cast<uint32_t>(kOmpPass);
         if (!fin && O.att0 >= kMaxPairAttempts) {
           O.error = 1;
           fin = true;
         }
         O.finished = fin ? 1 : 0;
       }
+      for (int v = lane; v < kOmpMaxValid; v += 64) {  // for the next pass
+        D.excl[v] = 0;
+        for (int w = 0; w < kOmpMaxValid / 32; ++w) D.conf[v][w] = 0;
+      }
+    } else if (wave == 1 && first) {
+      OmpDrawTests(c, O, r, s0, maxs, K);
     }
+    first = false;
     __syncthreads();
   }
   const int len = O.len;
-  // species, both environments and partner slots of every event
-  for (int e = tid; e < len; e += kOmpThreads) {
-    O.ep[e] = occ[O.p[e]];
-    O.eq[e] = occ[O.q[e]];
-  }
-  for (int i = tid; i < 2 * len * 64; i += kOmpThreads) {
-    const int e2 = i >> 6, j = i & 63;
-    if (j < kSiteSlots) {
-      int dx, dy, dz;
-      Unpack(L.off[j], dx, dy, dz);
-      const XYZ &x = (e2 & 1) ? O.xq[e2 >> 1] : O.xp[e2 >> 1];
-      const uint8_t v = occ[SiteAt(x, n, dx, dy, dz)];
-      O.env[e2][j] = v < t.S ? v : 0;  // codes are validated at creation
-    }
-  }
-  for (int e2 = tid; e2 < 2 * len; e2 += kOmpThreads) {  // partner slots
-    const XYZ &a = (e2 & 1) ? O.xq[e2 >> 1] : O.xp[e2 >> 1];
-    const XYZ &b = (e2 & 1) ? O.xp[e2 >> 1] : O.xq[e2 >> 1];
-    const int dx = MinImage(b.X - a.X, n), dy = MinImage(b.Y - a.Y, n), dz = MinImage(b.Z - a.Z, n);
-    const bool in = dx >= -2 && dx <= 2 && dy >= -2 && dy <= 2 && dz >= -2 && dz <= 2;
-    O.slot[e2] = in ? O.slot_lut[(dx + 2) * 25 + (dy + 2) * 5 + (dz + 2)] : -1;
-  }
-  __syncthreads();
-  {  // dE: thread (chunk, event) adds its chunk of site clusters for both swapped sites
-    const int e = tid % kOmpMaxK, ch = tid / kOmpMaxK;
-    if (e < len) {
-      const int ep = O.ep[e], eq = O.eq[e];
-      const uint8_t *ea = O.env[2 * e], *eb = O.env[2 * e + 1];
-      const int sa = O.slot[2 * e], sb = O.slot[2 * e + 1];
-      double v = 0.0;
+  {  // environments, a wave each
+    int ox = 0, oy = 0, oz = 0;
+    const bool in = lane < kSiteSlots;
+    if (in) Unpack(O.off[lane], ox, oy, oz);
 #pragma unroll 4
-      for (int i = 0; i < kOmpChunkLen; ++i) {
-        const SiteCluster q = DecodeSiteCluster(t, L.cl, ch * kOmpChunkLen + i);
-        v += ClusterDeltaAt(L, q, ea, ep, eq, sa) + ClusterDeltaAt(L, q, eb, eq, ep, sb);
+    for (int e2 = wave; e2 < 2 * len; e2 += kOmpThreads / 64) {
+      const XYZ x = UnpackSiteXYZ(e2 & 1 ? O.xq[e2 >> 1] : O.xp[e2 >> 1]);
+      const int v = in ? occ[SiteAt(x, n, ox, oy, oz)] : ref;
+      const int code = v < t.S ? v : 0;  // codes are validated at creation
+      const uint64_t m = __ballot(lane > 0 && code != ref && in);
+      if (in) O.env[e2][lane] = static_cast<uint8_t>(code);
+      if (lane == 0) {
+        O.other[e2] = m;
+        (e2 & 1 ? O.eq : O.ep)[e2 >> 1] = static_cast<uint8_t>(v);
       }
-      O.u.part[ch][e] = v;
+    }
+    if (tid < 2 * len) {  // partner slots
+      const XYZ xp = UnpackSiteXYZ(O.xp[tid >> 1]), xq = UnpackSiteXYZ(O.xq[tid >> 1]);
+      const XYZ &p = (tid & 1) ? xq : xp, &q = (tid & 1) ? xp : xq;
+      const int dx = MinImage(q.X - p.X, n), dy = MinImage(q.Y - p.Y, n), dz = MinImage(q.Z - p.Z, n);
+      const bool near = dx >= -2 && dx <= 2 && dy >= -2 && dy <= 2 && dz >= -2 && dz <= 2;
+      O.slot[tid] = near ? O.slot_lut[(dx + 2) * 25 + (dy + 2) * 5 + (dz + 2)] : -1;
     }
   }
   __syncthreads();
-  for (int e = tid; e < len; e += kOmpThreads) {
-    double sum = 0.0;
-    for (int ch = 0; ch < kOmpChunks; ++ch) sum += O.u.part[ch][e];
-    O.de[e] = sum;
-    const int64_t o = static_cast<int64_t>(r) * c.omp_k + e;
-    c.omp_p[o] = O.p[e];
-    c.omp_q[o] = O.q[e];
-    c.omp_de[o] = sum;
+  {  // dE: thread g of an environment adds the terms of the sites in slots g, g + 8, ...
+    const int e2 = tid / kOmpShare, g = tid % kOmpShare, S = t.S, SS = S * S;
+    double v = 0.0;
+    if (e2 < 2 * len) {
+      const uint8_t *env = O.env[e2];
+      const int eo = env[0], en = O.env[e2 ^ 1][0], skip = O.slot[e2];
+      const OmpTables &T = O.t;
+      uint64_t other = O.other[e2];
+      if (skip >= 0) other &= ~(1ull << skip);  // clusters with both sites keep their species
+      for (uint64_t i = other & (0x0101010101010101ull << g); i; i &= i - 1) {
+        const int a = __builtin_ctzll(i), ca = env[a];
+        const double *f1 = T.f + S + T.shell[a] * SS + ca;
+        v += f1[en * S] - f1[eo * S];
+        if (skip >= 0 && T.label[a][skip]) {
+          const double *h = T.g + (T.label[a][skip] - 1) * SS + ca;
+          v -= h[en * S] - h[eo * S];
+        }
+        for (uint64_t j = other & T.with[a] & ((~0ull << a) << 1); j; j &= j - 1) {
+          const int b = __builtin_ctzll(j);
+          const double *f2 = T.f + S + 3 * SS + (T.label[a][b] - 1) * SS * S + ca * S + env[b];
+          v += f2[en * SS] - f2[eo * SS];
+        }
+      }
+    }
+    v += RowShr<1>(v);
+    v += RowShr<2>(v);
+    v += RowShr<4>(v);  // lanes 7 and 15 of a row: the sums of its environments
+    v += RowShr<8>(v);
+    if ((lane & 15) == 15 && e2 < 2 * len) {
+      const int e = e2 >> 1;
+      const int64_t o = static_cast<int64_t>(r) * c.omp_k + e;
+      O.de[e] = v;
+      c.omp_p[o] = O.p[e];
+      c.omp_q[o] = O.q[e];
+      c.omp_de[o] = v;
+    }
   }
   if (tid == 0) O.pos = 0;
   __syncthreads();
@@ -1034,14 +1088,13 @@ template <bool kLdsOcc, bool kLog>
 __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
                                                             uint64_t ntrials,
                                                             uint64_t trace_base) {
-  __shared__ SiteLds L;
   __shared__ OmpLds O;
   __shared__ uint64_t s_steps;
   extern __shared__ uint32_t occ_words[];
   const int r = blockIdx.x;
-  const int tid = threadIdx.x;
-  LoadSiteTables(t, L);
-  const int n = c.ncell[r];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int n = c.ncell[r], ref = c.omp_ref[r];
+  LoadOmpTables(t, O, ref);
   const uint64_t N = 4ull * n * n * n;
   const int K = c.omp_k;
   uint8_t *occ = c.occ + c.off[r];
@@ -1054,18 +1107,13 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
   uint64_t acc = 0, log_i = 0, ring_i = 0, ring_at = 0;
   double energy = 0, abse = 0;
   LogClock clk;
-  if (tid < 125) O.slot_lut[tid] = -1;
-  __syncthreads();
-  if (tid >= 1 && tid < kSiteSlots) {  // the first slot of each offset (slot 0: the site itself)
-    int x, y, z;
-    Unpack(L.off[tid], x, y, z);
-    O.slot_lut[(x + 2) * 25 + (y + 2) * 5 + (z + 2)] = static_cast<int8_t>(tid);
-  }
-  if (tid == 0) {
-    s_steps = c.steps[r];
+  if (tid < 64) {  // wave 0 keeps the sums (the records: its first lane)
     acc = c.accepted[r];
     energy = c.energy[r];
     abse = c.abs_energy[r];
+  }
+  if (tid == 0) {
+    s_steps = c.steps[r];
     O.len = c.omp_len[r];
     O.pos = c.omp_pos[r];
     O.error = 0;
@@ -1086,19 +1134,17 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
   if (O.pos < O.len) {
     for (int e = tid; e < O.len; e += kOmpThreads) {
       const int64_t o = static_cast<int64_t>(r) * K + e;
-      O.p[e] = c.omp_p[o];
-      O.q[e] = c.omp_q[o];
+      O.p[e] = static_cast<uint32_t>(c.omp_p[o]);
+      O.q[e] = static_cast<uint32_t>(c.omp_q[o]);
       O.de[e] = c.omp_de[o];
-      O.xp[e] = ToXYZ(O.p[e], n);
-      O.xq[e] = ToXYZ(O.q[e], n);
+      O.xp[e] = PackSiteXYZ(O.p[e], n);
+      O.xq[e] = PackSiteXYZ(O.q[e], n);
       O.ep[e] = occ[O.p[e]];
       O.eq[e] = occ[O.q[e]];
     }
+    if (tid < 64) OmpDrawTests(c, O, r, s_steps - static_cast<uint64_t>(O.pos), maxs, K);
     __syncthreads();
   }
-  auto ramp_T = [&](uint64_t step) {
-    return c.t0[r] + (c.t1[r] - c.t0[r]) * (static_cast<double>(step) / static_cast<double>(maxs));
-  };
   uint64_t it = 0;
   while (it < ntrials) {
     // every thread reads the round state before BuildOmpRound's first lane rewrites it
@@ -1107,7 +1153,7 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
     __syncthreads();
     if (stop) break;
     if (need) {
-      BuildOmpRound(t, c, L, O, r, s_steps, occ, N, n, K);
+      BuildOmpRound(t, c, O, r, s_steps, maxs, occ, N, n, K, ref);
       if (O.error) break;
     }
     const int pos = O.pos;
@@ -1116,10 +1162,8 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
     const uint64_t s0 = s_steps;
     // Metropolis tests of the round's next m events, in parallel
     for (int e = pos + tid; e < pos + m; e += kOmpThreads) {
-      const uint64_t step = s0 + static_cast<uint64_t>(e - pos);
       const double de = O.de[e];
-      bool a = de < 0;
-      if (!a) a = TrialUniform(c, r, step) < exp(-de * (1.0 / kBoltzmann / ramp_T(step)));
+      const bool a = de < 0 || O.uni[e] < exp(-de * O.beta[e]);
       O.acc[e] = a ? 1 : 0;
       const uint64_t ti = trace_base + it + static_cast<uint64_t>(e - pos);
       if (ti < c.trace_cap) {
@@ -1131,48 +1175,65 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
       }
     }
     __syncthreads();
-    if (tid == 0) {  // energies in trial order, with the averaging ring and log records
+    if (tid < 64) {  // energies in trial order, with the averaging ring and log records
+      if constexpr (kLog) {
+        if (tid == 0) {
 #pragma unroll 4
-      for (int e = pos; e < pos + m; ++e) {
-        const uint64_t step = s0 + static_cast<uint64_t>(e - pos);
-        if constexpr (kLog) {
-          if (c.avg_m) {
-            c.ring[static_cast<uint64_t>(r) * c.ring_cap + ring_at] = energy;
-            if (++ring_at == c.ring_cap) ring_at = 0;
-            ++ring_i;
-          }
-          if (clk.Due(step)) {
-            if (log_i < c.log_cap) {
-              CmcLogRecord &rec = c.log[static_cast<uint64_t>(r) * c.log_cap + log_i];
-              rec.steps = step;
-              rec.temperature = ramp_T(step);
-              rec.energy = energy;
-              rec.second = 0.0;
-              rec.abs_energy = abse;
-              rec.count = ring_i;
+          for (int e = pos; e < pos + m; ++e) {
+            const uint64_t step = s0 + static_cast<uint64_t>(e - pos);
+            if (c.avg_m) {
+              c.ring[static_cast<uint64_t>(r) * c.ring_cap + ring_at] = energy;
+              if (++ring_at == c.ring_cap) ring_at = 0;
+              ++ring_i;
             }
-            ++log_i;
+            if (clk.Due(step)) {
+              if (log_i < c.log_cap) {
+                CmcLogRecord &rec = c.log[static_cast<uint64_t>(r) * c.log_cap + log_i];
+                rec.steps = step;
+                rec.temperature =
+                    c.t0[r] + (c.t1[r] - c.t0[r]) * (static_cast<double>(step) / static_cast<double>(maxs));
+                rec.energy = energy;
+                rec.second = 0.0;
+                rec.abs_energy = abse;
+                rec.count = ring_i;
+              }
+              ++log_i;
+            }
+            if (O.acc[e]) {
+              energy += O.de[e];
+              abse += O.de[e];
+              ++acc;
+            }
           }
         }
-        if (O.acc[e]) {
-          energy += O.de[e];
-          abse += O.de[e];
-          ++acc;
+      } else {
+        const bool on = lane >= pos && lane < pos + m && O.acc[lane];
+        const double taken = on ? O.de[lane] : 0.0;
+        acc += __builtin_popcountll(__ballot(on));
+#pragma unroll 16
+        for (int e = 0; e < kOmpMaxK; ++e) {
+          const double de = ReadLane(taken, e);
+          energy += de;
+          abse += de;
         }
       }
-      s_steps = s0 + static_cast<uint64_t>(m);
-      O.pos = pos + m;
+      if (tid == 0) {
+        s_steps = s0 + static_cast<uint64_t>(m);
+        O.pos = pos + m;
+      }
     }
     // the accepted swaps (disjoint sites)
-    for (int e = pos + tid; e < pos + m; e += kOmpThreads) {
-      if (!O.acc[e]) continue;
+    const int e = tid - kOmpThreads / 2;  // off wave 0
+    if (e >= pos && e < pos + m && O.acc[e]) {
+      const uint32_t p = O.p[e], q = O.q[e];
       if (c.atom) {
         const int64_t o = c.off[r];
-        AtomJump(c.atom + o, c.shift + 3 * o, O.p[e], O.q[e], ImageChange(O.xq[e].X - O.xp[e].X, n),
-                 ImageChange(O.xq[e].Y - O.xp[e].Y, n), ImageChange(O.xq[e].Z - O.xp[e].Z, n));
+        const XYZ xp = UnpackSiteXYZ(O.xp[e]), xq = UnpackSiteXYZ(O.xq[e]);
+        AtomJump(c.atom + o, c.shift + 3 * o, p, q, ImageChange(xq.X - xp.X, n),
+                 ImageChange(xq.Y - xp.Y, n), ImageChange(xq.Z - xp.Z, n));
       }
-      occ[O.p[e]] = static_cast<uint8_t>(O.eq[e]);
-      occ[O.q[e]] = static_cast<uint8_t>(O.ep[e]);
+      occ[p] = O.eq[e];
+      occ[q] = O.ep[e];
     }
     it += static_cast<uint64_t>(m);
     __syncthreads();
@@ -1194,6 +1255,33 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
       c.log_n[r] = log_i;
       if (c.avg_m) c.ring_n[r] = ring_i;
     }
+  }
+}
+
+// The most frequent species of each replica (the lowest code of equal ones): the reference of its rounds.
+// Swaps keep the composition, so every launch of a run has the same one.
+__global__ __launch_bounds__(kOmpThreads) void CmcReferenceKernel(CmcDev c, int S, uint8_t *ref) {
+  __shared__ unsigned long long count[kMaxSpecies];
+  const int r = blockIdx.x, tid = threadIdx.x;
+  if (tid < kMaxSpecies) count[tid] = 0;
+  __syncthreads();
+  const int n = c.ncell[r];
+  const uint64_t N = 4ull * n * n * n;
+  const uint8_t *occ = c.occ + c.off[r];
+  for (uint64_t base = 0; base < N; base += kOmpThreads) {
+    const uint64_t i = base + tid;
+    const int v = i < N ? occ[i] : kMaxSpecies;
+    for (int s = 0; s < S; ++s) {
+      const uint64_t m = __ballot(v == s);
+      if ((tid & 63) == 0 && m) atomicAdd(&count[s], static_cast<unsigned long long>(__builtin_popcountll(m)));
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int best = 0;
+    for (int s = 1; s < S; ++s)
+      if (count[s] > count[best]) best = s;
+    ref[r] = static_cast<uint8_t>(best);
   }
 }
 
@@ -1708,6 +1796,12 @@ hipError_t LaunchCmc(const KTables &t, const CmcDev &c, uint64_t trials, uint64_
                : launch(CmcOmpKernel<true, false>, CmcOmpKernel<false, false>, st_omp, kOmpThreads);
   return c.log_every ? launch(CmcKernel<true, true>, CmcKernel<false, true>, st_serial, kCmcThreads)
                      : launch(CmcKernel<true, false>, CmcKernel<false, false>, st_serial, kCmcThreads);
+}
+
+hipError_t LaunchCmcReference(const KTables &t, const CmcDev &c, uint8_t *ref, hipStream_t s) {
+  if (c.R <= 0) return hipSuccess;
+  hipLaunchKernelGGL(CmcReferenceKernel, dim3(c.R), dim3(kOmpThreads), 0, s, c, t.S, ref);
+  return hipGetLastError();
 }
 
 hipError_t LaunchCmcAverage(const CmcDev &c, hipStream_t s) {

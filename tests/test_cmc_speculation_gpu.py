@@ -76,3 +76,38 @@ def test_short_annealing_windows(coeffs, steps, T0):
         assert ga["temperature"][r] == pytest.approx(oa["temperature"], rel=1e-12)
         assert abs(ga["lowest"][r] - oa["lowest"]) <= TOL_E * steps
         assert int(ga["reheats"][r]) == oa["reheats"]
+
+
+@pytest.mark.parametrize("K, lds", [(64, True), (64, False), (3, True)])
+def test_rounds_over_compositions(coeffs, K, lds):
+    """Rounds where the most frequent species is not the first, where nothing is rare (every site of an
+    environment has terms), where pairs are found late, and where the swapped sites are neighbours."""
+    import latticemontecarlo_amd as L
+    import oracle as O
+    path, els = coeffs["e0_4n"]
+    sizes, chunks, seed = [4, 5, 6, 12], [1, 70, 5, 150], 23
+    gp, ge = L.Model(path, els, L.PAIRSITE), L.Model(path, els, L.ENERGY)
+    shares = [(0.25, 0.25, 0.25, 0.25), (0.05, 0.1, 0.8, 0.05), (0.98, 0.0, 0.0, 0.02), (0.1, 0.5, 0.1, 0.3)]
+    codes = [gp.species.index(e) for e in els]
+    rng = np.random.default_rng(3)
+    occs = [rng.choice(codes, 4 * n ** 3, p=w).astype(np.uint8) for n, w in zip(sizes, shares)]
+    total = sum(chunks)
+    drv = L.CanonicalMc(gp, ge, sizes, occs, 2500.0, 700.0, seed, maximum_steps=total)
+    drv.set_lds_occupancy(lds)
+    drv.set_parallel_trials(K)
+    drv.set_trace(total)
+    for k in chunks:
+        drv.run(k)
+    gst, gtr, gocc = drv.state(), drv.trace(), drv.occupancy()
+    gp.check_errors()
+    for r, n in enumerate(sizes):
+        lat = O.Lattice(n)
+        op, oe = O.Model(lat, path, els, O.PAIRSITE), O.Model(lat, path, els, O.ENERGY)
+        c = O.Cmc(op, oe, lat, occs[r], 2500.0, 700.0, seed, replica=r)
+        tr = c.run_omp(total, total, K, trace=True)
+        ran = int(gst["steps"][r])
+        assert ran == c.state()["steps"]
+        assert np.array_equal(gtr["p"][r][:ran], tr["p"][:ran]) and np.array_equal(gtr["q"][r][:ran], tr["q"][:ran])
+        np.testing.assert_allclose(gtr["de"][r][:ran], tr["de"][:ran], rtol=0, atol=TOL_E)
+        assert np.array_equal(gtr["acc"][r][:ran], tr["acc"][:ran])
+        assert np.array_equal(gocc[r], c.occupancy())

@@ -534,6 +534,66 @@ void DownloadAtoms(int32_t R, const int64_t *d_off, const int32_t *d_ncell, cons
 
 }  // namespace
 
+// The arrays that the state calls read lie in one allocation, so that one copy brings them to the host
+// (nine small copies took 110 us, more than 20 steps of 1 024 replicas).
+size_t PlaceState(lmc::KmcDev &d, char *base, size_t R) {
+  auto take = [&](auto *&p, size_t n) {
+    p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base);
+    base += n * sizeof(*p);
+  };
+  char *const first = base;
+  take(d.steps, R);
+  take(d.time, R);
+  take(d.energy, R);
+  take(d.abs_energy, R);
+  take(d.temp, R);
+  take(d.vac, R);
+  take(d.disp, 3 * R);
+  take(d.com, 3 * R);
+  take(d.escaped, R);
+  take(d.error, 1);
+  return static_cast<size_t>(base - first);
+}
+size_t PlaceState(lmc::CmcDev &d, char *base, size_t R) {
+  auto take = [&](auto *&p, size_t n) {
+    p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base);
+    base += n * sizeof(*p);
+  };
+  char *const first = base;
+  take(d.steps, R);
+  take(d.energy, R);
+  take(d.abs_energy, R);
+  take(d.accepted, R);
+  take(d.error, 1);
+  return static_cast<size_t>(base - first);
+}
+// Device copy of host arrays laid out by PlaceState (zeros but for what fill(host) sets), placed in d.
+template <typename Dev, typename Fill>
+char *UploadState(Dev &d, size_t R, Fill fill) {
+  alignas(8) static char probe[8];  // only for the size
+  Dev h;
+  std::vector<uint64_t> host(PlaceState(h, probe, R) / 8 + 1);
+  PlaceState(h, reinterpret_cast<char *>(host.data()), R);
+  fill(h);
+  uint64_t *dev = DevCopy(host);
+  PlaceState(d, reinterpret_cast<char *>(dev), R);
+  return reinterpret_cast<char *>(dev);
+}
+// Host copy of the arrays at `state`, placed in h (which lives as long as the result).
+template <typename Dev>
+std::vector<uint64_t> DownloadState(const char *state, Dev &h, size_t R) {
+  alignas(8) static char probe[8];
+  const size_t bytes = PlaceState(h, probe, R);
+  std::vector<uint64_t> host(bytes / 8 + 1);
+  ToHost(reinterpret_cast<char *>(host.data()), state, bytes);
+  PlaceState(h, reinterpret_cast<char *>(host.data()), R);
+  return host;
+}
+template <typename T>
+void CopyOut(T *dst, const T *src, size_t n) {
+  if (dst) std::copy_n(src, n, dst);
+}
+
 struct lmc_kmc {
   const lmc_model *bm = nullptr;
   lmc::KmcDev d;
@@ -543,6 +603,7 @@ struct lmc_kmc {
   std::vector<uint64_t> start_steps;
   std::vector<char> solute_disp, log_begun, log_fixed, log_skip_first;
   int64_t total_sites = 0;
+  char *state = nullptr;  // the arrays of PlaceState
   int formulation = 0;
   // surrogate evaluation (optional)
   const lmc_surrogate *sur = nullptr;
@@ -563,30 +624,21 @@ struct lmc_kmc {
     if (capture) (void)hipStreamDestroy(capture);
     DevFree(n_sur);
     DevFree(n_fb);
+    DevFree(state);
     DevFree(d.occ);
     DevFree(d.off);
     DevFree(d.ncell);
-    DevFree(d.vac);
-    DevFree(d.steps);
     DevFree(d.max_steps);
     DevFree(d.seed);
     DevFree(d.rid);
-    DevFree(d.time);
-    DevFree(d.energy);
-    DevFree(d.abs_energy);
-    DevFree(d.temp);
     DevFree(d.cv);
     DevFree(d.cs);
     DevFree(d.solute_mass);
     DevFree(d.flags);
     DevFree(d.solvent);
-    DevFree(d.escaped);
     DevFree(d.esc_time);
     DevFree(d.esc_step);
     DevFree(d.esc_site);
-    DevFree(d.disp);
-    DevFree(d.com);
-    DevFree(d.error);
     DevFree(d.prev_j);
     DevFree(d.atom);
     DevFree(d.shift);
@@ -605,6 +657,8 @@ struct lmc_kmc {
 struct lmc_cmc {
   const lmc_model *pm = nullptr;
   lmc::CmcDev d;
+  int64_t total_sites = 0;
+  char *state = nullptr;  // the arrays of PlaceState
   uint64_t trace_pos = 0;
   std::vector<uint64_t> start_steps;         // restart_steps of each replica
   std::vector<char> log_begun, log_skip_first;
@@ -627,19 +681,15 @@ struct lmc_cmc {
     DevFree(d.anneal);
     DevFree(d.atom);
     DevFree(d.shift);
+    DevFree(state);
     DevFree(d.occ);
     DevFree(d.off);
     DevFree(d.ncell);
-    DevFree(d.steps);
     DevFree(d.max_steps);
     DevFree(d.seed);
-    DevFree(d.accepted);
     DevFree(d.rid);
     DevFree(d.t0);
     DevFree(d.t1);
-    DevFree(d.energy);
-    DevFree(d.abs_energy);
-    DevFree(d.error);
     DevFree(d.tr_p);
     DevFree(d.tr_q);
     DevFree(d.tr_de);
@@ -1219,28 +1269,25 @@ int lmc_kmc_create(const lmc_model *barrier, const lmc_model *energy, int32_t R,
     d.occ = DevCopy(std::vector<uint8_t>(occ, occ + b.total));
     d.off = DevCopy(b.off);
     d.ncell = DevCopy(std::vector<int32_t>(ncell, ncell + R));
-    d.vac = DevCopy(vac);
-    d.steps = DevCopy(steps);
+    k->state = UploadState(d, static_cast<size_t>(R), [&](lmc::KmcDev &h) {
+      std::copy(vac.begin(), vac.end(), h.vac);
+      std::copy(steps.begin(), steps.end(), h.steps);
+      std::copy(time.begin(), time.end(), h.time);
+      std::copy(en.begin(), en.end(), h.energy);
+      std::copy(temp.begin(), temp.end(), h.temp);
+    });
     d.max_steps = DevCopy(maxs);
     d.seed = DevCopy(seed);
     d.rid = DevCopy(rid);
-    d.time = DevCopy(time);
-    d.energy = DevCopy(en);
-    d.abs_energy = DevCopy(std::vector<double>(R, 0.0));
-    d.temp = DevCopy(temp);
     d.cv = DevCopy(cv);
     d.cs = DevCopy(cs);
     d.solute_mass = DevCopy(smass);
     d.flags = DevCopy(flags);
     for (int32_t f : flags) d.options |= f;
     d.solvent = DevCopy(solvent);
-    d.escaped = DevCopy(std::vector<int32_t>(R, 0));
     d.esc_time = DevCopy(std::vector<double>(R, 0.0));
     d.esc_step = DevCopy(std::vector<uint64_t>(R, 0));
     d.esc_site = DevCopy(std::vector<int64_t>(R, -1));
-    d.disp = DevCopy(std::vector<int64_t>(3 * R, 0));
-    d.com = DevCopy(std::vector<double>(3 * R, 0.0));
-    d.error = DevCopy(std::vector<int32_t>(1, 0));
     {  // chain steps start with the vacancy's first neighbour in id order as the previous site
       std::vector<int64_t> prev(R);
       for (int r = 0; r < R; ++r) {
@@ -1507,11 +1554,14 @@ int lmc_kmc_run(lmc_kmc *k, uint64_t steps, void *stream) {
   });
 }
 
+static int KmcErrors(int32_t e) {
+  if (e) throw ModelError("Cluster not found in ClusterIndexer or element without barrier parameters");
+  return LMC_OK;
+}
 static int KmcErrors(lmc_kmc *k) {
   int32_t e = 0;
   Check(hipMemcpy(&e, k->d.error, sizeof(e), hipMemcpyDeviceToHost), "hipMemcpy");
-  if (e) throw ModelError("Cluster not found in ClusterIndexer or element without barrier parameters");
-  return LMC_OK;
+  return KmcErrors(e);
 }
 
 int lmc_kmc_state(lmc_kmc *k, uint64_t *steps, double *time, double *energy, double *abs_energy,
@@ -1521,16 +1571,18 @@ int lmc_kmc_state(lmc_kmc *k, uint64_t *steps, double *time, double *energy, dou
     if (!k) throw std::invalid_argument("null driver");
     Check(hipDeviceSynchronize(), "hipDeviceSynchronize");
     const size_t R = static_cast<size_t>(k->d.R);
-    ToHost(steps, k->d.steps, R);
-    ToHost(time, k->d.time, R);
-    ToHost(energy, k->d.energy, R);
-    ToHost(abs_energy, k->d.abs_energy, R);
-    ToHost(temperature, k->d.temp, R);
-    ToHost(vacancy, k->d.vac, R);
-    ToHost(disp, k->d.disp, 3 * R);
-    ToHost(com, k->d.com, 3 * R);
-    ToHost(escaped, k->d.escaped, R);
-    return KmcErrors(k);
+    lmc::KmcDev h;
+    const std::vector<uint64_t> host = DownloadState(k->state, h, R);
+    CopyOut(steps, h.steps, R);
+    CopyOut(time, h.time, R);
+    CopyOut(energy, h.energy, R);
+    CopyOut(abs_energy, h.abs_energy, R);
+    CopyOut(temperature, h.temp, R);
+    CopyOut(vacancy, h.vac, R);
+    CopyOut(disp, h.disp, 3 * R);
+    CopyOut(com, h.com, 3 * R);
+    CopyOut(escaped, h.escaped, R);
+    return KmcErrors(*h.error);
   });
 }
 
@@ -1550,12 +1602,7 @@ int lmc_kmc_occupancy(lmc_kmc *k, uint8_t *occ) {
   return Guard([&] {
     if (!k || !occ) throw std::invalid_argument("null argument");
     Check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-    std::vector<int64_t> off(k->d.R);
-    std::vector<int32_t> nc(k->d.R);
-    ToHost(off.data(), k->d.off, off.size());
-    ToHost(nc.data(), k->d.ncell, nc.size());
-    const int64_t total = off.back() + 4ll * nc.back() * nc.back() * nc.back();
-    ToHost(occ, k->d.occ, static_cast<size_t>(total));
+    ToHost(occ, k->d.occ, static_cast<size_t>(k->total_sites));
     return LMC_OK;
   });
 }
@@ -1763,16 +1810,16 @@ int lmc_cmc_create(const lmc_model *pairsite, const lmc_model *energy, int32_t R
     d.occ = DevCopy(std::vector<uint8_t>(occ, occ + b.total));
     d.off = DevCopy(b.off);
     d.ncell = DevCopy(std::vector<int32_t>(ncell, ncell + R));
-    d.steps = DevCopy(steps);
+    c->total_sites = b.total;
+    c->state = UploadState(d, static_cast<size_t>(R), [&](lmc::CmcDev &h) {
+      std::copy(steps.begin(), steps.end(), h.steps);
+      std::copy(en.begin(), en.end(), h.energy);
+    });
     d.max_steps = DevCopy(maxs);
     d.seed = DevCopy(seed);
-    d.accepted = DevCopy(std::vector<uint64_t>(R, 0));
     d.rid = DevCopy(rid);
     d.t0 = DevCopy(t0);
     d.t1 = DevCopy(t1);
-    d.energy = DevCopy(en);
-    d.abs_energy = DevCopy(std::vector<double>(R, 0.0));
-    d.error = DevCopy(std::vector<int32_t>(1, 0));
     c->start_steps = steps;
     lmc::Upload(*pairsite->m);
     if (energy) {
@@ -2027,13 +2074,13 @@ int lmc_cmc_state(lmc_cmc *c, uint64_t *steps, double *energy, double *abs_energ
     if (!c) throw std::invalid_argument("null driver");
     Check(hipDeviceSynchronize(), "hipDeviceSynchronize");
     const size_t R = static_cast<size_t>(c->d.R);
-    ToHost(steps, c->d.steps, R);
-    ToHost(energy, c->d.energy, R);
-    ToHost(abs_energy, c->d.abs_energy, R);
-    ToHost(accepted, c->d.accepted, R);
-    int32_t e = 0;
-    Check(hipMemcpy(&e, c->d.error, sizeof(e), hipMemcpyDeviceToHost), "hipMemcpy");
-    if (e) throw ModelError("no pair of distinct species found");
+    lmc::CmcDev h;
+    const std::vector<uint64_t> host = DownloadState(c->state, h, R);
+    CopyOut(steps, h.steps, R);
+    CopyOut(energy, h.energy, R);
+    CopyOut(abs_energy, h.abs_energy, R);
+    CopyOut(accepted, h.accepted, R);
+    if (*h.error) throw ModelError("no pair of distinct species found");
     return LMC_OK;
   });
 }
@@ -2042,12 +2089,7 @@ int lmc_cmc_occupancy(lmc_cmc *c, uint8_t *occ) {
   return Guard([&] {
     if (!c || !occ) throw std::invalid_argument("null argument");
     Check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-    std::vector<int64_t> off(c->d.R);
-    std::vector<int32_t> nc(c->d.R);
-    ToHost(off.data(), c->d.off, off.size());
-    ToHost(nc.data(), c->d.ncell, nc.size());
-    const int64_t total = off.back() + 4ll * nc.back() * nc.back() * nc.back();
-    ToHost(occ, c->d.occ, static_cast<size_t>(total));
+    ToHost(occ, c->d.occ, static_cast<size_t>(c->total_sites));
     return LMC_OK;
   });
 }

@@ -232,6 +232,17 @@ __device__ __forceinline__ XYZ UnpackSiteXYZ(uint32_t v) {
   return {X, Y, static_cast<int>(v >> 22) * 2 + ((X + Y) & 1)};
 }
 
+// Site at offset (dx, dy, dz), |d| <= n, of c: SiteAt in 32 bits without compares (24-bit factors).
+__device__ __forceinline__ uint32_t SiteNear(const XYZ &c, uint32_t n, int dx, int dy, int dz) {
+  const uint32_t m = 2 * n;
+  auto wrap = [&](int v) {
+    const uint32_t u = static_cast<uint32_t>(v);
+    return min(min(u, u + m), u - m);
+  };
+  const uint32_t X = wrap(c.X + dx), Y = wrap(c.Y + dy), Z = wrap(c.Z + dz);
+  return __umul24(X, 2 * __umul24(n, n)) + (__umul24(Y, n) + (Z >> 1));
+}
+
 // Metropolis uniform of step `steps`.
 __device__ __forceinline__ double TrialUniform(const CmcDev &c, int r, uint64_t steps) {
   const U4 u = Philox4x32_10(c.seed[r], steps, c.rid[r], 0xFFFFFFFEu);
@@ -517,8 +528,8 @@ __global__ __launch_bounds__(kCmcThreads) void CmcKernel(KTables t, CmcDev c, ui
         };
         const uint32_t p = lane_of(ta), q = lane_of(tb);
         const XYZ xp = UnpackSiteXYZ(lane_of(txa)), xq = UnpackSiteXYZ(lane_of(txb));
-        sp = static_cast<uint32_t>(SiteAt(xp, n, ox, oy, oz));
-        sq = static_cast<uint32_t>(SiteAt(xq, n, ox, oy, oz));
+        sp = SiteNear(xp, n, ox, oy, oz);
+        sq = SiteNear(xq, n, ox, oy, oz);
         const int vp = occ[sp] & ~kMark, vq = occ[sq] & ~kMark;
         // lane 0 is the site itself; codes are validated at creation
         const int ep = __builtin_amdgcn_readlane(vp, 0), eq = __builtin_amdgcn_readlane(vq, 0);
@@ -754,11 +765,12 @@ __global__ __launch_bounds__(kCmcThreads) void CmcKernel(KTables t, CmcDev c, ui
 //   dE     : a wave gathers an environment at a time and notes which sites are not of the replica's
 //            most frequent species; eight threads to an environment add those sites' terms and their
 //            pairs' (see OmpTables);
-//   trials : event lanes test their Metropolis steps in parallel; the accepted swaps are applied while
-//            wave 0 adds the energies in trial order (and takes the log records).
+//   trials : event lanes test their Metropolis steps in parallel, and the accepted swaps are applied; the
+//            energies are added in trial order (and the log records taken) beside the next draw walk.
 // Bound by the latency of these phases. 64 replicas of 30^3 cells, 5 at.% solute, 20 000 trials in
-// rounds of 64: 15.2 -> 7.6 ms (all site clusters of both sites for every event, conflicts by rows and one
-// lane walking the draws and the energies, before); 6^3 cells, 2 000 trials: 12.1 -> 6.9 ms.
+// rounds of 64: 15.5 -> 6.6 ms (all site clusters of both sites for every event, conflicts by rows and one
+// lane walking the draws and the energies, before); 6^3 cells, 2 000 trials: 12.1 -> 6.5 ms. Two attempts
+// to a thread: 0.88 -> 0.72 ms at 1 at.%, 2 000 trials.
 constexpr int kOmpThreads = 1024;
 constexpr int kOmpMaxK = 64;
 constexpr int kOmpPass = kOmpThreads;          // attempts per draw pass
@@ -817,6 +829,10 @@ __device__ void LoadOmpTables(const KTables &t, OmpLds &O, int ref) {
     O.off[tid] = t.site_off[tid];
   }
   if (tid < 125) O.slot_lut[tid] = -1;
+  if (tid < kOmpMaxValid) {
+    O.d.excl[tid] = 0;
+    for (int w = 0; w < kOmpMaxValid / 32; ++w) O.d.conf[tid][w] = 0;
+  }
   for (int i = tid; i < 4 * SS; i += kOmpThreads) {
     const int at = w3 + (i / SS) * SS * S + (i % SS) * S + ref, x = i / S % S;
     T.g[i] = t.w[at] - t.w[w3 + (i / SS) * SS * S + (x * S + ref) * S + ref];
@@ -877,9 +893,12 @@ __device__ __forceinline__ void OmpDrawTests(const CmcDev &c, OmpLds &O, int r, 
   O.beta[e] = 1.0 / kBoltzmann / T;
 }
 
-// The round starting at step s0: pairs, environments, partner slots and dE into O (all threads).
-__device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int r, uint64_t s0, uint64_t maxs,
-                              const uint8_t *occ, uint64_t N, int n, int K, int ref) {
+// The round starting at step s0: pairs, environments, partner slots and dE into O (all threads). Wave 2
+// calls add_sums, the sums of the trials before it, beside the draw walk.
+template <typename Sums>
+__device__ __forceinline__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int r, uint64_t s0, uint64_t maxs,
+                              const uint8_t *occ, uint64_t N, int n, int K, int ref, int &per_thread,
+                              const Sums &add_sums) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   OmpDraw &D = O.d;
   if (tid == 0) {
@@ -889,19 +908,25 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int 
     O.finished = 0;
     O.att0 = 0;
   }
-  if (tid < kOmpMaxValid) {
-    D.excl[tid] = 0;
-    for (int w = 0; w < kOmpMaxValid / 32; ++w) D.conf[tid][w] = 0;
-  }
   __syncthreads();
   bool first = true;
   while (!O.finished) {
-    const U4 u4 = Philox4x32_10(c.seed[r], s0, c.rid[r], 2u * (O.att0 + static_cast<uint32_t>(tid)) + 1u);
-    const uint32_t a = static_cast<uint32_t>(MulHi64(Join64(u4.x, u4.y), N));
-    const uint32_t b = static_cast<uint32_t>(MulHi64(Join64(u4.z, u4.w), N));
-    const bool valid = occ[a] != occ[b];
-    const uint64_t m = __ballot(valid);
-    if (lane == 0) O.wave_valid[wave] = __builtin_popcountll(m);
+    // thread t holds attempts t, or 2 t and 2 t + 1
+    const int per = per_thread;
+    uint32_t a[2], b[2];
+    bool valid[2] = {false, false};
+    uint64_t m[2] = {0, 0};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (k >= per) continue;
+      const U4 u4 = Philox4x32_10(c.seed[r], s0, c.rid[r],
+                                  2u * (O.att0 + static_cast<uint32_t>(per * tid + k)) + 1u);
+      a[k] = static_cast<uint32_t>(MulHi64(Join64(u4.x, u4.y), N));
+      b[k] = static_cast<uint32_t>(MulHi64(Join64(u4.z, u4.w), N));
+      valid[k] = occ[a[k]] != occ[b[k]];
+      m[k] = __ballot(valid[k]);
+    }
+    if (lane == 0) O.wave_valid[wave] = __builtin_popcountll(m[0]) + __builtin_popcountll(m[1]);
     __syncthreads();
     // valid attempts of the waves before this one, and in all (a running sum over each row of 16 lanes)
     int run = O.wave_valid[lane & 15];
@@ -910,27 +935,32 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int 
     run += __builtin_amdgcn_update_dpp(0, run, 0x114, 0xF, 0xF, true);
     run += __builtin_amdgcn_update_dpp(0, run, 0x118, 0xF, 0xF, true);
     const int total = __builtin_amdgcn_readlane(run, 15);
-    const int u = (wave ? __builtin_amdgcn_readlane(run, wave - 1) : 0) +
-                  __builtin_popcountll(m & ((1ull << lane) - 1));
+    const uint64_t lower = (1ull << lane) - 1;
+    int u = (wave ? __builtin_amdgcn_readlane(run, wave - 1) : 0) + __builtin_popcountll(m[0] & lower) +
+            __builtin_popcountll(m[1] & lower);
     const int len0 = O.len, nch0 = O.nch;
     const int cap = K - len0 + kOmpSpare;  // at most kOmpMaxValid
     const int nv = total < cap ? total : cap;
-    if (valid && u < nv) {
-      D.va[u] = a;
-      D.vb[u] = b;
-      D.xa[u] = PackSiteXYZ(a, n);
-      D.xb[u] = PackSiteXYZ(b, n);
-      D.vidx[u] = tid;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (valid[k] && u < nv) {
+        D.va[u] = a[k];
+        D.vb[u] = b[k];
+        D.xa[u] = PackSiteXYZ(a[k], n);
+        D.xb[u] = PackSiteXYZ(b[k], n);
+        D.vidx[u] = per * tid + k;
+      }
+      u += valid[k] ? 1 : 0;
     }
     __syncthreads();
     if (nv > 0) {
-      const float per = 1.0f / static_cast<float>(nv);
+      const float inv = 1.0f / static_cast<float>(nv);
       auto meet = [&](const XYZ &s, int v) {
         return Near(s, UnpackSiteXYZ(D.xa[v]), n) || Near(s, UnpackSiteXYZ(D.xb[v]), n);
       };
       // every pair of attempts once: (v, v + d mod nv) for d up to half way round
       for (int i = tid; i < nv * (nv / 2); i += kOmpThreads) {
-        const int d = static_cast<int>((i + 0.5f) * per), v = i - d * nv;  // i < 2^13: exact
+        const int d = static_cast<int>((i + 0.5f) * inv), v = i - d * nv;  // i < 2^13: exact
         const int w = v + d + 1 >= nv ? v + d + 1 - nv : v + d + 1;
         if (meet(UnpackSiteXYZ(D.xa[v]), w) || meet(UnpackSiteXYZ(D.xb[v]), w)) {
           const int lo = min(v, w);
@@ -938,7 +968,7 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int 
         }
       }
       for (int i = tid; i < nv * nch0; i += kOmpThreads) {  // against the events of earlier passes
-        const int j = static_cast<int>((i + 0.5f) * per), v = i - j * nv;  // i < 2^14: exact
+        const int j = static_cast<int>((i + 0.5f) * inv), v = i - j * nv;  // i < 2^14: exact
         if (meet(UnpackSiteXYZ(O.ch[j]), v)) D.excl[v] = 1;
       }
     }
@@ -1000,7 +1030,8 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int 
         O.len = len;
         O.nch = 2 * len;
         // the next pass starts after the last attempt looked at
-        O.att0 += total > cap ? static_cast<uint32_t>(D.vidx[nv - 1] + 1) : static_cast<uint32_t>(kOmpPass);
+        O.att0 += total > cap ? static_cast<uint32_t>(D.vidx[nv - 1] + 1)
+                                : static_cast<uint32_t>(kOmpPass * per);
         if (!fin && O.att0 >= kMaxPairAttempts) {
           O.error = 1;
           fin = true;
@@ -1013,9 +1044,17 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int 
       }
     } else if (wave == 1 && first) {
       OmpDrawTests(c, O, r, s0, maxs, K);
+    } else if (wave == 2 && first) {
+      add_sums();
     }
     first = false;
     __syncthreads();
+    // too few valid attempts in a round's first pass: two to a thread from the next pass on, until one to a
+    // thread would do (in a small box it is the conflicts that cost passes, and more attempts would not help)
+    if (len0 == 0) {
+      const bool few = total < per * (K + 8);
+      per_thread = few && (per == 2 || !O.finished) ? 2 : 1;
+    }
   }
   const int len = O.len;
   {  // environments, a wave each
@@ -1025,7 +1064,7 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int 
 #pragma unroll 4
     for (int e2 = wave; e2 < 2 * len; e2 += kOmpThreads / 64) {
       const XYZ x = UnpackSiteXYZ(e2 & 1 ? O.xq[e2 >> 1] : O.xp[e2 >> 1]);
-      const int v = in ? occ[SiteAt(x, n, ox, oy, oz)] : ref;
+      const int v = in ? occ[SiteNear(x, n, ox, oy, oz)] : ref;
       const int code = v < t.S ? v : 0;  // codes are validated at creation
       const uint64_t m = __ballot(lane > 0 && code != ref && in);
       if (in) O.env[e2][lane] = static_cast<uint8_t>(code);
@@ -1060,10 +1099,24 @@ __device__ void BuildOmpRound(const KTables &t, const CmcDev &c, OmpLds &O, int 
           const double *h = T.g + (T.label[a][skip] - 1) * SS + ca;
           v -= h[en * S] - h[eo * S];
         }
-        for (uint64_t j = other & T.with[a] & ((~0ull << a) << 1); j; j &= j - 1) {
-          const int b = __builtin_ctzll(j);
-          const double *f2 = T.f + S + 3 * SS + (T.label[a][b] - 1) * SS * S + ca * S + env[b];
-          v += f2[en * SS] - f2[eo * SS];
+        const double *f2 = T.f + S + 3 * SS + ca * S;
+        for (uint64_t j = other & T.with[a] & ((~0ull << a) << 1); j;) {  // four pairs' loads side by side
+          int at[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int b = j ? __builtin_ctzll(j) : a;
+            const int l = T.label[a][b], e = env[b];
+            at[k] = j ? (l - 1) * SS * S + e : ref;  // past the last pair: a term of the reference, zero
+            j &= j - 1;
+          }
+          double w[4][2];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            w[k][0] = f2[at[k] + en * SS];
+            w[k][1] = f2[at[k] + eo * SS];
+          }
+#pragma unroll
+          for (int k = 0; k < 4; ++k) v += w[k][0] - w[k][1];
         }
       }
     }
@@ -1107,7 +1160,8 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
   uint64_t acc = 0, log_i = 0, ring_i = 0, ring_at = 0;
   double energy = 0, abse = 0;
   LogClock clk;
-  if (tid < 64) {  // wave 0 keeps the sums (the records: its first lane)
+  const bool sums = (tid >> 6) == 2;  // the wave that keeps the sums (the records: its first lane)
+  if (sums) {
     acc = c.accepted[r];
     energy = c.energy[r];
     abse = c.abs_energy[r];
@@ -1117,9 +1171,11 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
     O.len = c.omp_len[r];
     O.pos = c.omp_pos[r];
     O.error = 0;
+  }
+  if (sums && lane == 0) {
     if constexpr (kLog) {
       clk.L = c.log_every;
-      clk.Reset(s_steps);
+      clk.Reset(c.steps[r]);
       log_i = c.log_n[r];
       c.log_lo[r] = log_i;
       if (c.avg_m) {
@@ -1145,7 +1201,56 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
     if (tid < 64) OmpDrawTests(c, O, r, s_steps - static_cast<uint64_t>(O.pos), maxs, K);
     __syncthreads();
   }
+  // Energies of the trials sum_pos .. sum_pos + sum_m - 1 of the round, tried from step sum_step on, in
+  // trial order, with the averaging ring and log records (the wave of the sums).
+  int sum_pos = 0, sum_m = 0;
+  uint64_t sum_step = 0;
+  auto add_sums = [&] {
+    if constexpr (kLog) {
+      if (lane == 0) {
+#pragma unroll 4
+        for (int e = sum_pos; e < sum_pos + sum_m; ++e) {
+          const uint64_t step = sum_step + static_cast<uint64_t>(e - sum_pos);
+          if (c.avg_m) {
+            c.ring[static_cast<uint64_t>(r) * c.ring_cap + ring_at] = energy;
+            if (++ring_at == c.ring_cap) ring_at = 0;
+            ++ring_i;
+          }
+          if (clk.Due(step)) {
+            if (log_i < c.log_cap) {
+              CmcLogRecord &rec = c.log[static_cast<uint64_t>(r) * c.log_cap + log_i];
+              rec.steps = step;
+              rec.temperature =
+                  c.t0[r] + (c.t1[r] - c.t0[r]) * (static_cast<double>(step) / static_cast<double>(maxs));
+              rec.energy = energy;
+              rec.second = 0.0;
+              rec.abs_energy = abse;
+              rec.count = ring_i;
+            }
+            ++log_i;
+          }
+          if (O.acc[e]) {
+            energy += O.de[e];
+            abse += O.de[e];
+            ++acc;
+          }
+        }
+      }
+    } else {
+      const bool on = lane >= sum_pos && lane < sum_pos + sum_m && O.acc[lane];
+      const double taken = on ? O.de[lane] : 0.0;
+      acc += __builtin_popcountll(__ballot(on));
+#pragma unroll 16
+      for (int e = 0; e < kOmpMaxK; ++e) {
+        const double de = ReadLane(taken, e);
+        energy += de;
+        abse += de;
+      }
+    }
+    sum_m = 0;
+  };
   uint64_t it = 0;
+  int per_thread = 1;
   while (it < ntrials) {
     // every thread reads the round state before BuildOmpRound's first lane rewrites it
     const bool need = O.pos == O.len;
@@ -1153,7 +1258,7 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
     __syncthreads();
     if (stop) break;
     if (need) {
-      BuildOmpRound(t, c, O, r, s_steps, maxs, occ, N, n, K, ref);
+      BuildOmpRound(t, c, O, r, s_steps, maxs, occ, N, n, K, ref, per_thread, add_sums);
       if (O.error) break;
     }
     const int pos = O.pos;
@@ -1175,52 +1280,12 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
       }
     }
     __syncthreads();
-    if (tid < 64) {  // energies in trial order, with the averaging ring and log records
-      if constexpr (kLog) {
-        if (tid == 0) {
-#pragma unroll 4
-          for (int e = pos; e < pos + m; ++e) {
-            const uint64_t step = s0 + static_cast<uint64_t>(e - pos);
-            if (c.avg_m) {
-              c.ring[static_cast<uint64_t>(r) * c.ring_cap + ring_at] = energy;
-              if (++ring_at == c.ring_cap) ring_at = 0;
-              ++ring_i;
-            }
-            if (clk.Due(step)) {
-              if (log_i < c.log_cap) {
-                CmcLogRecord &rec = c.log[static_cast<uint64_t>(r) * c.log_cap + log_i];
-                rec.steps = step;
-                rec.temperature =
-                    c.t0[r] + (c.t1[r] - c.t0[r]) * (static_cast<double>(step) / static_cast<double>(maxs));
-                rec.energy = energy;
-                rec.second = 0.0;
-                rec.abs_energy = abse;
-                rec.count = ring_i;
-              }
-              ++log_i;
-            }
-            if (O.acc[e]) {
-              energy += O.de[e];
-              abse += O.de[e];
-              ++acc;
-            }
-          }
-        }
-      } else {
-        const bool on = lane >= pos && lane < pos + m && O.acc[lane];
-        const double taken = on ? O.de[lane] : 0.0;
-        acc += __builtin_popcountll(__ballot(on));
-#pragma unroll 16
-        for (int e = 0; e < kOmpMaxK; ++e) {
-          const double de = ReadLane(taken, e);
-          energy += de;
-          abse += de;
-        }
-      }
-      if (tid == 0) {
-        s_steps = s0 + static_cast<uint64_t>(m);
-        O.pos = pos + m;
-      }
+    sum_pos = pos;
+    sum_m = m;
+    sum_step = s0;
+    if (tid == 0) {
+      s_steps = s0 + static_cast<uint64_t>(m);
+      O.pos = pos + m;
     }
     // the accepted swaps (disjoint sites)
     const int e = tid - kOmpThreads / 2;  // off wave 0
@@ -1243,14 +1308,17 @@ __global__ __launch_bounds__(kOmpThreads) void CmcOmpKernel(KTables t, CmcDev c,
     uint32_t *dst = reinterpret_cast<uint32_t *>(c.occ + c.off[r]);
     for (uint64_t i = tid; i < N / 4; i += kOmpThreads) dst[i] = occ_words[i];
   }
+  if (sums) add_sums();
   if (tid == 0) {
     if (O.error) atomicOr(c.error, 2);
     c.steps[r] = s_steps;
+    c.omp_len[r] = O.len;
+    c.omp_pos[r] = O.pos;
+  }
+  if (sums && lane == 0) {
     c.accepted[r] = acc;
     c.energy[r] = energy;
     c.abs_energy[r] = abse;
-    c.omp_len[r] = O.len;
-    c.omp_pos[r] = O.pos;
     if constexpr (kLog) {
       c.log_n[r] = log_i;
       if (c.avg_m) c.ring_n[r] = ring_i;

@@ -308,8 +308,19 @@ __global__ void MlpReduceAdamKernel(MlpMut w, const float *grad_part, int nparts
   const int m = idx / P, p = idx - m * P;
   float v = w.master[idx];
   if (grad_part) {
+    // sixteen loads in flight, added in tile order (each waited for alone: 17 us for 64 tiles)
     float g = 0.f;
-    for (int b = 0; b < nparts; ++b) g += grad_part[(static_cast<size_t>(b) * M + m) * P + p];
+    const float *part = grad_part + idx;
+    const size_t tile = static_cast<size_t>(M) * P;
+    int b = 0;
+    for (; b + 16 <= nparts; b += 16, part += 16 * tile) {
+      float v16[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v16[i] = part[i * tile];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) g += v16[i];
+    }
+    for (; b < nparts; ++b, part += tile) g += *part;
     if (grad_out) grad_out[idx] = g;
     if (update) {
       const float m1 = beta1 * w.adam_m[idx] + (1.f - beta1) * g;

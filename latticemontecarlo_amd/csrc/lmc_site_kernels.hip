@@ -21,6 +21,7 @@ struct SiteLds {
   uint8_t env[2][48];           // environments of the swap's sites
   int slot[2];                  // partner slots (q around p, p around q)
   double part[kThreads / 64];   // per-wave partial sums
+  double term[kThreads];        // a swap's terms by cluster
 };
 
 __device__ void LoadSiteTables(const KTables &t, SiteLds &L) {
@@ -110,11 +111,18 @@ __device__ void GatherPair(SiteLds &L, const uint8_t *occ, int n, int64_t p, int
 // dE of swapping species ep at p and eq at q, from the environments of GatherPair. Far pairs:
 // dE(p) + dE(q) on the unswapped config (...WithoutCoupling :136-146). Near pairs: clusters
 // containing both keep their multiset and are skipped (...WithCoupling :96-134). All threads
-// call; the result is valid in thread 0.
+// call; the result is valid in thread 0. Added in the serial trials' order (a lane's clusters lane,
+// lane + 64, ..., then the wave sum): the two give the same bits.
 __device__ double SwapDe(const KTables &t, SiteLds &L, int ep, int eq) {
-  const double v =
-      SitePartial(t, L, 0, ep, eq, L.slot[0]) + SitePartial(t, L, 1, eq, ep, L.slot[1]);
-  return BlockSum(L, v);
+  static_assert(kThreads >= kMaxSiteClusters, "one cluster per thread");
+  L.term[threadIdx.x] = SitePartial(t, L, 0, ep, eq, L.slot[0]) + SitePartial(t, L, 1, eq, ep, L.slot[1]);
+  __syncthreads();
+  double v = 0.0;
+  if (threadIdx.x < 64) {
+    for (int i = threadIdx.x; i < kThreads; i += 64) v += L.term[i];
+    v = WaveSum(v);
+  }
+  return v;
 }
 
 __global__ __launch_bounds__(kThreads) void SwapDeKernel(KTables t, const uint8_t *occ,

@@ -36,8 +36,8 @@ ALGO_BYTES_NOTE = ("137 B per replica-step = 135 distinct occupancy bytes read +
                    "are closed forms, so the 4 B neighbour index per site of a table-driven design "
                    "(677 B per step) is not read. The kernel's working set is cache/LDS resident "
                    "(traffic is measured HBM bytes per launch), so HBM is not its bound: the step is "
-                   "VALU/LDS-issue and latency bound (issue)")
-FORMS = ["dense", "solvent-baseline", "dense-wide"]  # kernel shapes of the autotuner
+                   "bound by the latency of its own chain of instructions (issue)")
+FORMS = ["one-wave", "one-wave (form 1)", "team"]  # kernel shapes of the autotuner
 METRIC = "KMC steps/s over all replicas, surrogate vs plain GPU at \u22645 meV barrier MAE"
 HBM_PEAK_GBS = 8000.0
 
@@ -867,8 +867,8 @@ def main():
     drv = L.KineticMcFirst(bm, em, [n] * R, occs, temps, seed=args.seed, maximum_steps=10 ** 12)
     stream = torch.cuda.current_stream()
     tune = drv.autotune(steps=300)
-    log(f"autotune: dense {tune['ms_dense']:.4f} ms, solvent baseline {tune['ms_solvent']:.4f} ms, "
-        f"dense wide {tune['ms_wide']:.4f} ms per KMC step of the batch -> "
+    log(f"autotune: form 0 {tune['ms_dense']:.4f} ms, form 1 {tune['ms_solvent']:.4f} ms, "
+        f"form 2 (team) {tune['ms_wide']:.4f} ms per KMC step of the batch -> "
         f"{FORMS[tune['formulation']]}")
     t0 = time.time()
     for c, k in launch_plan(args.warmup, args.chunk) if args.warmup > 0 else []:

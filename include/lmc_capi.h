@@ -213,8 +213,8 @@ int lmc_total_energy(const lmc_model *m, const uint8_t *d_occ, const int64_t *d_
 /* No counterpart in the reference. For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): lmc_total_energy
  * with the same kernels and results, its cluster-count scratch a fixed per-device array of
- * 2^19 counts (4 MiB, held until the process ends) instead of a hipMalloc'd buffer. It allocates
- * nothing, does not synchronise, and rejects with LMC_ERR_ARG
+ * 2^19 counts (8 MiB with those of clusters without an ECI, held until the process ends) instead of
+ * a hipMalloc'd buffer. It allocates nothing, does not synchronise, and rejects with LMC_ERR_ARG
  * - n_replicas * n_eci above 2^19 (n_eci = 95 for Al/Mg/Zn: at most 5518 replicas; 167 for
  *   Al/Cu/Mg/Zn: 3139), and
  * - a model whose tables are not yet on the current device (any other compute entry point with

@@ -304,7 +304,8 @@ const KTables &Upload(Model &m) {
   for (auto *v : {&e1, &e2, &e3})
     for (auto &x : *v)
       if (x < 0) x = 0;  // invalid keys only occur with two vacancies in one cluster
-  if (state.size() > kMaxStateClusters || mmm.size() > kMaxOrbitClusters ||
+  if (state.size() != kMaxStateClusters) throw std::logic_error("state list of another length");
+  if (mmm.size() > kMaxOrbitClusters ||
       site_cl.size() > kMaxSiteClusters || m.w.size() > kMaxW)
     throw std::invalid_argument("tables exceed the kernel's LDS capacity (too many species)");
 
@@ -343,6 +344,13 @@ const KTables &Upload(Model &m) {
   std::vector<uint32_t> site3;
   for (const auto &s : pg.site3) site3.insert(site3.end(), s.begin(), s.end());
   b.Add(site_of, &k.site_of);
+  std::vector<int32_t> env_pk(2 * 12 * 64, 0);
+  for (int d = 0; d < 12; ++d)
+    for (int s = 0; s < kEnvSlots; ++s) {
+      if (pg.site_of[d][s] < kPairSites) env_pk[64 * d + s] = site_pk[pg.site_of[d][s]];  // the vacancy's own: 0
+      env_pk[64 * (12 + d) + s] = PackOff(pg.back[d][s]);
+    }
+  b.Add(env_pk, &k.env_pk);
   b.Add(site3, &k.site3);
   b.Add(pt.cls, &k.cls);
   b.Add(pt.clsb, &k.clsb);

@@ -128,6 +128,13 @@ __device__ __forceinline__ double ReadLane(double v, int lane) {
                           __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
+// v of the other lane of each pair (DPP quad_perm 1, 0, 3, 2).
+__device__ __forceinline__ double PairLane(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0xB1, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
 // Sum over the 64 lanes of a full wave, returned to every lane: shifted adds within each row of
 // 16 leave the row sum in its last lane; the four row sums are then added in order.
 __device__ __forceinline__ double WaveSum(double v) {

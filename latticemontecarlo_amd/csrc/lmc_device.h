@@ -15,7 +15,7 @@ namespace lmc {
 //   orbit    : s0[0:8] | s1[8:16] | feature base[16:28] | kind[28:30]
 //   mm2      : the forward orbit entries, then the backward ones (slots mirrored)
 //   site     : label[0:3] | other1[4:10] | other2[10:16]
-constexpr int kMaxStateClusters = 512;
+constexpr int kMaxStateClusters = 504;  // the state list of every model: 452 clusters, padded
 constexpr int kMaxOrbitClusters = 768;
 // Cluster lists are padded to multiples of this (4 entries per lane of an event's 21 lanes).
 constexpr int kClusterPad = 84;
@@ -62,6 +62,7 @@ struct KTables {
   int kind, S, ne, x_code, F1, F2, nw;
   int nwd, wrow;
   uint32_t rank_lut;        // species code -> element rank, 4 bits per code (vacancy: 0)
+  const int32_t *env_pk;    // [2][12][64] offsets of the slots of an event and of its reverse, packed as site_pk
 };
 
 struct DeviceTables {

@@ -34,11 +34,12 @@ namespace {
 
 constexpr int kEvalWaves = 8;  // waves of an evaluation workgroup
 constexpr int kTeam = 4;       // waves of a replica in the team shape
+constexpr int kChainTeam = kTeam + 1;  // of a team that makes chain steps, with the one that keeps the energies
 
 // Dynamic LDS of a workgroup (byte offsets): value tables, replicas' and waves' working sets.
 struct KmcLayout {
   PairLayout tab;
-  int team, wave, extra, bytes;
+  int team, wave, extra, wd, bytes;  // wd: the state clusters' weights (teams)
 };
 
 __device__ __forceinline__ int WaveIndex() {
@@ -180,10 +181,10 @@ __device__ __forceinline__ Jump TakeJump(const EventTargets &e, int mig, double 
 
 // The first half of a step's end, before the next gather: what depends on the state before the jump
 // (escape record, log, atoms; kFull), then the occupancy (kStore) and the vacancy's new position. Every
-// lane holds Q; lane 0 keeps the records.
+// lane holds Q; lane 0 keeps the records. energies: the log's too.
 template <bool kFull, bool kStore = true>
 __device__ __forceinline__ void ApplyJump(const KTables &t, const KmcDev &k, ReplicaLds &Q, uint8_t *occ,
-                                          int r, const Jump &j, bool escaped) {
+                                          int r, const Jump &j, bool escaped, bool energies = true) {
   if constexpr (kFull) {
     const bool writer = kStore && LaneId() == 0;
     if (escaped) {
@@ -196,7 +197,7 @@ __device__ __forceinline__ void ApplyJump(const KTables &t, const KmcDev &k, Rep
       Q.steps = Q.max_steps + 1;
     }
     if (writer && k.log_every && LogDue(Q.steps, k.log_every))
-      LogStep(k, Q, r, static_cast<int64_t>(j.site), j.ea, j.de);
+      LogStep(k, Q, r, static_cast<int64_t>(j.site), j.ea, j.de, energies);
     if (writer && k.atom) {  // the vacancy at Q.vac is the lhs of the reference's jump pair
       const int64_t o = k.off[r];
       const int h = Q.m2 >> 1;
@@ -217,17 +218,17 @@ __device__ __forceinline__ void ApplyJump(const KTables &t, const KmcDev &k, Rep
 }
 
 // The second half, under the next gather's loads: clock, energies, trace, displacements
-// (KineticMcAbstract.cpp:147-181).
+// (KineticMcAbstract.cpp:147-181). energies: the trace's too.
 template <bool kFull>
 __device__ __forceinline__ void FinishStep(const KmcDev &k, ReplicaLds &Q, int r, uint64_t trace_index,
-                                           const Jump &j, double dt, XYZ &moved) {
+                                           const Jump &j, double dt, XYZ &moved, bool energies = true) {
   const XYZ &d = j.move;
   if constexpr (kFull) {
     if (trace_index < k.trace_cap && LaneId() == 0) {
       const uint64_t o = static_cast<uint64_t>(r) * k.trace_cap + trace_index;
       k.tr_sel[o] = static_cast<int64_t>(j.site);
       k.tr_ea[o] = j.ea;
-      k.tr_de[o] = j.de;
+      if (energies) k.tr_de[o] = j.de;
       k.tr_time[o] = Q.time + dt;
     }
     if ((Q.flags & 4) && j.mig != Q.solvent) {  // solute COM (KineticMcAbstract.cpp:163-177)
@@ -264,12 +265,122 @@ __device__ __forceinline__ int SelectEvent(double cum, double goal) {
 struct TeamExchange {
   double part[kTeam][16][3];
   int info[16];
-  int K;
+  int K;  // listed sites + 1 (0: the replica or the launch has ended) | choice of the step before << 8, and
+          // at the end whether that step escaped << 12
+  OrderedLds ordered;
+  int32_t off[12][64];  // slots' offsets by direction (EnergyKeeper)
 };
+
+// The energies of a team's replica (OrderedDe), kept by one wave beside the leading wave's work, two steps
+// late, so that nothing waits for them: the species of a step's slots are loaded one step later, when
+// its choice is known, and summed another step later. In between the leading wave may have stored the
+// next jump: of the slots that are read, that changes the target only, whose species the jump names.
+// It takes 0.04 us of a step's 1.74 us (64 replicas, E0; the step without it and with one code for all
+// waves: 1.82 us), and with chain steps, in a wave of its own, 0.1 us of 8.5. Batches with more replicas
+// than CUs have no wave to spare and add the quadratic form's changes.
+template <bool kFull>
+struct EnergyKeeper {
+  ReplicaLds Q;
+  LaneSites ls;
+  const uint8_t *occ;
+  const int32_t *off;  // offsets of the event's slots by direction
+  int n, r;
+  double sign;         // chain steps add the reverse event's change, negated
+  uint64_t log_n, trace_base;
+  XYZ c;               // the vacancy before the step to come
+  uint32_t site;       // the step loaded: site and species of its slot `lane`, migrating species
+  int code, mig;
+  __device__ __forceinline__ void Start(const KTables &t, const KmcDev &k, int replica, int wv, const int32_t *slots,
+                                        double way, uint64_t base) {
+    r = replica;
+    n = k.ncell[r];
+    ls = LoadSites(t, wv);
+    occ = k.occ + k.off[r];
+    off = slots;
+    sign = way;
+    trace_base = base;
+    LoadReplica(k, r, n, Q);
+    log_n = kFull && k.log_every ? k.log_n[r] : 0;
+    c = VacancyXYZ(Q);
+    site = 0;
+    code = mig = 0;
+  }
+  // The choice of step `it` of the launch (direction | migrating species << 8), whose jump is stored; the
+  // next one is not before the barrier that follows. last: no step follows; escaped: in the last.
+  __device__ __forceinline__ void Take(const KTables &t, const KmcDev &k, OrderedLds &D, const char *wd, int it,
+                                       int choice, bool last, bool escaped) {
+    const XYZ to = WrapAdd(c, PackedXYZ(ReadLaneInt(ls.pk[0], choice & 255)), Q.m2);
+    const uint32_t new_site = SiteId<uint32_t>(WrapSite(c, n, off[64 * (choice & 255) + LaneId()]), n);
+    const int new_code = occ[new_site];
+    const uint32_t target = SiteId<uint32_t>(
+        {static_cast<uint32_t>(to.X), static_cast<uint32_t>(to.Y), static_cast<uint32_t>(to.Z)}, n);
+    code = site == target ? choice >> 8 : code;
+    int i = it - 1;  // the last step is summed at once
+#pragma nounroll
+    do {
+      if (i >= 0) {
+        const double de = sign * OrderedDe(t, D, code, wd, mig);
+        if constexpr (kFull) {
+          const uint64_t steps = i == it && escaped ? Q.max_steps + 1 : Q.steps + i;
+          if (k.log_every && LogDue(steps, k.log_every)) {
+            if (log_n < k.log_cap && LaneId() == 0)
+              LogEnergy(k.log[static_cast<uint64_t>(r) * k.log_cap + log_n], Q.energy, de);
+            ++log_n;
+          }
+          if (trace_base + i < k.trace_cap && LaneId() == 0)
+            k.tr_de[static_cast<uint64_t>(r) * k.trace_cap + (trace_base + i)] = de;
+        }
+        Q.energy += de;
+        Q.abse += de;
+      }
+      code = new_code;
+      mig = choice >> 8;
+      ++i;
+    } while (last && i <= it);
+    c = to;
+    site = new_site;
+    asm volatile("" : "+v"(code));  // loaded before the barrier that follows
+  }
+};
+
+// A helper wave of a team: its share of the sums of every step, from barrier to barrier; it ends when the
+// leading wave announces no further step (X.K). The last helper also keeps the energies, after a step's
+// second barrier, while the leading wave finishes the step.
+template <bool kQ, bool kFull>
+__device__ __forceinline__ void HelpTeam(const KTables &t, const PairShared<kQ> &G, const PairTab &T,
+                                         const TeamLds &S, WaveLds &W, TeamExchange &X, const char *wd,
+                                         const KmcDev &k, int r, int wv, uint64_t trace_base) {
+  const int lane = LaneId();
+  const bool keeps = wv == kTeam - 1;
+  EnergyKeeper<kFull> keeper;
+  keeper.Start(t, k, r, wv, X.off[0], 1.0, trace_base);
+  int before = 0;  // X.info of the step before
+  for (int it = 0;; ++it) {
+    __syncthreads();
+    const int word = __builtin_amdgcn_readfirstlane(X.K), K = (word & 255) - 1;
+    const int info = X.info[lane & 15];
+    if (K >= 0) {
+      const PairSums s =
+          PairTerms<kQ, kTeam>(G, T, S, W, keeper.ls, K, MakeRow<kQ>(t, T, info & 255, info >> 8), wv);
+      if (lane < 16) {
+        double *p = X.part[wv][lane];
+        p[0] = s.de;
+        p[1] = s.la;
+        if (kQ) p[2] = s.lb;
+      }
+      __syncthreads();
+    }
+    if (keeps && it > 0)
+      keeper.Take(t, k, X.ordered, wd, it - 1, ReadLaneInt(before, (word >> 8) & 15), K < 0, word >> 12);
+    before = info;
+    if (K < 0) break;
+  }
+  if (keeps && lane == 0) StoreEnergy(k, r, keeper.Q);
+}
 
 // Persistent KMC. kWaves 1: `group` replicas per workgroup, one wave each; the waves never meet after
 // the table copy. kWaves kTeam: one replica per workgroup, a leading wave makes the step and three
-// helpers share its sums, with two barriers per step.
+// helpers share its sums, with two barriers per step (HelpTeam).
 // kFull: options, schedule, trace, log and atoms are compiled in.
 template <bool kQ, bool kTab, int kWaves, bool kFull>
 __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) void KmcKernel(
@@ -277,16 +388,26 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) voi
   __shared__ PairShared<kQ> G;
   extern __shared__ __align__(16) char dyn[];
   const int lane = LaneId(), wave = WaveIndex();
-  const int first = blockIdx.x * group, mine = kWaves == 1 ? wave : 0, wv = kWaves == 1 ? 0 : wave;
+  const int first = blockIdx.x * group, mine = kWaves == 1 ? wave : 0;
   const PairTab T =
       LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, k.solvent[first], threadIdx.x, blockDim.x);
   TeamExchange &X = *reinterpret_cast<TeamExchange *>(dyn + lay.extra);
+  if (kWaves > 1) {
+    CopyTable(dyn + lay.wd, t.wd, 8 * t.nwd, threadIdx.x, blockDim.x);
+    CopyTable(reinterpret_cast<char *>(X.off), t.env_pk, sizeof(X.off), threadIdx.x, blockDim.x);
+  }
   __syncthreads();
   const int r = first + mine;
   if (mine >= group || r >= k.R) return;
   TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[mine];
   WaveLds &W = reinterpret_cast<WaveLds *>(dyn + lay.wave)[wave];
-  const LaneSites ls = LoadSites(t, wv);
+  if constexpr (kWaves > 1) {
+    if (wave != 0) {
+      HelpTeam<kQ, kFull>(t, G, T, S, W, X, dyn + lay.wd, k, r, wave, trace_base);
+      return;
+    }
+  }
+  const LaneSites ls = LoadSites(t, 0);
   const ExpConst E = MakeExpConst();
   uint8_t *occ = k.occ + k.off[r];
   const int n = k.ncell[r];
@@ -297,53 +418,37 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) voi
   StepClock clock{1.0, 0.0};
   Around<uint32_t> a;
   double u2 = 0.0, log_u1 = 0.0;
-  int dir = 0;
+  int dir = 0, sel = 0;
   bool error = false;
-  if (wv == 0 && !Q.done) {
+  if (!Q.done) {
     GatherAround(ls, occ, n, VacancyXYZ(Q), a);
     dir = EventDirection(G, VacancyXYZ(Q), n);
     DrawStep(draws, Q, u2, log_u1);
   }
   for (int it = 0; it < nsteps; ++it) {
-    if (wv == 0 && Q.done && kWaves == 1) break;
-    EventConst ec;
-    EventRow row;
-    EventTargets to;
-    bool bad = false;
-    int K = -1;  // team: the replica has ended
-    if (wv == 0 && !Q.done) {
-      if (kFull) UpdateTemperature(k, Q, clock);
-      bad = CheckCodes(t, a, dir, k.error);
-      const int M = Bpermute(dir, a.code[0]);
-      to = MakeTargets(ls, a, dir);
-      row = MakeRow<kQ>(t, T, dir, M);
-      ec = LoadConst(t, G, M);
-      K = ListSites<kQ>(t, G, T, S, ls, a);
-    }
+    if (Q.done) break;
+    if (kFull) UpdateTemperature(k, Q, clock);
+    const bool bad = CheckCodes(t, a, dir, k.error);
+    const int M = Bpermute(dir, a.code[0]);
+    const EventTargets to = MakeTargets(ls, a, dir);
+    const EventRow row = MakeRow<kQ>(t, T, dir, M);
+    const EventConst ec = LoadConst(t, G, M);
+    const int K = ListSites<kQ>(t, G, T, S, ls, a);
     PairSums s;
     if constexpr (kWaves == 1) {
       s = PairTerms<kQ, 1>(G, T, S, W, ls, K, row, 0);
     } else {
-      if (wv == 0) {
-        if (lane < 16) X.info[lane] = row.dir | (row.M << 8);
-        if (lane == 0) X.K = K;
-      }
+      if (lane < 16) X.info[lane] = row.dir | (row.M << 8);
+      if (lane == 0) X.K = (K + 1) | (sel << 8);
       __syncthreads();
-      K = __builtin_amdgcn_readfirstlane(X.K);
-      if (K < 0) break;  // uniform over the workgroup
-      if (wv != 0) {
-        const int i = X.info[lane & 15];
-        row = MakeRow<kQ>(t, T, i & 255, i >> 8);
-      }
-      s = PairTerms<kQ, kWaves>(G, T, S, W, ls, K, row, wv);
+      s = PairTerms<kQ, kWaves>(G, T, S, W, ls, K, row, 0);
       if (lane < 16) {
-        double *p = X.part[wv][lane];
+        double *p = X.part[0][lane];
         p[0] = s.de;
         p[1] = s.la;
         if (kQ) p[2] = s.lb;
       }
       __syncthreads();
-      if (wv != 0) continue;
       const double *p = X.part[0][lane & 15];
       s = {p[0], p[1], kQ ? p[2] : 0.0};
 #pragma unroll
@@ -357,20 +462,23 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) voi
     error = error || EventError(e);
     const double cum = RowScan((lane & 15) < 12 ? Exp(E, -e.ea * Q.beta) : 0.0);
     const double total = ReadLane(cum, 11);
-    const int sel = SelectEvent(cum, u2 * total);
+    sel = SelectEvent(cum, u2 * total);
     const Jump j = TakeJump(to, row.M, kFull ? ReadLane(e.ea, sel) : 0.0, ReadLane(e.de, sel), sel);
-    ApplyJump<kFull>(t, k, Q, occ, r, j, kFull && Escaped(Q, a.code[0]));
+    ApplyJump<kFull>(t, k, Q, occ, r, j, kFull && Escaped(Q, a.code[0]), kWaves == 1);
     WaveFence();
     GatherAround(ls, occ, n, VacancyXYZ(Q), a);
     dir = EventDirection(G, VacancyXYZ(Q), n);
     double dt = -log_u1 / (total * kPrefactor);
     if (kFull && (Q.flags & 1)) dt *= clock.corr;
-    FinishStep<kFull>(k, Q, r, trace_base + it, j, dt, moved);
+    FinishStep<kFull>(k, Q, r, trace_base + it, j, dt, moved, kWaves == 1);
     DrawStep(draws, Q, u2, log_u1);
   }
-  if (wv != 0) return;
+  if constexpr (kWaves > 1) {  // no further step
+    if (lane == 0) X.K = (sel << 8) | (kFull ? Q.esc << 12 : 0);
+    __syncthreads();
+  }
   if (__ballot(error) && lane == 0) atomicOr(k.error, 1);
-  if (lane == 0) StoreReplica<kFull>(k, r, Q, moved);
+  if (lane == 0) StoreReplica<kFull>(k, r, Q, moved, kWaves == 1);
 }
 
 // Persistent second-order (chain) KMC, KineticMcChainOmpi (KineticMcChainOmpi.cpp:56-151). Each step
@@ -379,9 +487,16 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) voi
 // reverse of i -> k, and forms the second-order probabilities and the time with lane r on neighbour
 // r (id order). kWaves 1: one wave makes all passes of a replica. kWaves kTeam: four waves hold the
 // replica's state and make every fourth pass; one barrier per step exchanges their results, wave 0
-// writes.
+// writes. A fifth wave, where the launch has one, keeps the energies.
+struct ChainExchange {
+  double res[2][12][3];  // as res below
+  int choice[2];         // by step parity: direction | migrating species << 8
+  int end[2];            // by step parity: 1, no such step; 3, and the step before it escaped
+  OrderedLds ordered;
+  int32_t off[12][64];
+};
 template <bool kQ, bool kTab, int kWaves, bool kFull>
-__global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) void KmcChainKernel(
+__global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kChainTeam) LMC_WAVES(1, 2) void KmcChainKernel(
     KTables t, KmcLayout lay, KmcDev k, int group, int nsteps, uint64_t trace_base) {
   __shared__ PairShared<kQ> G;
   extern __shared__ __align__(16) char dyn[];
@@ -389,10 +504,30 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) voi
   const int first = blockIdx.x * group;
   const PairTab T =
       LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, k.solvent[first], threadIdx.x, blockDim.x);
+  ChainExchange &X = *reinterpret_cast<ChainExchange *>(dyn + lay.extra);
+  const bool kept = kWaves > 1 && blockDim.x > 64 * kWaves;  // the energies, by the wave past the last
+  if (kept) {
+    CopyTable(dyn + lay.wd, t.wd, 8 * t.nwd, threadIdx.x, blockDim.x);
+    CopyTable(reinterpret_cast<char *>(X.off), t.env_pk + 12 * 64, sizeof(X.off), threadIdx.x, blockDim.x);
+    if (threadIdx.x < 2) X.end[threadIdx.x] = 0;
+  }
   __syncthreads();
   const int r = kWaves == 1 ? first + wave : first;
   if (kWaves == 1 && (wave >= group || r >= k.R)) return;
   const int wv = kWaves == 1 ? 0 : wave;
+  if (kWaves > 1 && wv == kWaves) {
+    EnergyKeeper<kFull> keeper;
+    keeper.Start(t, k, r, 0, X.off[0], -1.0, trace_base);
+    for (int it = 0;; ++it) {
+      __syncthreads();
+      const int end = __builtin_amdgcn_readfirstlane(X.end[it & 1]);
+      if (it > 0) keeper.Take(t, k, X.ordered, dyn + lay.wd, it - 1,
+                              __builtin_amdgcn_readfirstlane(X.choice[(it - 1) & 1]), end != 0, end == 3);
+      if (end) break;
+    }
+    if (lane == 0) StoreEnergy(k, r, keeper.Q);
+    return;
+  }
   TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[wave];
   WaveLds &W = reinterpret_cast<WaveLds *>(dyn + lay.wave)[wave];
   // results of the passes, [step parity][neighbour rank][total rate, Ea, dE]
@@ -409,7 +544,8 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) voi
   StepDraws draws{0.0, 0.0, 0, false};
   XYZ moved{0, 0, 0};  // displacement of this launch
   StepClock clock{1.0, 0.0};
-  for (int it = 0; it < nsteps; ++it) {
+  int it = 0;
+  for (; it < nsteps; ++it) {
     if (Q.done) break;
     if (kFull) UpdateTemperature(k, Q, clock);
     const XYZ c = VacancyXYZ(Q);
@@ -475,27 +611,32 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) voi
     const int sel = SelectEvent(cum, u2);
     const Jump j = TakeJump(MakeTargets(ls, a, dir), Bpermute(dir, a.code[0]), ReadLane(barrier, sel),
                             ReadLane(de, sel), sel);
+    if (kept && wv == 0) X.choice[it & 1] = ReadLaneInt(dir, sel) | (j.mig << 8);
     prev = static_cast<uint32_t>(Q.vac);
     prev_mig = j.mig;
     const bool escaped = kFull && Escaped(Q, a.code[0]);
-    if (wv == 0) ApplyJump<kFull>(t, k, Q, occ, r, j, escaped);
+    if (wv == 0) ApplyJump<kFull>(t, k, Q, occ, r, j, escaped, !kept);
     else ApplyJump<kFull, false>(t, k, Q, occ, r, j, escaped);
     WaveFence();
     if (kFull && (Q.flags & 1)) dt *= clock.corr;
-    if (wv == 0) FinishStep<kFull>(k, Q, r, trace_base + it, j, dt, moved);
+    if (wv == 0) FinishStep<kFull>(k, Q, r, trace_base + it, j, dt, moved, !kept);
     else FinishStep<kFull>(k, Q, r, ~0ull, j, dt, moved);
+  }
+  if (kept) {
+    if (wv == 0) X.end[it & 1] = Q.esc ? 3 : 1;
+    __syncthreads();
   }
   if (wv != 0) return;
   if (__ballot(error) && lane == 0) atomicOr(k.error, 1);
   if (lane == 0) {
-    StoreReplica<kFull>(k, r, Q, moved);
+    StoreReplica<kFull>(k, r, Q, moved, !kept);
     k.prev_j[r] = static_cast<int64_t>(prev);
   }
 }
 
 // Dynamic LDS plan for workgroups of `teams` replicas and `waves` waves: the value tables go to LDS
 // when per_cu workgroups then still fit a CU.
-KmcLayout PlanLds(const KTables &t, int teams, int waves, size_t extra, int per_cu) {
+KmcLayout PlanLds(const KTables &t, int teams, int waves, size_t extra, int per_cu, bool ordered = false) {
   const DeviceLimits &dl = CurrentDeviceLimits();
   const bool quartic = t.kind == kQuartic;
   const size_t fixed = quartic ? sizeof(PairShared<true>) : sizeof(PairShared<false>);
@@ -509,6 +650,7 @@ KmcLayout PlanLds(const KTables &t, int teams, int waves, size_t extra, int per_
   add(lay.team, teams * sizeof(TeamLds));
   add(lay.wave, waves * sizeof(WaveLds));
   add(lay.extra, extra);
+  if (ordered) add(lay.wd, 8 * static_cast<size_t>(t.nwd));
   const size_t row = 8 * static_cast<size_t>(t.ne);
   const size_t tabs = row * (t.de_row + t.la_row + (quartic ? t.lb_row : 0)) + 48;
   if (fixed + at + tabs <= share) {
@@ -571,9 +713,12 @@ KmcPlan PlanKmc(const KTables &t, int32_t R, int form) {
   p.group = p.team ? 1 : std::min(8, std::max(1, (R + cus - 1) / cus));
   p.blocks = (R + p.group - 1) / p.group;
   const int waves = std::max(kTeam, p.group);
-  p.threads = 64 * waves;
-  const size_t extra = p.chain ? waves * 72 * sizeof(double) : p.team ? sizeof(TeamExchange) : 0;
-  p.lay = PlanLds(t, p.chain ? waves : p.group, waves, extra, p.blocks > cus ? 2 : 1);
+  // chain teams: the wave that keeps the energies only where one team has the CU; two teams of five waves
+  // would not fit beside each other (400 replicas: 332 us for 30 steps, 452 with it)
+  p.threads = 64 * (p.chain && p.team && R <= cus ? kChainTeam : waves);
+  const size_t extra = p.team ? (p.chain ? sizeof(ChainExchange) : sizeof(TeamExchange))
+                              : p.chain ? waves * 72 * sizeof(double) : 0;
+  p.lay = PlanLds(t, p.chain ? waves : p.group, waves, extra, p.blocks > cus ? 2 : 1, p.team);
   return p;
 }
 

@@ -592,6 +592,53 @@ __device__ __forceinline__ PairSums PairTerms(const PairShared<kQ> &G, const Pai
   return s;
 }
 
+// The energy change of one event, added cluster by cluster in the order of the state list: 84 running
+// sums (of entries c, c + 84, ...), the four that are 21 apart added two and two, then the 21 results
+// one after another. A trajectory whose changes cancel (a vacancy among solvent atoms, or back at its
+// start) has nothing but the rounding of these sums in its energy, so that a small batch's energies keep
+// this order; the quadratic form, which decides the rates, adds in another one. One wave: lanes 2 i and
+// 2 i + 1 hold the four running sums i, i + 21, i + 42 and i + 63.
+constexpr int kOrderedRounds = kMaxStateClusters / kClusterPad;
+struct OrderedLds {  // element ranks of the event's slots, as the entries of t.state index them
+  uint16_t rn8[64];  // rank * 8 * ne
+  uint8_t r8[64];    // rank * 8
+};
+// The event whose slot s = lane holds species `code`; M: migrating species; w: the rows of t.wd.
+__device__ __forceinline__ double OrderedDe(const KTables &t, OrderedLds &D, int code, const char *w, int M) {
+  const int lane = LaneId(), half = lane < 42 ? lane : 41;  // lanes past the last sum repeat it
+  const uint32_t *list = t.state + (half >> 1) + 42 * (half & 1);
+  uint32_t entry[2][kOrderedRounds];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int b = 0; b < kOrderedRounds; ++b) entry[j][b] = list[21 * j + kClusterPad * b];
+  const uint32_t rank = lane < kEnvSlots ? (t.rank_lut >> (4 * code)) & 15u : 0u;
+  D.r8[lane] = static_cast<uint8_t>(rank << 3);
+  D.rn8[lane] = static_cast<uint16_t>(__umul24(rank, 8 * t.ne));
+  WaveFence();
+  const char *row = w + __umul24((t.rank_lut >> (4 * M)) & 15u, 8 * t.wrow);
+  uint32_t at[2][kOrderedRounds];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int b = 0; b < kOrderedRounds; ++b) {
+      const uint32_t e = entry[j][b];
+      at[j][b] = D.r8[e & 255u] + D.rn8[(e >> 9) & 127u] + (e >> 16);
+    }
+  double v[2] = {0.0, 0.0};
+#pragma unroll
+  for (int b = 0; b < kOrderedRounds; ++b)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) v[j] += *reinterpret_cast<const double *>(row + at[j][b]);
+  double four = v[0] + v[1];
+  four += PairLane(four);
+  double sum = 0.0;
+#pragma unroll
+  for (int i = 0; i < 21; ++i) sum += ReadLane(four, 2 * i);
+  WaveFence();
+  return sum;
+}
+
 // exp to within one unit in the last place: x = k ln 2 + r by Cody and Waite's two-part reduction, the
 // Taylor series to r^13 (truncation below 2^-57 at |r| = ln 2 / 2) in even and odd halves, then the
 // scaling by 2^k, which takes care of overflow and gradual underflow. NaN stays NaN. The

@@ -43,6 +43,11 @@ PairGeometry BuildPairGeometry() {
         }
     }
   }
+  for (int d = 0; d < 12; ++d)  // the direction back is 11 - d
+    for (int s = 0; s < kEnvSlots; ++s) {
+      const I3 &o = jt.off[dir[11 - d]][s];
+      g.back[d][s] = I3{g.site[d].x + o.x, g.site[d].y + o.y, g.site[d].z + o.z};
+    }
   for (int d = 0; d < 12; ++d)
     for (int s = 0; s < kEnvSlots; ++s)
       g.site3[s][d / 3] |= static_cast<uint32_t>(g.site_of[d][s]) << (8 * (d % 3));

@@ -31,6 +31,8 @@ struct PairGeometry {
                                       // other sites within three shells, the rest
   std::array<std::array<uint8_t, kPairSiteRow>, 12> slot{};   // [direction][site]
   std::array<std::array<uint8_t, kEnvSlots>, 12> site_of{};   // [direction][slot]; vacancy: kPairSites
+  // offsets from the vacancy of the slots of the reverse event, from the neighbour in a direction back
+  std::array<std::array<I3, kEnvSlots>, 12> back{};
   // sites of a slot for the directions 3 g .. 3 g + 2, a byte each: [slot][g]
   std::array<std::array<uint32_t, 4>, kEnvSlots> site3{};
   // directions by ascending neighbour id for a vacancy inside the box (0), at coordinate 0 (1) or at

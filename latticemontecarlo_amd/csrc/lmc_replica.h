@@ -52,9 +52,16 @@ __device__ bool LogDue(uint64_t steps, uint64_t log_every) {
   return steps % every == 0;
 }
 
-// The kmc_log.txt record of the step about to jump the vacancy to `jump` (one lane).
+// The energies of a log record: before the step's jump, and the jump's change.
+__device__ __forceinline__ void LogEnergy(KmcLogRecord &L, double energy, double de) {
+  L.energy = energy;
+  L.de = de;
+}
+
+// The kmc_log.txt record of the step about to jump the vacancy to `jump` (one lane); energies: with its
+// energies.
 __device__ void LogStep(const KmcDev &k, const ReplicaLds &Q, int r, int64_t jump, double ea,
-                        double de) {
+                        double de, bool energies = true) {
   const uint64_t i = k.log_n[r];
   k.log_n[r] = i + 1;  // counts past the capacity too, so the host can report the loss
   if (i >= k.log_cap) return;
@@ -62,9 +69,8 @@ __device__ void LogStep(const KmcDev &k, const ReplicaLds &Q, int r, int64_t jum
   L.steps = Q.steps;
   L.time = Q.time;
   L.temperature = Q.T;
-  L.energy = Q.energy;
   L.ea = ea;
-  L.de = de;
+  if (energies) LogEnergy(L, Q.energy, de);
   const int64_t o = k.off[r];
   const int32_t *sv = nullptr;
   L.atom = -1;
@@ -109,13 +115,17 @@ __device__ void LoadReplica(const KmcDev &k, int r, int n, ReplicaLds &Q) {
 }
 
 // Replica r's state back to HBM (one thread); `moved`: its displacement in this launch. Without
-// kFull the temperature, the escape flag and the solute displacement have not changed.
-template <bool kFull>
-__device__ void StoreReplica(const KmcDev &k, int r, const ReplicaLds &Q, const XYZ &moved) {
-  k.steps[r] = Q.steps;
-  k.time[r] = Q.time;
+// kFull the temperature, the escape flag and the solute displacement have not changed. energies:
+// with its energies.
+__device__ __forceinline__ void StoreEnergy(const KmcDev &k, int r, const ReplicaLds &Q) {
   k.energy[r] = Q.energy;
   k.abs_energy[r] = Q.abse;
+}
+template <bool kFull>
+__device__ void StoreReplica(const KmcDev &k, int r, const ReplicaLds &Q, const XYZ &moved, bool energies = true) {
+  k.steps[r] = Q.steps;
+  k.time[r] = Q.time;
+  if (energies) StoreEnergy(k, r, Q);
   k.vac[r] = Q.vac;
   k.disp[3 * r] += moved.X;
   k.disp[3 * r + 1] += moved.Y;

@@ -390,8 +390,13 @@ __device__ void ExactDe(const KTables &t, const JumpLds &L, const Tabs &T, SurLd
   if ((lt & 63) == 0) S.dsum[g][lt >> 6] = v;
 }
 
+// The waves per SIMD that the registers are planned for (two are resident) are stated: the compiler
+// otherwise takes them from the static LDS alone, and 6 KB less of it per replica made it plan for more
+// and spill 100 registers instead of 63 (C = 3, 1 024 replicas: 40.2 us per KMC step, 33.8 stated; the
+// evaluation kernel at C = 2: 31.5 and 30.5 us). Limits of 2, 3 and 4 at C = 2: 30.8, 31.5 and 30.5 us,
+// and 30.1, 28.9 and 28.3 us per KMC step.
 template <int C, int G, int kSub, bool kKmc, bool kBL>
-__global__ __launch_bounds__(G * kSub) void SurrogateKernel(KTables t, DynLayout lay, KmcDev k,
+__global__ __launch_bounds__(G * kSub) __attribute__((amdgpu_waves_per_eu(2, 4))) void SurrogateKernel(KTables t, DynLayout lay, KmcDev k,
                                                              SurDev sd, uint64_t nsteps,
                                                              uint64_t trace_base, SurOut out) {
   constexpr int kBlock = Shape<G, kSub>::kBlock, Kp = MlpDims<C>::Kp;

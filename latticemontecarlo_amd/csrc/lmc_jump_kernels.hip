@@ -63,7 +63,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) LMC_WAVES(1, 2) void EvalJumpsKern
   __syncthreads();
   TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[wave];
   WaveLds &W = reinterpret_cast<WaveLds *>(dyn + lay.wave)[wave];
-  const LaneSites ls = LoadSites(t, 0);
+  const LaneSites ls = LoadSites<!kScan>(t, 0);
   const ExpConst E = MakeExpConst();
   for (int64_t r = static_cast<int64_t>(blockIdx.x) * kEvalWaves + wave; r < R;
        r += static_cast<int64_t>(gridDim.x) * kEvalWaves) {
@@ -98,8 +98,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) LMC_WAVES(1, 2) void EvalJumpsKern
       WaveFence();
 #pragma unroll
       for (int u = 0; u < 3; ++u)
-        if (lane + 64 * u < kPairSites) S.code[lane + 64 * u] = static_cast<uint16_t>(a.code[u]);
-      if (lane == 0) S.code[kPairSites] = static_cast<uint16_t>(t.x_code);
+        if (lane + 64 * u <= kPairSites) S.code[lane + 64 * u] = static_cast<uint16_t>(a.code[u]);
       WaveFence();
       for (int q = 0; q < 12; ++q) {
         const int d = ReadLaneInt(dir, q);

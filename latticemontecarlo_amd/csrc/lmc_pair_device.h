@@ -159,8 +159,9 @@ __device__ __forceinline__ PairTab LoadPairTables(const KTables &t, PairShared<k
   return T;
 }
 
-// The lane's sites (lane, lane + 64, lane + 128; lanes past the last site repeat site 0) and the
-// pair of list entries it tests first, read once per launch.
+// The lane's sites (lane, lane + 64, lane + 128; lanes past the last site repeat site 0, or with kOwn have
+// the vacancy's own, whose species is then checked too) and the pair of list entries it tests first,
+// read once per launch.
 struct LaneSites {
   int32_t pk[3];
   uint32_t word[3];  // site | |offset|^2 << 24
@@ -172,12 +173,14 @@ __device__ __forceinline__ void PairOf(int p, int &i, int &j) {
   i = static_cast<int>((__builtin_amdgcn_sqrtf(8.0f * p + 1.5f) + 1.0f) * 0.5f);
   j = p - ((i * (i - 1)) >> 1);
 }
+template <bool kOwn = false>
 __device__ __forceinline__ LaneSites LoadSites(const KTables &t, int wv) {
   LaneSites s;
   const int lane = LaneId();
 #pragma unroll
   for (int u = 0; u < 3; ++u) {
-    s.pk[u] = t.site_pk[lane + 64 * u < kPairSites ? lane + 64 * u : 0];
+    const bool in = lane + 64 * u < kPairSites;
+    s.pk[u] = kOwn && !in ? 0 : t.site_pk[in ? lane + 64 * u : 0];
     const uint32_t r2 = static_cast<uint32_t>(__builtin_amdgcn_sdot4(s.pk[u], s.pk[u], 0, false));
     s.word[u] = static_cast<uint32_t>(lane + 64 * u) | (r2 << 24);
   }

@@ -37,7 +37,7 @@ ALGO_BYTES_NOTE = ("137 B per replica-step = 135 distinct occupancy bytes read +
                    "(677 B per step) is not read. The kernel's working set is cache/LDS resident "
                    "(traffic is measured HBM bytes per launch), so HBM is not its bound: the step is "
                    "bound by the latency of its own chain of instructions (issue)")
-FORMS = ["one-wave", "one-wave (form 1)", "team"]  # kernel shapes of the autotuner
+FORMS = ["by batch size", "one-wave", "team"]  # formulations
 METRIC = "KMC steps/s over all replicas, surrogate vs plain GPU at \u22645 meV barrier MAE"
 HBM_PEAK_GBS = 8000.0
 

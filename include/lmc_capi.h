@@ -68,9 +68,7 @@ void lmc_model_free(lmc_model *m);
 int32_t lmc_model_num_species(const lmc_model *m);
 /* Species code of an element string, -1 if not in the model. */
 int32_t lmc_model_species_code(const lmc_model *m, const char *element);
-/* Default formulation of new KMC drivers: 0 (default) or 1. Both evaluate a jump from all-solvent
- * sums and the exact one- and two-site changes at the sites that hold another species; the stateless
- * calls always do. */
+/* Formulation of new KMC drivers: 0 (default) or 1, see lmc_kmc_set_formulation. */
 int lmc_model_set_formulation(lmc_model *m, int32_t formulation);
 /* Element string of a species code (NULL if out of range); valid while m lives. */
 const char *lmc_model_species_name(const lmc_model *m, int32_t code);
@@ -273,20 +271,20 @@ void lmc_kmc_free(lmc_kmc *k);
 int lmc_kmc_set_schedule(lmc_kmc *k, int32_t n_points, const double *time, const double *temp);
 /* Per-replica trace of the next `capacity` steps (selected neighbour, Ea, dE, time). 0 = off. */
 int lmc_kmc_set_trace(lmc_kmc *k, uint64_t capacity);
-/* Kernel of this driver: 0 and 1 one wave per replica, or four when every replica has a CU of its
- * own; 2 always four waves per replica. These are first-order steps, differ in FP64 summation order
- * only, and have no reference counterpart. 3: second-order residence-time steps, replacing
+/* Kernel of this driver: 1 one wave per replica; 2 four waves per replica; 0 (default) four when
+ * every replica has a CU of its own, else one. These are first-order steps, differ in FP64 summation
+ * order only, and have no reference counterpart. 3: second-order residence-time steps, replacing
  * KineticMcChainOmpi (lmc/mc/include/KineticMcChainOmpi.h, KineticMcChainOmpi.cpp:56-151):
  * the 12 x 12 jumps out of the vacancy's first neighbours after each virtual jump, the
  * second-order probabilities and the deterministic time t_2; the previous site starts as the
  * vacancy's first neighbour in id order (KineticMcAbstract.cpp:252). Takes no surrogate. */
 int lmc_kmc_set_formulation(lmc_kmc *k, int32_t formulation);
-/* Autotuner (no reference counterpart): runs `steps` KMC steps with each kernel shape on a
- * scratch copy of the batch state (HIP events), keeps the fastest and leaves the replicas
- * untouched. ms_per_step[3]: per-step times of formulations 0, 1, 2 (NaN when not tried: the
- * wide shape is tried only when every replica has a CU of its own). */
+/* Autotuner (no reference counterpart): runs `steps` KMC steps with one wave and with four waves per
+ * replica on a scratch copy of the batch state (HIP events, after a few steps that are not timed), keeps
+ * the faster formulation, 1 or 2, and leaves the replicas untouched. ms_per_step[3]: per-step times of
+ * formulations 0 (the time of the shape it stands for), 1, 2; NaN for chain steps. */
 int lmc_kmc_autotune_shapes(lmc_kmc *k, int32_t steps, int32_t *chosen, double *ms_per_step);
-/* lmc_kmc_autotune_shapes reporting formulations 0 and 1 only. */
+/* lmc_kmc_autotune_shapes reporting formulations 0 and 1 only (the arguments' names are historical). */
 int lmc_kmc_autotune(lmc_kmc *k, int32_t steps, int32_t *chosen, double *ms_dense,
                      double *ms_solvent);
 /* Advance every replica by `steps` steps (fewer if it reaches maximum_steps or escapes).

@@ -359,9 +359,9 @@ class KineticMcFirst:
         check(lib().lmc_kmc_set_formulation(self.h, formulation))
 
     def autotune(self, steps=200):
-        """Times each kernel shape for `steps` steps on a scratch copy and keeps the fastest:
-        formulations 0, 1 and 2 (2, four waves per replica, tried only with at most one replica per
-        CU); ms_* per batch step (NaN when not tried)."""
+        """Times one and four waves per replica for `steps` steps each on a scratch copy and keeps the
+        faster formulation, 1 or 2. Times per batch step: ms_solvent with one wave, ms_wide with four,
+        ms_dense with the shape that formulation 0 takes for this batch (the keys' names are historical)."""
         ch, ms = C.c_int32(), (C.c_double * 3)()
         check(lib().lmc_kmc_autotune_shapes(self.h, steps, C.byref(ch), ms))
         return dict(formulation=ch.value, ms_dense=ms[0], ms_solvent=ms[1], ms_wide=ms[2])

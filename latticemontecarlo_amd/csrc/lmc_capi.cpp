@@ -1326,14 +1326,6 @@ int lmc_kmc_set_formulation(lmc_kmc *k, int32_t formulation) {
   return LMC_OK;
 }
 
-static int DeviceCUs() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
-  return cus;
-}
-
 int lmc_kmc_autotune(lmc_kmc *k, int32_t steps, int32_t *chosen, double *ms_dense,
                      double *ms_solvent) {
   double ms[3];
@@ -1372,14 +1364,13 @@ int lmc_kmc_autotune_shapes(lmc_kmc *k, int32_t steps, int32_t *chosen, double *
     };
     hipEvent_t e0 = nullptr, e1 = nullptr;
     float ms[3] = {0, 0, 0};
-    // the wide shape only when every replica has a CU of its own
-    const int cus = DeviceCUs();
-    const int forms = (cus > 0 && k->d.R <= cus) ? 3 : 2;
+    // not timed: the first launch of a kernel, which loads its code (2.5 ms)
+    const uint64_t warm = std::min<uint64_t>(static_cast<uint64_t>(steps), 8);
     try {
       Check(hipDeviceSynchronize(), "hipDeviceSynchronize");
       Check(hipEventCreate(&e0), "hipEventCreate");
       Check(hipEventCreate(&e1), "hipEventCreate");
-      for (int f = 0; f < forms; ++f) {
+      for (int f = 1; f < 3; ++f) {
         for (void *p : owned) (void)hipFree(p);
         owned.clear();
         clone(s.occ, k->d.occ, static_cast<size_t>(k->total_sites));
@@ -1408,6 +1399,7 @@ int lmc_kmc_autotune_shapes(lmc_kmc *k, int32_t steps, int32_t *chosen, double *
           clone(s.atom, k->d.atom, static_cast<size_t>(k->total_sites));
           clone(s.shift, k->d.shift, 3 * static_cast<size_t>(k->total_sites));
         }
+        Check(lmc::LaunchKmc(t, s, warm, 0, nullptr, f), "autotune KMC launch");
         Check(hipEventRecord(e0, nullptr), "hipEventRecord");
         Check(lmc::LaunchKmc(t, s, static_cast<uint64_t>(steps), 0, nullptr, f),
               "autotune KMC launch");
@@ -1419,7 +1411,7 @@ int lmc_kmc_autotune_shapes(lmc_kmc *k, int32_t steps, int32_t *chosen, double *
         ToHost(a.data(), s.steps, R);
         ToHost(b.data(), k->d.steps, R);
         uint64_t ran = static_cast<uint64_t>(steps);
-        for (size_t r = 0; r < R; ++r) ran = std::min<uint64_t>(ran, a[r] - b[r]);
+        for (size_t r = 0; r < R; ++r) ran = std::min<uint64_t>(ran, a[r] - b[r] - std::min<uint64_t>(a[r] - b[r], warm));
         if (ran == 0) throw std::runtime_error("autotune: a timing run advanced no step");
         ms[f] /= static_cast<float>(ran);
       }
@@ -1432,14 +1424,11 @@ int lmc_kmc_autotune_shapes(lmc_kmc *k, int32_t steps, int32_t *chosen, double *
     for (void *p : owned) (void)hipFree(p);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    int best = 0;
-    for (int f = 1; f < forms; ++f)
-      if (ms[f] < ms[best]) best = f;
-    k->formulation = best;
+    k->formulation = ms[2] < ms[1] ? 2 : 1;
+    ms[0] = ms[lmc::KmcTeam(k->d.R, 0) ? 2 : 1];
     if (chosen) *chosen = k->formulation;
     if (ms_per_step)
-      for (int f = 0; f < 3; ++f)
-        ms_per_step[f] = f < forms ? ms[f] : std::numeric_limits<double>::quiet_NaN();
+      for (int f = 0; f < 3; ++f) ms_per_step[f] = ms[f];
     return LMC_OK;
   });
 }

@@ -199,10 +199,12 @@ hipError_t LaunchEvalJumps(const KTables &t, const uint8_t *occ, const int64_t *
 hipError_t LaunchVacancyScan(const KTables &t, const uint8_t *occ, int32_t n, int64_t sub_site,
                              int sub_code, const int64_t *sites, int32_t K, int64_t *nb,
                              double *ea, double *de, int32_t *err, hipStream_t s);
-// form: 0 or 1 one wave per replica, 2 wide shape (four waves per replica), 3 second-order chain
-// steps (KineticMcChainOmpi).
+// form: 0 the shape that suits the batch's size, 1 one wave per replica, 2 four waves per replica, 3
+// second-order chain steps (KineticMcChainOmpi).
 hipError_t LaunchKmc(const KTables &t, const KmcDev &k, uint64_t steps, uint64_t trace_base,
                      hipStream_t s, int form);
+// Whether a batch of R replicas is stepped by four waves per replica.
+bool KmcTeam(int32_t R, int form);
 // Everything LaunchKmc sets up outside the stream (LDS plan, kernel attributes), so that its
 // launches can then be captured in a graph.
 hipError_t PrepareKmc(const KTables &t, int32_t R, int form);

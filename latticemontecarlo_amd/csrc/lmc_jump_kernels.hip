@@ -696,8 +696,8 @@ hipError_t LaunchEval(const KTables &t, const uint8_t *occ, const int64_t *off, 
   });
 }
 
-// How a KMC batch is laid over the chip. form: 0, 1 one wave per replica; 2 a team of four waves per
-// replica; 3 chain steps.
+// How a KMC batch is laid over the chip. form: 0 by the batch's size, 1 one wave per replica, 2 a team of
+// four waves per replica, 3 chain steps (by the batch's size).
 struct KmcPlan {
   KmcLayout lay;
   int group, blocks, threads;
@@ -707,7 +707,7 @@ KmcPlan PlanKmc(const KTables &t, int32_t R, int form) {
   const int cus = CurrentDeviceLimits().cus;
   KmcPlan p;
   p.chain = form == 3;
-  p.team = form == 2 || R <= cus || (p.chain && R <= 2 * cus);
+  p.team = KmcTeam(R, form);
   // one-wave replicas: as many per workgroup as it takes to give every CU one workgroup, up to eight
   p.group = p.team ? 1 : std::min(8, std::max(1, (R + cus - 1) / cus));
   p.blocks = (R + p.group - 1) / p.group;
@@ -749,6 +749,17 @@ hipError_t LaunchVacancyScan(const KTables &t, const uint8_t *occ, int32_t n, in
                              double *ea, double *de, int32_t *err, hipStream_t s) {
   return LaunchEval<true>(t, occ, nullptr, nullptr, sites, K, nb, ea, de, err, s, nullptr, nullptr, n,
                           sub_site, sub_code);
+}
+
+// Measured, us per step of batches of 12^3 cells (E0, ternary), one wave / four waves per replica:
+//   replicas              1           64          256         512        1 024
+//   1-5 at.% solutes   1.3 / 1.5   2.2 / 1.8   2.3 / 1.8   2.4 / 2.0   2.5 / 3.9
+//   4-20 at.%          4.6 / 2.6   5.4 / 2.8   5.4 / 2.8   5.8 / 3.3   5.9 / 6.5
+//   chain steps                   24.8 / 9.0  25.0 / 9.3  26.4 / 10.9  29.6 / 19.7
+// Formulation 0 takes four where every replica has a CU, and chain steps where two replicas share one.
+bool KmcTeam(int32_t R, int form) {
+  const int cus = CurrentDeviceLimits().cus;
+  return form == 2 || (form == 0 && R <= cus) || (form == 3 && R <= 2 * cus);
 }
 
 hipError_t PrepareKmc(const KTables &t, int32_t R, int form) {

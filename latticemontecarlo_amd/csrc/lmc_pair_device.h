@@ -58,18 +58,18 @@ struct WaveLds {
   double sum[12][3];
 };
 
-// Geometry tables of a workgroup.
+// Geometry tables of a workgroup, each where 16-byte copies may start.
 template <bool kQ>
-struct alignas(16) PairShared {
-  uint32_t cls[(kNoSlot + 1) * kClsRow];
-  uint16_t clsb[kQ ? (kNoSlot + 1) * kClsRow : 8];
-  uint32_t one[12 * kOneRow];                 // cls of a site's slot with itself
-  uint16_t oneb[kQ ? 12 * kOneRow : 8];
-  uint8_t slot[12 * kPairSiteRow];
-  uint8_t order[27 * 16];                     // event directions by the faces the vacancy touches
-  uint2 dense[kMaxDense];                     // slot pairs with a term: cls; 16 s1 | 16 s2 << 16
-  uint16_t denseb[kQ ? kMaxDense : 8];
-  uint32_t site3[4 * kEnvSlots];
+struct PairShared {
+  alignas(16) uint32_t cls[(kNoSlot + 1) * kClsRow];
+  alignas(16) uint16_t clsb[kQ ? (kNoSlot + 1) * kClsRow : 8];
+  alignas(16) uint32_t one[12 * kOneRow];     // cls of a site's slot with itself
+  alignas(16) uint16_t oneb[kQ ? 12 * kOneRow : 8];
+  alignas(16) uint8_t slot[12 * kPairSiteRow];
+  alignas(16) uint8_t order[27 * 16];         // event directions by the faces the vacancy touches
+  alignas(16) uint2 dense[kMaxDense];         // slot pairs with a term: cls; 16 s1 | 16 s2 << 16
+  alignas(16) uint16_t denseb[kQ ? kMaxDense : 8];
+  alignas(16) uint32_t site3[4 * kEnvSlots];
   double base[5 * 3], par[kMaxSpecies * 6];
 };
 
@@ -94,7 +94,8 @@ __device__ __forceinline__ int RankInMask(uint64_t m) {
                           __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
 }
 
-// Copies `bytes` (a multiple of 4, both sides 16-byte aligned) to LDS, 16 bytes per thread and
+// Copies `bytes` (a multiple of 4; both sides 16-byte aligned: the blob's tables lie 256 bytes apart and
+// its value rows of a reference are PairStride doubles) to LDS, 16 bytes per thread and
 // load, four loads in flight: the copy is bound by the latency of its few rounds.
 __device__ __forceinline__ void CopyTable(char *dst, const void *src, int bytes, int tid, int size) {
   const uint4 *s = reinterpret_cast<const uint4 *>(src);
@@ -143,9 +144,9 @@ __device__ __forceinline__ PairTab LoadPairTables(const KTables &t, PairShared<k
   }
   for (int i = tid; i < 3 * t.ne; i += size) G.base[i] = t.pbase[3 * t.ne * rr + i];
   for (int i = tid; i < 6 * t.S; i += size) G.par[i] = t.par[i];
-  const char *de = reinterpret_cast<const char *>(t.de) + rr * t.ne * T.de_row;
-  const char *la = reinterpret_cast<const char *>(t.la) + rr * t.ne * T.la_row;
-  const char *lb = reinterpret_cast<const char *>(t.lb) + rr * t.ne * T.lb_row;
+  const char *de = reinterpret_cast<const char *>(t.de + rr * PairStride(t.ne, t.de_row));
+  const char *la = reinterpret_cast<const char *>(t.la + rr * PairStride(t.ne, t.la_row));
+  const char *lb = reinterpret_cast<const char *>(t.lb + rr * PairStride(t.ne, t.lb_row));
   if (kTab) {
     CopyTable(dyn + lay.de, de, t.ne * T.de_row, tid, size);
     CopyTable(dyn + lay.la, la, t.ne * T.la_row, tid, size);

@@ -223,7 +223,8 @@ PairTables BuildPairTables(const Model &m) {
     for (int s = 0; s < kEnvSlots * kEnvSlots; ++s)
       offs[x][s / kEnvSlots * kClsRow + s % kEnvSlots] = static_cast<uint16_t>(ct.of[s] * block * 8);
     std::vector<double> &tab = *out[x];
-    tab.assign(static_cast<size_t>(ne) * ne * *rows[x], 0.0);
+    const size_t stride = PairStride(ne, *rows[x]);
+    tab.assign(ne * stride, 0.0);
     for (int ref = 0; ref < ne; ++ref) {
       std::vector<int> rank;  // non-reference ranks
       for (int r = 0; r < ne; ++r)
@@ -232,7 +233,7 @@ PairTables BuildPairTables(const Model &m) {
       for (int M = 0; M < ne; ++M)
         for (size_t c = 0; c < ct.classes.size(); ++c) {
           const PairClass &pc = ct.classes[c];
-          double *val = tab.data() + (static_cast<size_t>(ref) * ne + M) * *rows[x] + (c + 1) * block;
+          double *val = tab.data() + ref * stride + static_cast<size_t>(M) * *rows[x] + (c + 1) * block;
           for (int i = 0; i < nr; ++i)
             for (int j = 0; j < nr; ++j) {
               if (pc.single && i != j) continue;

@@ -41,6 +41,9 @@ struct PairGeometry {
 };
 const PairGeometry &GetPairGeometry();
 
+// Doubles between the values of two references: even, so that each starts on 16 bytes.
+constexpr int PairStride(int ne, int row) { return (ne * row + 1) & ~1; }
+
 // Class tables of one model. A class is a block of q * q values (q = ne - 1 non-reference ranks) and
 // one zero after them, block 0 all zero. cls[s1 * 64 + s2] holds the byte offsets of the blocks of the ordered slot pair
 // (s1 == s2: the one-site term, on the block's diagonal) within a row: dE in the low half-word,
@@ -54,7 +57,7 @@ struct PairTables {
   // slot pairs with a term: cls, then 16 s1 | 16 s2 << 16, and clsb; blanks after them
   std::vector<uint32_t> dense;
   std::vector<uint16_t> denseb;
-  std::vector<double> de, la, lb;  // [reference rank][migrating rank][row]
+  std::vector<double> de, la, lb;  // [reference rank][migrating rank][row], references PairStride apart
   int de_row = 0, la_row = 0, lb_row = 0;  // rows in doubles
 };
 PairTables BuildPairTables(const Model &m);

@@ -73,6 +73,10 @@ int main(int argc, char **argv) {
   std::vector<int> code;
   for (int c = 0; c < m->S; ++c)
     if (c != m->x_code) code.push_back(c);
+  // the values of every reference can be copied 16 bytes at a time
+  for (int row : {t.de_row, t.la_row, t.lb_row})
+    if (PairStride(ne, row) % 2 || PairStride(ne, row) < ne * row) return std::puts("stride of the references"), 1;
+  if (t.de.size() != static_cast<size_t>(ne) * PairStride(ne, t.de_row)) return std::puts("size of the values"), 1;
   // geometry: slots and sites name the same offsets, and pairs with a term are near
   for (int d = 0; d < 12; ++d)
     for (int i = 0; i < kPairSites; ++i) {
@@ -118,14 +122,15 @@ int main(int argc, char **argv) {
       none[jt.n_slot] = env[jt.n_slot];
       env[jt.v_slot] = none[jt.v_slot] = ref;
       const Sums want = Clusters(*m, jt, code, env), base = Clusters(*m, jt, code, none);
-      const int M = env[jt.n_slot], of = ref * ne + M;
+      const int M = env[jt.n_slot];
+      auto row = [&](int r) { return static_cast<size_t>(ref) * PairStride(ne, r) + static_cast<size_t>(M) * r; };
       double sparse[3], dense[3];
       for (int i = 0; i < 3; ++i) sparse[i] = dense[i] = static_cast<double>(base.v[i]);
       auto rank = [&](int s) { return env[s] - (env[s] > ref ? 1 : 0); };
       auto add = [&](double *sum, uint32_t c, uint32_t cb, int a, int b) {
-        sum[0] += t.de[static_cast<size_t>(of) * t.de_row + (c & 0xFFFF) / 8 + a * q + b];
-        sum[1] += t.la[static_cast<size_t>(of) * t.la_row + (c >> 16) / 8 + a * q + b];
-        if (m->kind == kQuartic) sum[2] += t.lb[static_cast<size_t>(of) * t.lb_row + cb / 8 + a * q + b];
+        sum[0] += t.de[row(t.de_row) + (c & 0xFFFF) / 8 + a * q + b];
+        sum[1] += t.la[row(t.la_row) + (c >> 16) / 8 + a * q + b];
+        if (m->kind == kQuartic) sum[2] += t.lb[row(t.lb_row) + cb / 8 + a * q + b];
       };
       auto other = [&](int s) { return s != jt.v_slot && s != jt.n_slot && env[s] != ref; };
       for (int a = 0; a < kEnvSlots; ++a)

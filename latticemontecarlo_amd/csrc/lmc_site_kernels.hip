@@ -664,6 +664,9 @@ __global__ __launch_bounds__(kCmcThreads) void CmcKernel(KTables t, CmcDev c, ui
         occ[tp] = L.ep[slot];
         occ[tq] = L.eq[slot];
       }
+      // a taken trial may share a site with one that was not taken (that is what ended the round): its
+      // species are written after
+      WaveFence();
       if (lane < adv) {
         const uint64_t index = trace_base + it + static_cast<uint64_t>(lane);
         if (index < c.trace_cap) {

@@ -169,35 +169,6 @@ Model::~Model() {
   }
 }
 
-// Sums (dE, MMM logit, MM2 logit) of a jump environment whose non-endpoint sites all hold element rank s,
-// by migrating rank M: base[s][M][3].
-static std::vector<double> BuildBaseSums(const Model &m, const JumpTables &jt, const std::vector<int> &code) {
-  const int S = m.S;
-  std::vector<double> base;
-  auto w_of = [&](int label, int a, int s) -> long double {
-    if (label == 0) return m.w[a];
-    if (label < 4) return m.w[S + (label - 1) * S * S + a * S + s];
-    return m.w[S + 3 * S * S + (label - 4) * S * S * S + (a * S + s) * S + s];
-  };
-  auto tt = [&](int kind, int a, int b) { return m.type_tab[(kind * S + a) * S + b]; };
-  for (int s : code)
-    for (int M : code) {
-      long double de = 0, la = 0, lb = 0;
-      for (const auto &c : jt.state_v_only) de += w_of(c.label, M, s) - w_of(c.label, m.x_code, s);
-      for (const auto &c : jt.state_n_only) de -= w_of(c.label, M, s) - w_of(c.label, m.x_code, s);
-      if (m.kind == kE0 || m.kind == kQuartic)
-        for (const auto &c : jt.mmm.clusters)
-          la += m.b_mmm[static_cast<size_t>(M) * m.F_mmm + m.base_mmm[c.orbit] +
-                        tt(jt.mmm.orbit_kind[c.orbit], s, s)];
-      if (m.kind == kQuartic)
-        for (const auto &c : jt.mm2.clusters)
-          lb += 2.0L * m.b_mm2[static_cast<size_t>(M) * m.F_mm2 + m.base_mm2[c.orbit] +
-                               tt(jt.mm2.orbit_kind[c.orbit], s, s)];
-      for (long double x : {de, la, lb}) base.push_back(static_cast<double>(x));
-    }
-  return base;
-}
-
 // Models are shared by host threads (the reference's predictors are const objects called from
 // OpenMP threads), so the lazy upload and every read of m.dev take this lock.
 static std::mutex &UploadMutex() {
@@ -329,52 +300,61 @@ const KTables &Upload(Model &m) {
   b.Add(e1, &k.eci1);
   b.Add(e2, &k.eci2);
   b.Add(e3, &k.eci3);
-  const PairGeometry &pg = GetPairGeometry();
-  const PairTables pt = BuildPairTables(m);
-  std::vector<int32_t> site_pk;
-  for (const I3 &o : pg.site) site_pk.push_back(PackOff(o));
-  std::vector<uint8_t> slot, site_of;
-  for (int d = 0; d < 12; ++d) {
-    slot.insert(slot.end(), pg.slot[d].begin(), pg.slot[d].end());
-    site_of.insert(site_of.end(), pg.site_of[d].begin(), pg.site_of[d].end());
-  }
-  const std::vector<double> pbase = BuildBaseSums(m, jt, code);
-  b.Add(site_pk, &k.site_pk);
-  b.Add(slot, &k.slot);
-  std::vector<uint32_t> site3;
-  for (const auto &s : pg.site3) site3.insert(site3.end(), s.begin(), s.end());
-  b.Add(site_of, &k.site_of);
-  std::vector<int32_t> env_pk(2 * 12 * 64, 0);
-  for (int d = 0; d < 12; ++d)
-    for (int s = 0; s < kEnvSlots; ++s) {
-      if (pg.site_of[d][s] < kPairSites) env_pk[64 * d + s] = site_pk[pg.site_of[d][s]];  // the vacancy's own: 0
-      env_pk[64 * (12 + d) + s] = PackOff(pg.back[d][s]);
+  const bool barrier = m.kind == kE0 || m.kind == kQuartic;
+  if (barrier) {  // the jump kernels' tables
+    const PairGeometry &pg = GetPairGeometry();
+    const PairTables &pt = GetPairTables(ne, m.kind == kQuartic);
+    std::vector<int32_t> site_pk;
+    for (const I3 &o : pg.site) site_pk.push_back(PackOff(o));
+    std::vector<uint8_t> slot, site_of;
+    for (int d = 0; d < 12; ++d) {
+      slot.insert(slot.end(), pg.slot[d].begin(), pg.slot[d].end());
+      site_of.insert(site_of.end(), pg.site_of[d].begin(), pg.site_of[d].end());
     }
-  b.Add(env_pk, &k.env_pk);
-  b.Add(site3, &k.site3);
-  b.Add(pt.cls, &k.cls);
-  b.Add(pt.clsb, &k.clsb);
-  b.Add(pt.dense, &k.dense);
-  b.Add(pt.denseb, &k.denseb);
-  b.Add(pt.one, &k.one);
-  b.Add(pt.oneb, &k.oneb);
-  std::vector<uint8_t> order;
-  for (const auto &o : pg.order) order.insert(order.end(), o.begin(), o.end());
-  b.Add(order, &k.order);
-  b.Add(pt.de, &k.de);
-  b.Add(pt.la, &k.la);
-  b.Add(pt.lb, &k.lb);
-  b.Add(pbase, &k.pbase);
-  k.de_row = pt.de_row;
-  k.la_row = pt.la_row;
-  k.lb_row = pt.lb_row;
+    b.Add(site_pk, &k.site_pk);
+    b.Add(slot, &k.slot);
+    std::vector<uint32_t> site3;
+    for (const auto &s : pg.site3) site3.insert(site3.end(), s.begin(), s.end());
+    b.Add(site_of, &k.site_of);
+    std::vector<int32_t> env_pk(2 * 12 * 64, 0);
+    for (int d = 0; d < 12; ++d)
+      for (int s = 0; s < kEnvSlots; ++s) {
+        if (pg.site_of[d][s] < kPairSites) env_pk[64 * d + s] = site_pk[pg.site_of[d][s]];  // the vacancy's own: 0
+        env_pk[64 * (12 + d) + s] = PackOff(pg.back[d][s]);
+      }
+    b.Add(env_pk, &k.env_pk);
+    b.Add(site3, &k.site3);
+    b.Add(pt.cls, &k.cls);
+    b.Add(pt.clsb, &k.clsb);
+    b.Add(pt.dense, &k.dense);
+    b.Add(pt.denseb, &k.denseb);
+    b.Add(pt.one, &k.one);
+    b.Add(pt.oneb, &k.oneb);
+    std::vector<uint8_t> order;
+    for (const auto &o : pg.order) order.insert(order.end(), o.begin(), o.end());
+    b.Add(order, &k.order);
+    k.de_row = pt.de_row;
+    k.la_row = pt.la_row;
+    k.lb_row = pt.lb_row;
+  }
   std::vector<int32_t> errflag(1, 0);
   const int32_t *err_ptr = nullptr;
   b.Add(errflag, &err_ptr);
+  k.solvent_default = 0;
+  for (int c = 0; c < m.S; ++c)
+    if (m.eci.species[c] == "Al") k.solvent_default = c;
+  if (k.solvent_default == m.x_code) k.solvent_default = m.x_code == 0 ? 1 : 0;
 
   auto dev = std::make_unique<DeviceTables>();
   dev->device = device;
-  Check(hipMalloc(&dev->blob, b.bytes.size()), "hipMalloc(model tables)");
+  size_t others = 0;  // room behind the tables for the other references' values
+  if (barrier) {
+    k.first_ref = m.onehot[k.solvent_default];
+    b.Add(BuildPairValues(m, k.first_ref), &k.pairs);
+    others = static_cast<size_t>(ne - 1) * PairBlockOf(ne, k.de_row, k.la_row, k.lb_row).size * sizeof(double);
+    dev->refs = 1u << k.first_ref;
+  }
+  Check(hipMalloc(&dev->blob, b.bytes.size() + others), "hipMalloc(model tables)");
   Check(hipMemcpy(dev->blob, b.bytes.data(), b.bytes.size(), hipMemcpyHostToDevice),
         "hipMemcpy(model tables)");
   for (auto &f : b.fix) *f.second = static_cast<char *>(dev->blob) + f.first;
@@ -397,14 +377,22 @@ const KTables &Upload(Model &m) {
   k.nwd = static_cast<int>(wd.size());
   k.wrow = wrow;
   k.rank_lut = rank_lut;
-  k.solvent_default = 0;
-  for (int c = 0; c < m.S; ++c)
-    if (m.eci.species[c] == "Al") k.solvent_default = c;
-  if (k.solvent_default == m.x_code) k.solvent_default = m.x_code == 0 ? 1 : 0;
   dev->k = k;
   m.dev = dev.release();
   m.dev_err = const_cast<int32_t *>(err_ptr);
   return m.dev->k;
+}
+
+void NeedReference(Model &m, int code) {
+  const KTables &k = Upload(m);
+  const int ref = m.onehot[code];
+  std::lock_guard<std::mutex> lock(UploadMutex());
+  if (!k.pairs || ref < 0 || (m.dev->refs >> ref) & 1) return;
+  const std::vector<double> v = BuildPairValues(m, ref);
+  const size_t at = v.size() * static_cast<size_t>(ref + (ref < k.first_ref ? 1 : 0));
+  Check(hipMemcpy(const_cast<double *>(k.pairs) + at, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice),
+        "hipMemcpy(model tables)");
+  m.dev->refs |= 1u << ref;
 }
 
 }  // namespace lmc
@@ -1305,7 +1293,7 @@ int lmc_kmc_create(const lmc_model *barrier, const lmc_model *energy, int32_t R,
       }
       d.prev_j = DevCopy(prev);
     }
-    lmc::Upload(*barrier->m);
+    for (int32_t c : solvent) lmc::NeedReference(*barrier->m, c);
     if (energy) {
       RequireModel(energy);
       ComputeTotalEnergy(energy, d.occ, d.off, d.ncell, R, d.abs_energy, nullptr);

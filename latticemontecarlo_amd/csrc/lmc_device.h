@@ -43,9 +43,9 @@ struct KTables {
   const int32_t *eci1;      // [S]
   const int32_t *eci2;      // [3][S][S]
   const int32_t *eci3;      // [4][S][S][S]
-  // Quadratic form of the jump sums (lmc_pairs.h): geometry, class offsets, values by
-  // [reference rank][migrating rank][row], and the all-reference sums pbase (dE, MMM, MM2 logit)
-  // by [reference rank][migrating rank][3].
+  // Quadratic form of the jump sums (lmc_pairs.h): geometry, class offsets, and a block of values
+  // (PairBlock) per reference: the model's default one first, then the others by rank. A block is there
+  // once NeedReference has been called for its species.
   const int32_t *site_pk;   // [134] signed byte offsets x | y << 8 | z << 16
   const uint8_t *slot;      // [12][136]
   const uint8_t *site_of;   // [12][60]
@@ -53,8 +53,8 @@ struct KTables {
   const uint8_t *order;     // [27][16]
   const uint32_t *cls, *one, *dense;
   const uint16_t *clsb, *oneb, *denseb;
-  const double *de, *la, *lb, *pbase;
-  int de_row, la_row, lb_row;
+  const double *pairs;
+  int de_row, la_row, lb_row, first_ref;
   int solvent_default;
   uint64_t vac_shell_mask;  // env slots within 3NN of the vacancy
   int n_state, n_mmm, n_mm2, n_site, n_eci;  // n_mm2 counts forward + backward entries
@@ -69,11 +69,14 @@ struct DeviceTables {
   int device = -1;
   void *blob = nullptr;  // one allocation holding every table
   KTables k{};
+  uint32_t refs = 0;     // references whose block of values is there, a bit per rank
 };
 
 // Uploads (once) and returns the kernel view of a model on the current device. Thread-safe, as
-// are the two queries below.
+// are the calls below.
 const KTables &Upload(Model &m);
+// Forms the values of reference species `code` if they are not there (Upload has formed the default's).
+void NeedReference(Model &m, int code);
 bool IsUploaded(const Model &m);
 // The kernel view when the model is already on `device`, else null (never uploads).
 const KTables *UploadedOn(const Model &m, int device);

@@ -95,7 +95,7 @@ __device__ __forceinline__ int RankInMask(uint64_t m) {
 }
 
 // Copies `bytes` (a multiple of 4; both sides 16-byte aligned: the blob's tables lie 256 bytes apart and
-// its value rows of a reference are PairStride doubles) to LDS, 16 bytes per thread and
+// the parts of a PairBlock start on 16 bytes) to LDS, 16 bytes per thread and
 // load, four loads in flight: the copy is bound by the latency of its few rounds.
 __device__ __forceinline__ void CopyTable(char *dst, const void *src, int bytes, int tid, int size) {
   const uint4 *s = reinterpret_cast<const uint4 *>(src);
@@ -142,11 +142,14 @@ __device__ __forceinline__ PairTab LoadPairTables(const KTables &t, PairShared<k
     CopyTable(reinterpret_cast<char *>(G.oneb), t.oneb, sizeof(G.oneb), tid, size);
     CopyTable(reinterpret_cast<char *>(G.denseb), t.denseb, sizeof(G.denseb), tid, size);
   }
-  for (int i = tid; i < 3 * t.ne; i += size) G.base[i] = t.pbase[3 * t.ne * rr + i];
+  // the first reference's block, then the others' by rank
+  const PairBlock at = PairBlockOf(t.ne, t.de_row, t.la_row, t.lb_row);
+  const double *v = t.pairs + (rr == t.first_ref ? 0 : rr + (rr < t.first_ref ? 1 : 0)) * at.size;
+  for (int i = tid; i < 3 * t.ne; i += size) G.base[i] = v[at.base + i];
   for (int i = tid; i < 6 * t.S; i += size) G.par[i] = t.par[i];
-  const char *de = reinterpret_cast<const char *>(t.de + rr * PairStride(t.ne, t.de_row));
-  const char *la = reinterpret_cast<const char *>(t.la + rr * PairStride(t.ne, t.la_row));
-  const char *lb = reinterpret_cast<const char *>(t.lb + rr * PairStride(t.ne, t.lb_row));
+  const char *de = reinterpret_cast<const char *>(v);
+  const char *la = reinterpret_cast<const char *>(v + at.la);
+  const char *lb = reinterpret_cast<const char *>(v + at.lb);
   if (kTab) {
     CopyTable(dyn + lay.de, de, t.ne * T.de_row, tid, size);
     CopyTable(dyn + lay.la, la, t.ne * T.la_row, tid, size);

@@ -2,6 +2,9 @@
 #include "lmc_pairs.h"
 
 #include <algorithm>
+#include <map>
+#include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <tuple>
 
@@ -18,10 +21,12 @@ PairGeometry BuildPairGeometry() {
   for (int k = 0; k < 12; ++k) dir[k] = k;
   std::sort(dir.begin(), dir.end(), [](int a, int b) { return Key(kNN1[a]) < Key(kNN1[b]); });
   std::vector<I3> sites;
+  uint8_t at[9][9][9];  // site at an offset, every component of which is within four
+  std::fill_n(&at[0][0][0], 9 * 9 * 9, static_cast<uint8_t>(kPairSites));
+  auto site_at = [&](const I3 &o) -> uint8_t & { return at[o.x + 4][o.y + 4][o.z + 4]; };
   auto add = [&](const I3 &o) {
-    if (Key(o) == Key(I3{0, 0, 0})) return;
-    for (const I3 &s : sites)
-      if (Key(s) == Key(o)) return;
+    if (Key(o) == Key(I3{0, 0, 0}) || site_at(o) != kPairSites) return;
+    site_at(o) = static_cast<uint8_t>(sites.size());
     sites.push_back(o);
   };
   for (int k : dir) add(kNN1[k]);
@@ -34,13 +39,9 @@ PairGeometry BuildPairGeometry() {
   for (int d = 0; d < 12; ++d) {
     g.slot[d].fill(kNoSlot);
     for (int s = 0; s < kEnvSlots; ++s) {
-      const I3 &o = jt.off[dir[d]][s];
-      g.site_of[d][s] = kPairSites;
-      for (int i = 0; i < kPairSites; ++i)
-        if (Key(g.site[i]) == Key(o)) {
-          g.site_of[d][s] = static_cast<uint8_t>(i);
-          if (s != jt.v_slot && s != jt.n_slot) g.slot[d][i] = static_cast<uint8_t>(s);
-        }
+      const int i = site_at(jt.off[dir[d]][s]);
+      g.site_of[d][s] = static_cast<uint8_t>(i);
+      if (s != jt.v_slot && s != jt.n_slot) g.slot[d][i] = static_cast<uint8_t>(s);
     }
   }
   for (int d = 0; d < 12; ++d)  // the direction back is 11 - d
@@ -79,12 +80,6 @@ namespace {
 enum { kVacancyState, kNeighbourState, kMmm, kMm2, kMm2Backward };
 struct Member {
   int kind, id, role, count;
-  bool operator<(const Member &o) const {
-    return std::tie(kind, id, role) < std::tie(o.kind, o.id, o.role);
-  }
-  bool operator==(const Member &o) const {
-    return kind == o.kind && id == o.id && role == o.role && count == o.count;
-  }
 };
 struct PairClass {
   bool single;
@@ -126,94 +121,71 @@ ClassTable BuildClasses(int sum) {
     orbits(jt.mm2, kMm2, false);
     orbits(jt.mm2, kMm2Backward, true);
   }
-  std::vector<std::vector<Member>> mem(kEnvSlots * kEnvSlots);
+  // cluster kind, id and role of every slot pair's members
+  constexpr int kPairs = kEnvSlots * kEnvSlots;
+  std::vector<std::pair<int, uint32_t>> all;
+  std::vector<int> start(kPairs + 1, 0);
+  all.reserve(4 * terms.size());
   auto put = [&](int s1, int s2, const Term &e, int role) {
-    mem[s1 * kEnvSlots + s2].push_back({e.kind, e.id, e.symmetric ? 0 : role, 1});
+    const int s = s1 * kEnvSlots + s2;
+    ++start[s + 1];
+    all.emplace_back(s, static_cast<uint32_t>(e.kind << 24 | e.id << 2 | role));
   };
   for (const Term &e : terms) {
     if (e.s1 < 0) {
-      mem[e.s0 * kEnvSlots + e.s0].push_back({e.kind, e.id, 2, 1});
+      put(e.s0, e.s0, e, 2);
       continue;
     }
+    const int second = e.symmetric ? 0 : 1;
     put(e.s0, e.s0, e, 0);
-    put(e.s1, e.s1, e, 1);
+    put(e.s1, e.s1, e, second);
     put(e.s0, e.s1, e, 0);
-    put(e.s1, e.s0, e, 1);
+    put(e.s1, e.s0, e, second);
   }
+  for (int s = 0; s < kPairs; ++s) start[s + 1] += start[s];
+  std::vector<uint32_t> members(all.size());
+  std::vector<int> end(start.begin(), start.end() - 1);
+  for (const auto &[s, m] : all) members[end[s]++] = m;
   ClassTable t;
   t.of.assign(kEnvSlots * kEnvSlots, 0);
-  for (int s = 0; s < kEnvSlots * kEnvSlots; ++s) {
-    if (mem[s].empty()) continue;
-    std::sort(mem[s].begin(), mem[s].end());
-    std::vector<Member> merged;
-    for (const Member &m : mem[s]) {
-      if (!merged.empty() && !(merged.back() < m)) ++merged.back().count;
-      else merged.push_back(m);
-    }
+  std::map<std::vector<uint32_t>, int> known;  // the members of a class, each followed by its count
+  std::vector<uint32_t> key;
+  for (int s = 0; s < kPairs; ++s) {
+    if (start[s] == end[s]) continue;
+    std::sort(members.begin() + start[s], members.begin() + end[s]);
     const bool single = s / kEnvSlots == s % kEnvSlots;
-    int at = -1;
-    for (size_t i = 0; i < t.classes.size() && at < 0; ++i)
-      if (t.classes[i].single == single && t.classes[i].members == merged) at = static_cast<int>(i);
-    if (at < 0) {
-      at = static_cast<int>(t.classes.size());
-      t.classes.push_back({single, merged});
+    key.assign(1, single);
+    for (int i = start[s]; i < end[s]; ++i) {
+      if (key.size() > 1 && key[key.size() - 2] == members[i]) ++key.back();
+      else key.insert(key.end(), {members[i], 1u});
     }
-    t.of[s] = at + 1;
+    auto at = known.find(key);
+    if (at == known.end()) {
+      at = known.emplace(key, static_cast<int>(t.classes.size())).first;
+      PairClass c{single, {}};
+      for (size_t k = 1; k < key.size(); k += 2)
+        c.members.push_back({static_cast<int>(key[k] >> 24), static_cast<int>(key[k] >> 2) & 0x3FFFFF,
+                             static_cast<int>(key[k] & 3), static_cast<int>(key[k + 1])});
+      t.classes.push_back(std::move(c));
+    }
+    t.of[s] = at->second + 1;
   }
   return t;
 }
 
+template <int kSum>
+const ClassTable &ClassesOf() {
+  static const ClassTable t = BuildClasses(kSum);
+  return t;
+}
 const ClassTable &Classes(int sum) {
-  static const ClassTable t[3] = {BuildClasses(0), BuildClasses(1), BuildClasses(2)};
-  return t[sum];
+  return sum == 0 ? ClassesOf<0>() : sum == 1 ? ClassesOf<1>() : ClassesOf<2>();
 }
 
-}  // namespace
-
-PairTables BuildPairTables(const Model &m) {
-  const JumpTables &jt = GetJumpTables();
-  const int S = m.S, ne = m.ne, q = std::max(1, ne - 1), block = q * q + 1;
-  const bool quartic = m.kind == kQuartic;
+PairTables BuildPairTables(int ne, bool quartic) {
+  const int q = std::max(1, ne - 1), block = q * q + 1;
   PairTables t;
-  if (m.kind != kE0 && m.kind != kQuartic) return t;
-  std::vector<int> code;  // element rank -> species code
-  for (int c = 0; c < S; ++c)
-    if (c != m.x_code) code.push_back(c);
-  // value of a cluster of each kind and label or orbit: [id][M][a][b] over ranks
-  const size_t row = static_cast<size_t>(ne) * ne * ne;
-  std::vector<long double> values[5];
-  auto each = [&](std::vector<long double> &v, int ids, auto &&f) {
-    v.resize(ids * row);
-    size_t i = 0;
-    for (int id = 0; id < ids; ++id)
-      for (int M = 0; M < ne; ++M)
-        for (int a = 0; a < ne; ++a)
-          for (int b = 0; b < ne; ++b) v[i++] = f(id, M, a, b);
-  };
-  auto w = [&](int label, int x, int a, int b) -> long double {
-    if (label == 0) return m.w[x];
-    if (label < 4) return m.w[S + (label - 1) * S * S + x * S + code[a]];
-    return m.w[S + 3 * S * S + (label - 4) * S * S * S + (x * S + code[a]) * S + code[b]];
-  };
-  each(values[kVacancyState], 8, [&](int id, int M, int a, int b) {
-    return w(id, code[M], a, b) - w(id, m.x_code, a, b);
-  });
-  values[kNeighbourState] = values[kVacancyState];
-  for (long double &x : values[kNeighbourState]) x = -x;
-  auto orbit = [&](const OrbitTable &ot, const std::vector<double> &bw, int F, const std::vector<int> &base) {
-    return [&, F](int id, int M, int a, int b) -> long double {
-      const int kind = ot.orbit_kind[id];
-      const int ty = m.type_tab[(kind * S + code[a]) * S + (kind == 0 ? code[0] : code[b])];
-      return bw[static_cast<size_t>(code[M]) * F + base[id] + ty];
-    };
-  };
-  each(values[kMmm], static_cast<int>(jt.mmm.orbit_kind.size()), orbit(jt.mmm, m.b_mmm, m.F_mmm, m.base_mmm));
-  if (quartic) {
-    each(values[kMm2], static_cast<int>(jt.mm2.orbit_kind.size()), orbit(jt.mm2, m.b_mm2, m.F_mm2, m.base_mm2));
-    values[kMm2Backward] = values[kMm2];
-  }
   std::vector<uint16_t> offs[3];
-  std::vector<double> *out[3] = {&t.de, &t.la, &t.lb};
   int *rows[3] = {&t.de_row, &t.la_row, &t.lb_row};
   for (int x = 0; x < (quartic ? 3 : 2); ++x) {
     const ClassTable &ct = Classes(x);
@@ -222,36 +194,6 @@ PairTables BuildPairTables(const Model &m) {
     offs[x].assign((kNoSlot + 1) * kClsRow, 0);
     for (int s = 0; s < kEnvSlots * kEnvSlots; ++s)
       offs[x][s / kEnvSlots * kClsRow + s % kEnvSlots] = static_cast<uint16_t>(ct.of[s] * block * 8);
-    std::vector<double> &tab = *out[x];
-    const size_t stride = PairStride(ne, *rows[x]);
-    tab.assign(ne * stride, 0.0);
-    for (int ref = 0; ref < ne; ++ref) {
-      std::vector<int> rank;  // non-reference ranks
-      for (int r = 0; r < ne; ++r)
-        if (r != ref) rank.push_back(r);
-      const int nr = static_cast<int>(rank.size());  // 0 with one element: every term is zero
-      for (int M = 0; M < ne; ++M)
-        for (size_t c = 0; c < ct.classes.size(); ++c) {
-          const PairClass &pc = ct.classes[c];
-          double *val = tab.data() + ref * stride + static_cast<size_t>(M) * *rows[x] + (c + 1) * block;
-          for (int i = 0; i < nr; ++i)
-            for (int j = 0; j < nr; ++j) {
-              if (pc.single && i != j) continue;
-              const int a = rank[i], b = rank[j];
-              long double sum = 0;
-              for (const Member &e : pc.members) {
-                const long double *v = values[e.kind].data() + e.id * row + static_cast<size_t>(M) * ne * ne;
-                auto at = [&](int p, int r) { return v[p * ne + r]; };
-                if (pc.single)  // role 2: a singlet, whose value ignores the second rank
-                  sum += e.count * ((e.role == 1 ? at(ref, a) : at(a, ref)) - at(ref, ref));
-                else
-                  sum += e.count * ((e.role ? at(b, a) - at(b, ref) - at(ref, a)
-                                            : at(a, b) - at(a, ref) - at(ref, b)) + at(ref, ref));
-              }
-              val[i * q + j] = static_cast<double>(sum);
-            }
-        }
-    }
   }
   t.cls.resize(offs[0].size());
   for (size_t i = 0; i < t.cls.size(); ++i)
@@ -276,6 +218,125 @@ PairTables BuildPairTables(const Model &m) {
       t.oneb.push_back(quartic ? t.clsb[at] : 0);
     }
   return t;
+}
+
+}  // namespace
+
+const PairTables &GetPairTables(int ne, bool quartic) {
+  static std::mutex mu;
+  static std::unique_ptr<const PairTables> known[kMaxSpecies + 1][2];
+  std::lock_guard<std::mutex> lock(mu);
+  auto &t = known[std::clamp(ne, 0, kMaxSpecies)][quartic];
+  if (!t) t = std::make_unique<const PairTables>(BuildPairTables(ne, quartic));
+  return *t;
+}
+
+std::vector<double> BuildPairValues(const Model &m, int ref) {
+  const JumpTables &jt = GetJumpTables();
+  const int S = m.S, ne = m.ne, q = std::max(1, ne - 1), block = q * q + 1;
+  const bool quartic = m.kind == kQuartic;
+  const PairTables &t = GetPairTables(ne, quartic);
+  const PairBlock at = PairBlockOf(ne, t.de_row, t.la_row, t.lb_row);
+  std::vector<double> out(at.size, 0.0);
+  std::vector<int> code;  // element rank -> species code
+  for (int c = 0; c < S; ++c)
+    if (c != m.x_code) code.push_back(c);
+  // weight of a cluster of a label or orbit over element ranks: [label][M, or ne: the vacancy][a][b] and
+  // [orbit][M][a][b]
+  const size_t cells = static_cast<size_t>(ne) * ne, state_row = cells * (ne + 1), row = cells * ne;
+  std::vector<double> state(8 * state_row), mmm(jt.mmm.orbit_kind.size() * row), mm2(quartic ? jt.mm2.orbit_kind.size() * row : 0);
+  size_t i = 0;
+  for (int label = 0; label < 8; ++label)
+    for (int M = 0; M <= ne; ++M) {
+      const int x = M < ne ? code[M] : m.x_code;
+      for (int a = 0; a < ne; ++a)
+        for (int b = 0; b < ne; ++b)
+          state[i++] = label == 0  ? m.w[x]
+                       : label < 4 ? m.w[S + (label - 1) * S * S + x * S + code[a]]
+                                   : m.w[S + 3 * S * S + (label - 4) * S * S * S + (x * S + code[a]) * S + code[b]];
+    }
+  std::vector<int> type(3 * cells);  // one-hot type by orbit kind and ranks
+  for (int kind = 0; kind < 3; ++kind)
+    for (int a = 0; a < ne; ++a)
+      for (int b = 0; b < ne; ++b) type[kind * cells + a * ne + b] = m.type_tab[(kind * S + code[a]) * S + (kind == 0 ? code[0] : code[b])];
+  auto orbits = [&](std::vector<double> &v, const OrbitTable &ot, const std::vector<double> &bw, int F, const std::vector<int> &base) {
+    for (size_t id = 0, at = 0; id < ot.orbit_kind.size(); ++id)
+      for (int M = 0; M < ne; ++M) {
+        const double *w = bw.data() + static_cast<size_t>(code[M]) * F + base[id];
+        const int *ty = type.data() + ot.orbit_kind[id] * cells;
+        for (size_t k = 0; k < cells; ++k) v[at++] = w[ty[k]];
+      }
+  };
+  orbits(mmm, jt.mmm, m.b_mmm, m.F_mmm, m.base_mmm);
+  if (quartic) orbits(mm2, jt.mm2, m.b_mm2, m.F_mm2, m.base_mm2);
+  // the weights that a class adds, for one migrating rank; sums in 64-bit mantissas
+  struct Weights {
+    const double *v;
+    long double count;
+    int da, db;  // strides of the first site's rank and the second's
+  };
+  std::vector<Weights> terms;
+  const int rows[3] = {t.de_row, t.la_row, t.lb_row}, part[3] = {0, at.la, at.lb};
+  for (int x = 0; x < (quartic ? 3 : 2); ++x) {
+    const ClassTable &ct = Classes(x);
+    for (size_t c = 0; c < ct.classes.size(); ++c)
+      for (int M = 0; M < ne; ++M) {
+        const PairClass &pc = ct.classes[c];
+        terms.clear();
+        for (const Member &e : pc.members) {
+          const int da = e.role == 1 ? 1 : ne, db = e.role == 1 ? ne : 1;
+          if (e.kind <= kNeighbourState) {  // the endpoint's change from a vacancy to M, or back
+            const double *v = state.data() + e.id * state_row;
+            const long double count = e.kind == kVacancyState ? e.count : -e.count;
+            terms.push_back({v + M * cells, count, da, db});
+            terms.push_back({v + ne * cells, -count, da, db});
+          } else {
+            terms.push_back({(e.kind == kMmm ? mmm : mm2).data() + e.id * row + M * cells, static_cast<long double>(e.count), da, db});
+          }
+        }
+        double *val = out.data() + part[x] + static_cast<size_t>(M) * rows[x] + (c + 1) * block;
+        for (int k = 0, a = 0; a < ne; ++a) {  // with one element there is none but the reference: zeros
+          if (a == ref) continue;
+          if (pc.single) {  // its pairs are with reference sites; a singlet's weight ignores the second rank
+            long double f1 = 0;
+            for (const Weights &w : terms) {
+              const double *v = w.v + ref * w.db;
+              f1 += w.count * (static_cast<long double>(v[a * w.da]) - v[ref * w.da]);
+            }
+            val[k * q + k] = static_cast<double>(f1);
+          } else {
+            for (int l = 0, b = 0; b < ne; ++b) {
+              if (b == ref) continue;
+              long double f2 = 0;
+              for (const Weights &w : terms) {
+                const double *va = w.v + a * w.da, *vr = w.v + ref * w.da;
+                f2 += w.count * ((static_cast<long double>(va[b * w.db]) - va[ref * w.db]) - (static_cast<long double>(vr[b * w.db]) - vr[ref * w.db]));
+              }
+              val[k * q + l++] = static_cast<double>(f2);
+            }
+          }
+          ++k;
+        }
+      }
+  }
+  // all-reference sums: every cluster of a label or orbit has the same weight
+  const size_t same = static_cast<size_t>(ref) * ne + ref;
+  int of_label[8] = {};
+  for (const auto &c : jt.state_v_only) ++of_label[c.label];
+  for (const auto &c : jt.state_n_only) --of_label[c.label];
+  for (int M = 0; M < ne; ++M) {
+    long double de = 0, la = 0, lb = 0;
+    for (int label = 0; label < 8; ++label)
+      de += of_label[label] * (static_cast<long double>(state[label * state_row + M * cells + same]) - state[label * state_row + ne * cells + same]);
+    for (size_t o = 0; o < jt.mmm.orbit_size.size(); ++o) la += jt.mmm.orbit_size[o] * static_cast<long double>(mmm[o * row + M * cells + same]);
+    if (quartic)
+      for (size_t o = 0; o < jt.mm2.orbit_size.size(); ++o) lb += 2 * jt.mm2.orbit_size[o] * static_cast<long double>(mm2[o * row + M * cells + same]);
+    double *o = out.data() + at.base + 3 * M;
+    o[0] = static_cast<double>(de);
+    o[1] = static_cast<double>(la);
+    o[2] = static_cast<double>(lb);
+  }
+  return out;
 }
 
 }  // namespace lmc

@@ -41,10 +41,7 @@ struct PairGeometry {
 };
 const PairGeometry &GetPairGeometry();
 
-// Doubles between the values of two references: even, so that each starts on 16 bytes.
-constexpr int PairStride(int ne, int row) { return (ne * row + 1) & ~1; }
-
-// Class tables of one model. A class is a block of q * q values (q = ne - 1 non-reference ranks) and
+// Class lists of the models with one number of elements. A class is a block of q * q values (q = ne - 1 non-reference ranks) and
 // one zero after them, block 0 all zero. cls[s1 * 64 + s2] holds the byte offsets of the blocks of the ordered slot pair
 // (s1 == s2: the one-site term, on the block's diagonal) within a row: dE in the low half-word,
 // the MMM logit in the high one; clsb the MM2 logit's. A block is indexed by the rank at s1 times q
@@ -57,9 +54,22 @@ struct PairTables {
   // slot pairs with a term: cls, then 16 s1 | 16 s2 << 16, and clsb; blanks after them
   std::vector<uint32_t> dense;
   std::vector<uint16_t> denseb;
-  std::vector<double> de, la, lb;  // [reference rank][migrating rank][row], references PairStride apart
-  int de_row = 0, la_row = 0, lb_row = 0;  // rows in doubles
+  int de_row = 0, la_row = 0, lb_row = 0;  // rows of the values, in doubles
 };
-PairTables BuildPairTables(const Model &m);
+const PairTables &GetPairTables(int ne, bool quartic);  // ne: the model's elements
+
+// The values of one reference species, in doubles: [migrating rank][row] of the dE, MMM and MM2 classes and
+// the all-reference sums [migrating rank][dE, MMM, MM2 logit]. Each part starts on 16 bytes, as does the
+// next reference's block.
+struct PairBlock {
+  int la, lb, base, size;  // where the parts start (dE: at 0), and the length of all
+};
+constexpr PairBlock PairBlockOf(int ne, int de_row, int la_row, int lb_row) {
+  const int la = (ne * de_row + 1) & ~1, lb = la + ((ne * la_row + 1) & ~1), base = lb + ((ne * lb_row + 1) & ~1);
+  return {la, lb, base, base + ((3 * ne + 1) & ~1)};
+}
+// The block of reference rank ref. The engine forms a species' block when a batch first has it as its
+// solvent: all of a five-element Quartic model's take 1 ms.
+std::vector<double> BuildPairValues(const Model &m, int ref);
 
 }  // namespace lmc

@@ -68,15 +68,16 @@ int main(int argc, char **argv) {
   Model *m = LoadModel(argv[1], els, std::atoi(argv[2]));
   const JumpTables &jt = GetJumpTables();
   const PairGeometry &g = GetPairGeometry();
-  const PairTables t = BuildPairTables(*m);
+  const PairTables &t = GetPairTables(m->ne, m->kind == kQuartic);
   const int ne = m->ne, q = std::max(1, ne - 1);
   std::vector<int> code;
   for (int c = 0; c < m->S; ++c)
     if (c != m->x_code) code.push_back(c);
-  // the values of every reference can be copied 16 bytes at a time
-  for (int row : {t.de_row, t.la_row, t.lb_row})
-    if (PairStride(ne, row) % 2 || PairStride(ne, row) < ne * row) return std::puts("stride of the references"), 1;
-  if (t.de.size() != static_cast<size_t>(ne) * PairStride(ne, t.de_row)) return std::puts("size of the values"), 1;
+  // the parts of a block can be copied 16 bytes at a time and do not overlap
+  const PairBlock bl = PairBlockOf(ne, t.de_row, t.la_row, t.lb_row);
+  if (bl.la % 2 || bl.lb % 2 || bl.base % 2 || bl.size % 2 || bl.la < ne * t.de_row || bl.lb < bl.la + ne * t.la_row ||
+      bl.base < bl.lb + ne * t.lb_row || bl.size < bl.base + 3 * ne)
+    return std::puts("parts of a block"), 1;
   // geometry: slots and sites name the same offsets, and pairs with a term are near
   for (int d = 0; d < 12; ++d)
     for (int i = 0; i < kPairSites; ++i) {
@@ -111,7 +112,9 @@ int main(int argc, char **argv) {
       return std::puts("directions are not in opposite order"), 1;
   std::mt19937 rng(7);
   double worst = 0;
-  for (int ref = 0; ref < ne; ++ref)
+  for (int ref = 0; ref < ne; ++ref) {
+    const std::vector<double> v = BuildPairValues(*m, ref);
+    if (v.size() != static_cast<size_t>(bl.size)) return std::puts("size of the values"), 1;
     for (int trial = 0; trial < 200; ++trial) {
       int env[kEnvSlots], none[kEnvSlots];
       const double fill = trial % 4 == 3 ? 1.0 : 0.15 * (1 + trial % 4);
@@ -123,14 +126,17 @@ int main(int argc, char **argv) {
       env[jt.v_slot] = none[jt.v_slot] = ref;
       const Sums want = Clusters(*m, jt, code, env), base = Clusters(*m, jt, code, none);
       const int M = env[jt.n_slot];
-      auto row = [&](int r) { return static_cast<size_t>(ref) * PairStride(ne, r) + static_cast<size_t>(M) * r; };
       double sparse[3], dense[3];
-      for (int i = 0; i < 3; ++i) sparse[i] = dense[i] = static_cast<double>(base.v[i]);
+      for (int i = 0; i < 3; ++i) {
+        sparse[i] = dense[i] = v[bl.base + 3 * M + i];
+        const double size = static_cast<double>(base.size[i]) + 1e-300;
+        worst = std::max(worst, std::fabs(sparse[i] - static_cast<double>(base.v[i])) / size);
+      }
       auto rank = [&](int s) { return env[s] - (env[s] > ref ? 1 : 0); };
       auto add = [&](double *sum, uint32_t c, uint32_t cb, int a, int b) {
-        sum[0] += t.de[row(t.de_row) + (c & 0xFFFF) / 8 + a * q + b];
-        sum[1] += t.la[row(t.la_row) + (c >> 16) / 8 + a * q + b];
-        if (m->kind == kQuartic) sum[2] += t.lb[row(t.lb_row) + cb / 8 + a * q + b];
+        sum[0] += v[M * t.de_row + (c & 0xFFFF) / 8 + a * q + b];
+        sum[1] += v[bl.la + M * t.la_row + (c >> 16) / 8 + a * q + b];
+        if (m->kind == kQuartic) sum[2] += v[bl.lb + M * t.lb_row + cb / 8 + a * q + b];
       };
       auto other = [&](int s) { return s != jt.v_slot && s != jt.n_slot && env[s] != ref; };
       for (int a = 0; a < kEnvSlots; ++a)
@@ -151,6 +157,7 @@ int main(int argc, char **argv) {
         worst = std::max(worst, std::fabs(dense[i] - static_cast<double>(want.v[i])) / scale);
       }
     }
+  }
   std::printf("%.3e\n", worst);
   return 0;
 }

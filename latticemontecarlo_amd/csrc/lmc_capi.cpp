@@ -200,7 +200,6 @@ const KTables &Upload(Model &m) {
   std::vector<int32_t> off;
   for (int d = 0; d < 12; ++d)
     for (int s = 0; s < kEnvSlots; ++s) off.push_back(PackOff(jt.off[d][s]));
-  std::vector<uint8_t> mirror(jt.mirror.begin(), jt.mirror.end());
   // Jump dE weights by migrating species M and reduced index r over element ranks (see
   // ReducedBlock): wd[rank M][r] = w(cluster | endpoint M) - w(cluster | endpoint X); rows
   // ne .. 2 ne - 1 hold the same values negated (the neighbour endpoint's clusters). Each row
@@ -282,7 +281,6 @@ const KTables &Upload(Model &m) {
 
   BlobBuilder b;
   b.Add(off, &k.off);
-  b.Add(mirror, &k.mirror);
   b.Add(state, &k.state);
   b.Add(mmm, &k.mmm);
   b.Add(mm2, &k.mm2);

@@ -25,7 +25,6 @@ constexpr int kMaxW = 1024;  // w1 | w2 | w3 for S <= 6
 // Kernel view of a model (passed by value).
 struct KTables {
   const int32_t *off;       // [12][60]
-  const uint8_t *mirror;    // [60]
   const uint32_t *state;    // one-endpoint state clusters
   const uint32_t *mmm;
   const uint32_t *mm2;
@@ -249,5 +248,8 @@ struct DeviceLimits {
   size_t lds_cu, lds_block;
 };
 const DeviceLimits &CurrentDeviceLimits();
+// Raises a kernel's dynamic LDS limit on the current device to `bytes`; it is never lowered, so that
+// a launch with less on one thread leaves another thread's launch (or a captured one) its limit.
+hipError_t RaiseDynamicLds(const void *kernel, size_t bytes);
 
 }  // namespace lmc

@@ -664,8 +664,7 @@ KmcLayout PlanLds(const KTables &t, int teams, int waves, size_t extra, int per_
 
 template <typename K>
 hipError_t AllowLds(K kernel, size_t bytes) {
-  return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+  return RaiseDynamicLds(reinterpret_cast<const void *>(kernel), bytes);
 }
 
 // f(quartic, tables in LDS) with compile-time arguments.
@@ -682,10 +681,13 @@ hipError_t LaunchEval(const KTables &t, const uint8_t *occ, const int64_t *off, 
                       hipStream_t s, uint8_t *env_out, double *ekra_out, int n, int64_t sub_site,
                       int sub_code) {
   if (R <= 0) return hipSuccess;
-  // two workgroups per CU is what the LDS of a ternary model holds
-  const int cus = CurrentDeviceLimits().cus;
-  const int blocks = std::min((R + kEvalWaves - 1) / kEvalWaves, 2 * cus);
   const KmcLayout lay = PlanLds(t, kEvalWaves, kEvalWaves, 0, 1);
+  // As many workgroups as are resident at once (one per CU for a ternary model's 92 KB; 2 where two fit), so
+  // that none copies the tables again. Two per CU where one fits: 32 000 sites 73.8 us, one 71.8; 8 192
+  // sites 48.7 and 45.5; Quartic 85.4 and 82.1, 52.5 and 49.0.
+  const DeviceLimits &dl = CurrentDeviceLimits();
+  const size_t lds = (t.kind == kQuartic ? sizeof(PairShared<true>) : sizeof(PairShared<false>)) + lay.bytes;
+  const int blocks = std::min((R + kEvalWaves - 1) / kEvalWaves, (2 * lds <= dl.lds_cu ? 2 : 1) * dl.cus);
   return WithModel(t, lay, [&](auto q, auto tab) {
     auto kernel = EvalJumpsKernel<decltype(q)::value, decltype(tab)::value, kScan>;
     const hipError_t e = AllowLds(kernel, lay.bytes);
@@ -787,6 +789,20 @@ hipError_t LaunchKmc(const KTables &t, const KmcDev &k, uint64_t steps, uint64_t
                        trace_base);
     return hipGetLastError();
   });
+}
+
+hipError_t RaiseDynamicLds(const void *kernel, size_t bytes) {
+  static std::mutex mu;
+  static std::map<std::pair<int, const void *>, size_t> allowed;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(mu);
+  size_t &most = allowed[{dev, kernel}];
+  if (bytes <= most) return hipSuccess;
+  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+  if (e == hipSuccess) most = bytes;
+  return e;
 }
 
 const DeviceLimits &CurrentDeviceLimits() {

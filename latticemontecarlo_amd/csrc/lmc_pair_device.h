@@ -648,11 +648,11 @@ __device__ __forceinline__ double OrderedDe(const KTables &t, OrderedLds &D, int
   return sum;
 }
 
-// exp to within one unit in the last place: x = k ln 2 + r by Cody and Waite's two-part reduction, the
-// Taylor series to r^13 (truncation below 2^-57 at |r| = ln 2 / 2) in even and odd halves, then the
-// scaling by 2^k, which takes care of overflow and gradual underflow. NaN stays NaN. The
-// constants are made opaque so that they stay in vector registers: as literals each would take two scalar
-// moves at every use.
+// exp: x = k ln 2 + r by Cody and Waite's two-part reduction, the Taylor series to r^13 (truncation below
+// 2^-57 at |r| = ln 2 / 2) in even and odd halves, then the scaling by 2^k, which takes care of overflow
+// and gradual underflow. NaN stays NaN. The same fused steps on 6e7 arguments up to 708 either way are at
+// most 1.04 units in the last place off. The constants are made opaque so that they stay in vector
+// registers: as literals each would take two scalar moves at every use.
 struct ExpConst {
   double log2e, hi, lo, c[12];  // c[i] = 1 / (i + 2)!
 };

@@ -1858,9 +1858,7 @@ hipError_t LaunchCmc(const KTables &t, const CmcDev &c, uint64_t trials, uint64_
   auto launch = [&](auto kernel_lds, auto kernel_hbm, size_t st, int threads) {
     if (c.lds_occupancy && dyn % 4 == 0 && st + dyn <= lds_block) {
       if (dyn > 65536 - st) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel_lds),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 static_cast<int>(dyn));
+        const hipError_t e = RaiseDynamicLds(reinterpret_cast<const void *>(kernel_lds), dyn);
         if (e != hipSuccess) return e;
       }
       hipLaunchKernelGGL(kernel_lds, dim3(c.R), dim3(threads), dyn, s, t, c, trials, trace_base);

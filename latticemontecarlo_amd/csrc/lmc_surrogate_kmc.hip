@@ -27,8 +27,6 @@
 //   7. apply.
 #include <hip/hip_runtime.h>
 
-#include <map>
-#include <mutex>
 
 #include "lmc_jump_device.h"
 #include "lmc_mlp.h"
@@ -590,20 +588,9 @@ DynLayout PlanSurrogateLds(const KTables &t, int G) {
   return lay;
 }
 
-// Raises a kernel's dynamic LDS limit to `bytes` once (the largest size allowed so far is kept
-// per kernel function; every instance of the surrogate kernel has the same pointer type).
 template <typename K>
 hipError_t AllowSurrogateLds(K kernel, size_t bytes) {
-  static std::mutex mu;
-  static std::map<const void *, int> allowed;
-  const void *f = reinterpret_cast<const void *>(kernel);
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = allowed.find(f);
-  if (it != allowed.end() && static_cast<int>(bytes) <= it->second) return hipSuccess;
-  const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           static_cast<int>(bytes));
-  if (e == hipSuccess) allowed[f] = static_cast<int>(bytes);
-  return e;
+  return RaiseDynamicLds(reinterpret_cast<const void *>(kernel), bytes);
 }
 
 // Workgroup shapes: 4 replicas x 128 threads when the batch has more replicas than the device

@@ -142,3 +142,28 @@ def test_formulations_are_different_kernels(torch, coeffs, R):
     tune = drv.autotune(steps=40)
     assert tune["formulation"] in (1, 2) and tune["ms_solvent"] > 0 and tune["ms_wide"] > 0
     assert tune["ms_dense"] == (tune["ms_wide"] if R <= cus else tune["ms_solvent"])
+
+
+def test_captured_launches_keep_their_lds(torch, coeffs):
+    """A captured launch with much dynamic LDS, replayed after launches of the same kernel with less."""
+    import latticemontecarlo_amd as L
+    path, els = coeffs["e0_3n"]
+    model = L.Model(path, els, L.E0)
+
+    def driver(R):
+        sizes, occs = _batch(model.species, R)
+        d = L.KineticMcFirst(model, None, sizes, occs, 600.0, 5, maximum_steps=10 ** 9)
+        d.set_formulation(1)
+        return d
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    large, small, want = driver(8 * cus), driver(1), driver(8 * cus)  # eight replicas in a workgroup, and one
+    large.build_graph(20, 2)
+    for _ in range(3):
+        small.run(20)
+        large.run_graph(20, 2)
+        small.state()
+        for _ in range(2):
+            want.run(20)
+        a, b = large.state(), want.state()
+        assert np.array_equal(a["vacancy"], b["vacancy"]) and np.array_equal(a["time"], b["time"])
+        assert np.array_equal(a["energy"], b["energy"])

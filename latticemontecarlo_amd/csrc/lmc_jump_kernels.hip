@@ -281,6 +281,7 @@ template <bool kFull>
 struct EnergyKeeper {
   ReplicaLds Q;
   LaneSites ls;
+  OrderedClusters clusters;
   const uint8_t *occ;
   const int32_t *off;  // offsets of the event's slots by direction
   int n, r;
@@ -294,6 +295,7 @@ struct EnergyKeeper {
     r = replica;
     n = k.ncell[r];
     ls = LoadSites(t, wv);
+    clusters = LoadOrdered(t);
     occ = k.occ + k.off[r];
     off = slots;
     sign = way;
@@ -318,7 +320,7 @@ struct EnergyKeeper {
 #pragma nounroll
     do {
       if (i >= 0) {
-        const double de = sign * OrderedDe(t, D, code, wd, mig);
+        const double de = sign * OrderedDe(t, clusters, D, code, wd, mig);
         if constexpr (kFull) {
           const uint64_t steps = i == it && escaped ? Q.max_steps + 1 : Q.steps + i;
           if (k.log_every && LogDue(steps, k.log_every)) {
@@ -347,7 +349,7 @@ struct EnergyKeeper {
 // second barrier, while the leading wave finishes the step.
 template <bool kQ, bool kFull>
 __device__ __forceinline__ void HelpTeam(const KTables &t, const PairShared<kQ> &G, const PairTab &T,
-                                         const TeamLds &S, WaveLds &W, TeamExchange &X, const char *wd,
+                                         const TeamLds &S, WaveLds &W, TeamExchange &X, char *wd,
                                          const KmcDev &k, int r, int wv, uint64_t trace_base) {
   const int lane = LaneId();
   const bool keeps = wv == kTeam - 1;
@@ -368,6 +370,11 @@ __device__ __forceinline__ void HelpTeam(const KTables &t, const PairShared<kQ> 
         if (kQ) p[2] = s.lb;
       }
       __syncthreads();
+    }
+    if (keeps && it == 0) {  // the keeper's tables, needed from the next step on
+      CopyTable(reinterpret_cast<char *>(X.off), t.env_pk, sizeof(X.off), lane, 64);
+      CopyTable(wd, t.wd, 8 * t.nwd, lane, 64);
+      WaveFence();
     }
     if (keeps && it > 0)
       keeper.Take(t, k, X.ordered, wd, it - 1, ReadLaneInt(before, (word >> 8) & 15), K < 0, word >> 12);
@@ -391,10 +398,6 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) voi
   const PairTab T =
       LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, k.solvent[first], threadIdx.x, blockDim.x);
   TeamExchange &X = *reinterpret_cast<TeamExchange *>(dyn + lay.extra);
-  if (kWaves > 1) {
-    CopyTable(dyn + lay.wd, t.wd, 8 * t.nwd, threadIdx.x, blockDim.x);
-    CopyTable(reinterpret_cast<char *>(X.off), t.env_pk, sizeof(X.off), threadIdx.x, blockDim.x);
-  }
   __syncthreads();
   const int r = first + mine;
   if (mine >= group || r >= k.R) return;

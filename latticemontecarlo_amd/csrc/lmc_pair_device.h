@@ -612,15 +612,23 @@ struct OrderedLds {  // element ranks of the event's slots, as the entries of t.
   uint16_t rn8[64];  // rank * 8 * ne
   uint8_t r8[64];    // rank * 8
 };
-// The event whose slot s = lane holds species `code`; M: migrating species; w: the rows of t.wd.
-__device__ __forceinline__ double OrderedDe(const KTables &t, OrderedLds &D, int code, const char *w, int M) {
+struct OrderedClusters {
+  uint32_t entry[2][kOrderedRounds];  // the lane's
+};
+__device__ __forceinline__ OrderedClusters LoadOrdered(const KTables &t) {
   const int lane = LaneId(), half = lane < 42 ? lane : 41;  // lanes past the last sum repeat it
   const uint32_t *list = t.state + (half >> 1) + 42 * (half & 1);
-  uint32_t entry[2][kOrderedRounds];
+  OrderedClusters o;
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int b = 0; b < kOrderedRounds; ++b) entry[j][b] = list[21 * j + kClusterPad * b];
+    for (int b = 0; b < kOrderedRounds; ++b) o.entry[j][b] = list[21 * j + kClusterPad * b];
+  return o;
+}
+// The event whose slot s = lane holds species `code`; M: migrating species; w: the rows of t.wd.
+__device__ __forceinline__ double OrderedDe(const KTables &t, const OrderedClusters &o, OrderedLds &D, int code,
+                                            const char *w, int M) {
+  const int lane = LaneId();
   const uint32_t rank = lane < kEnvSlots ? (t.rank_lut >> (4 * code)) & 15u : 0u;
   D.r8[lane] = static_cast<uint8_t>(rank << 3);
   D.rn8[lane] = static_cast<uint16_t>(__umul24(rank, 8 * t.ne));
@@ -631,7 +639,7 @@ __device__ __forceinline__ double OrderedDe(const KTables &t, OrderedLds &D, int
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int b = 0; b < kOrderedRounds; ++b) {
-      const uint32_t e = entry[j][b];
+      const uint32_t e = o.entry[j][b];
       at[j][b] = D.r8[e & 255u] + D.rn8[(e >> 9) & 127u] + (e >> 16);
     }
   double v[2] = {0.0, 0.0};

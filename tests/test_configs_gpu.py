@@ -170,7 +170,7 @@ def test_surrogate_12x1024_rows_full_fallback_and_exact_energies(torch, bench_co
 @pytest.mark.parametrize("form", [0, 1, 2, 3])
 def test_uneven_size_batch_matches_oracle(torch, coeffs, form):
     """Replicas of 8, 11, 13 and 16 cells (and 9 twice) in one batch: per-replica offsets and box
-    sizes through every kernel shape (0 dense, 1 solvent baseline, 2 dense wide, 3 chain)."""
+    sizes with one wave per replica (1), four (0, 2) and in chain steps (3)."""
     sizes = [8, 11, 13, 16, 9, 9]
     steps = 100 if form == 3 else 300
     print(f"uneven sizes {sizes} form {form}", flush=True)
@@ -347,9 +347,8 @@ def test_early_stop_matches_oracle(torch, coeffs, form):
 
 @pytest.mark.parametrize("name,kind,record", [("e0_3n", 1, False), ("q_3n", 2, True)])
 def test_occupancy_window_long_trajectories(torch, coeffs, name, kind, record):
-    """The dense kernel's LDS occupancy window (boxes of at least 8 cells): 1500 steps on boxes of
-    8 cells (the window spans the whole box along Z), 9 and 12 cells, with the window reloaded
-    many times; with atom tracking and the log compiled in (record) or not."""
+    """1500 steps on boxes of 8, 9 and 12 cells, in which the vacancy crosses the box many times; with atom
+    tracking and the log compiled in (record) or not."""
     import latticemontecarlo_amd as L
     sizes = [8, 8, 9, 12]
     steps = 1500

@@ -31,8 +31,9 @@ def _oracle_models(path, els, n, kinds):
                                        ("q_4", 2)])
 @pytest.mark.parametrize("n", [5, 8])
 def test_eval_jumps_matches_oracle(torch, coeffs, name, kind, n, form):
-    """Both jump formulations (0 dense, 1 solvent baseline) against the oracle, solute
-    fractions 8-28 % per element, vacancies on box corners and edges."""
+    """The jump evaluation against the oracle, solute fractions 8-28 % per element (environments on both
+    sides of the sparse limit), vacancies on box corners and edges. The model's formulation is that of
+    new KMC drivers and leaves the evaluation alone."""
     import latticemontecarlo_amd as L
     path, els = coeffs[name]
     lat, (om,) = _oracle_models(path, els, n, [kind])
@@ -172,7 +173,8 @@ def _compare_kmc(gst, gtr, gocc, refs, steps):
 @pytest.mark.parametrize("form", [0, 1, 2])
 @pytest.mark.parametrize("name,kind", [("e0_3n", 1), ("q_3n", 2)])
 def test_kmc_trajectory_matches_oracle(torch, coeffs, name, kind, form):
-    """Every kernel shape (0 dense, 1 solvent baseline, 2 dense wide) against the oracle."""
+    """The first-order formulations (0 by batch size, here four waves per replica, 1 one wave, 2 four)
+    against the oracle."""
     steps = 400
     gst, gtr, gocc, refs = _run_kmc_pair(coeffs, name, kind, n=6, R=4, steps=steps,
                                          temps=np.array([450.0, 500.0, 600.0, 700.0]), form=form)
@@ -191,7 +193,7 @@ def test_chain_kmc_trajectory_matches_oracle(torch, coeffs, name, kind, opts):
 
 
 def test_kmc_autotune_keeps_results(torch, coeffs, tmp_path):
-    """The autotuner times every kernel shape without changing the replicas' state, tracked
+    """The autotuner times one and four waves per replica without changing the replicas' state, tracked
     atoms or log records."""
     import latticemontecarlo_amd as L
     path, els = coeffs["e0_3"]

@@ -388,8 +388,19 @@ void NeedReference(Model &m, int code) {
   if (!k.pairs || ref < 0 || (m.dev->refs >> ref) & 1) return;
   const std::vector<double> v = BuildPairValues(m, ref);
   const size_t at = v.size() * static_cast<size_t>(ref + (ref < k.first_ref ? 1 : 0));
-  Check(hipMemcpy(const_cast<double *>(k.pairs) + at, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice),
-        "hipMemcpy(model tables)");
+  // on a stream of its own, so that a caller may be capturing its stream
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  Check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+  hipStream_t s = nullptr;
+  hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+  if (e == hipSuccess) {
+    e = hipMemcpyAsync(const_cast<double *>(k.pairs) + at, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice, s);
+    const hipError_t done = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = done;
+    (void)hipStreamDestroy(s);
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  Check(e, "hipMemcpy(model tables)");
   m.dev->refs |= 1u << ref;
 }
 
@@ -936,6 +947,7 @@ int lmc_vacancy_scan(const lmc_model *m, const uint8_t *d_occ, int32_t ncell, in
     if (n_sites > 0 && (!d_occ || !d_sites || !d_nb || !d_ea || !d_de))
       throw std::invalid_argument("null buffer");
     const auto &t = lmc::Upload(*m->m);
+    if (solvent != t.solvent_default) lmc::NeedReference(*m->m, solvent);
     Check(lmc::LaunchVacancyScan(t, d_occ, ncell, vacancy, solvent, d_sites, n_sites, d_nb, d_ea,
                                  d_de, m->m->dev_err, S(stream)),
           "vacancy scan kernel");

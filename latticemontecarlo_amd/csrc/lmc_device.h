@@ -196,8 +196,10 @@ hipError_t LaunchEvalJumps(const KTables &t, const uint8_t *occ, const int64_t *
                            double *ea, double *de, int32_t *err, hipStream_t s,
                            uint8_t *env_out = nullptr, double *ekra_out = nullptr);
 // The 12 jumps of a vacancy placed at each of sites[K] in the single occupancy occ (n^3 cells),
-// with site sub_site holding species sub_code instead (the ExitTime analysis' configuration);
-// outputs [K][12] in neighbour-id order.
+// with site sub_site holding species sub_code instead (the ExitTime analysis' configuration), whose block
+// of values has to be there (NeedReference): the frame is mostly of that species, and the sums run over
+// the sites of other ones. 32 000 sites with 97 % Mg, us, about Al and about Mg: ternary E0 153 and 72,
+// quaternary Quartic 502 and 92. Outputs [K][12] in neighbour-id order.
 hipError_t LaunchVacancyScan(const KTables &t, const uint8_t *occ, int32_t n, int64_t sub_site,
                              int sub_code, const int64_t *sites, int32_t K, int64_t *nb,
                              double *ea, double *de, int32_t *err, hipStream_t s);

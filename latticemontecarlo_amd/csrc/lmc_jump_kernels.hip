@@ -54,12 +54,12 @@ template <bool kQ, bool kTab, bool kScan>
 __global__ __launch_bounds__(64 * kEvalWaves) LMC_WAVES(1, 2) void EvalJumpsKernel(
     KTables t, KmcLayout lay, const uint8_t *occ, const int64_t *off, const int32_t *ncell,
     const int64_t *vac, int32_t R, int64_t *nb, double *ea, double *de, int32_t *err,
-    uint8_t *env_out, double *ekra_out, int scan_n, int64_t sub_site, int sub_code) {
+    uint8_t *env_out, double *ekra_out, int ref, int scan_n, int64_t sub_site, int sub_code) {
   __shared__ PairShared<kQ> G;
   extern __shared__ __align__(16) char dyn[];
   const int lane = LaneId(), wave = WaveIndex();
   const PairTab T =
-      LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, t.solvent_default, threadIdx.x, 64 * kEvalWaves);
+      LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, ref, threadIdx.x, 64 * kEvalWaves);
   __syncthreads();
   TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[wave];
   WaveLds &W = reinterpret_cast<WaveLds *>(dyn + lay.wave)[wave];
@@ -696,7 +696,7 @@ hipError_t LaunchEval(const KTables &t, const uint8_t *occ, const int64_t *off, 
     const hipError_t e = AllowLds(kernel, lay.bytes);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kEvalWaves), lay.bytes, s, t, lay, occ, off, ncell,
-                       vac, R, nb, ea, de, err, env_out, ekra_out, n, sub_site, sub_code);
+                       vac, R, nb, ea, de, err, env_out, ekra_out, kScan ? sub_code : t.solvent_default, n, sub_site, sub_code);
     return hipGetLastError();
   });
 }

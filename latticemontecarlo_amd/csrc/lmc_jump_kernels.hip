@@ -50,7 +50,7 @@ __device__ __forceinline__ int WaveIndex() {
 // with kScan of a vacancy placed at each site vac[r] of the single occupancy occ (scan_n^3 cells)
 // whose site sub_site holds sub_code. One wave per replica or site; the workgroups stride over
 // them, so that one copy of the tables serves many.
-template <bool kQ, bool kTab, bool kScan>
+template <bool kQ, int kTab, bool kScan>
 __global__ __launch_bounds__(64 * kEvalWaves) LMC_WAVES(1, 2) void EvalJumpsKernel(
     KTables t, KmcLayout lay, const uint8_t *occ, const int64_t *off, const int32_t *ncell,
     const int64_t *vac, int32_t R, int64_t *nb, double *ea, double *de, int32_t *err,
@@ -388,7 +388,7 @@ __device__ __forceinline__ void HelpTeam(const KTables &t, const PairShared<kQ> 
 // the table copy. kWaves kTeam: one replica per workgroup, a leading wave makes the step and three
 // helpers share its sums, with two barriers per step (HelpTeam).
 // kFull: options, schedule, trace, log and atoms are compiled in.
-template <bool kQ, bool kTab, int kWaves, bool kFull>
+template <bool kQ, int kTab, int kWaves, bool kFull>
 __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kTeam) LMC_WAVES(1, 2) void KmcKernel(
     KTables t, KmcLayout lay, KmcDev k, int group, int nsteps, uint64_t trace_base) {
   __shared__ PairShared<kQ> G;
@@ -497,7 +497,7 @@ struct ChainExchange {
   OrderedLds ordered;
   int32_t off[12][64];
 };
-template <bool kQ, bool kTab, int kWaves, bool kFull>
+template <bool kQ, int kTab, int kWaves, bool kFull>
 __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kChainTeam) LMC_WAVES(1, 2) void KmcChainKernel(
     KTables t, KmcLayout lay, KmcDev k, int group, int nsteps, uint64_t trace_base) {
   __shared__ PairShared<kQ> G;
@@ -637,7 +637,10 @@ __global__ __launch_bounds__(kWaves == 1 ? 512 : 64 * kChainTeam) LMC_WAVES(1, 2
 }
 
 // Dynamic LDS plan for workgroups of `teams` replicas and `waves` waves: the value tables go to LDS
-// when per_cu workgroups then still fit a CU.
+// when per_cu workgroups then still fit a CU, of a Quartic model also dE and MMM alone (63 of a quaternary
+// one's 163 KB). Quaternary Quartic, none of them in LDS and mixed: first-order steps of equiatomic boxes 6.8
+// and 4.1 us (64 replicas), 16.4 and 8.4 us (1 024); with 3 % solutes 2.58 and 2.26 us, 2.44 and 2.22 us; a scan
+// of 32 000 sites of an equiatomic frame 497 and 222 us. The sums over all clusters took 7.5, 15.6 and 468.
 KmcLayout PlanLds(const KTables &t, int teams, int waves, size_t extra, int per_cu, bool ordered = false) {
   const DeviceLimits &dl = CurrentDeviceLimits();
   const bool quartic = t.kind == kQuartic;
@@ -654,13 +657,13 @@ KmcLayout PlanLds(const KTables &t, int teams, int waves, size_t extra, int per_
   add(lay.extra, extra);
   if (ordered) add(lay.wd, 8 * static_cast<size_t>(t.nwd));
   const size_t row = 8 * static_cast<size_t>(t.ne);
-  const size_t tabs = row * (t.de_row + t.la_row + (quartic ? t.lb_row : 0)) + 48;
-  if (fixed + at + tabs <= share) {
-    lay.tab.tab_lds = 1;
+  const size_t some = row * (t.de_row + t.la_row) + 32, all = some + (quartic ? row * t.lb_row + 16 : 0);
+  lay.tab.tab_lds = fixed + at + all <= share ? kShared : quartic && fixed + at + some <= share ? kMixed : kGlobal;
+  if (lay.tab.tab_lds != kGlobal) {
     add(lay.tab.de, row * t.de_row);
     add(lay.tab.la, row * t.la_row);
-    if (quartic) add(lay.tab.lb, row * t.lb_row);
   }
+  if (quartic && lay.tab.tab_lds == kShared) add(lay.tab.lb, row * t.lb_row);
   lay.bytes = static_cast<int>(at);
   return lay;
 }
@@ -673,9 +676,12 @@ hipError_t AllowLds(K kernel, size_t bytes) {
 // f(quartic, tables in LDS) with compile-time arguments.
 template <typename F>
 hipError_t WithModel(const KTables &t, const KmcLayout &lay, F &&f) {
-  if (t.kind == kQuartic)
-    return lay.tab.tab_lds ? f(std::true_type{}, std::true_type{}) : f(std::true_type{}, std::false_type{});
-  return lay.tab.tab_lds ? f(std::false_type{}, std::true_type{}) : f(std::false_type{}, std::false_type{});
+  constexpr std::integral_constant<int, kGlobal> global;
+  constexpr std::integral_constant<int, kShared> shared;
+  constexpr std::integral_constant<int, kMixed> mixed;
+  if (t.kind != kQuartic) return lay.tab.tab_lds ? f(std::false_type{}, shared) : f(std::false_type{}, global);
+  if (lay.tab.tab_lds == kMixed) return f(std::true_type{}, mixed);
+  return lay.tab.tab_lds ? f(std::true_type{}, shared) : f(std::true_type{}, global);
 }
 
 template <bool kScan>
@@ -730,7 +736,8 @@ KmcPlan PlanKmc(const KTables &t, int32_t R, int form) {
 template <typename F>
 hipError_t WithKmcKernel(const KTables &t, const KmcPlan &p, bool full, F &&f) {
   return WithModel(t, p.lay, [&](auto q, auto tab) {
-    constexpr bool kQ = decltype(q)::value, kT = decltype(tab)::value;
+    constexpr bool kQ = decltype(q)::value;
+    constexpr int kT = decltype(tab)::value;
     auto pick = [&](auto all) {
       constexpr bool kF = decltype(all)::value;
       if (p.chain) return p.team ? f(KmcChainKernel<kQ, kT, kTeam, kF>) : f(KmcChainKernel<kQ, kT, 1, kF>);

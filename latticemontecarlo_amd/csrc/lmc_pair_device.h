@@ -73,7 +73,8 @@ struct PairShared {
   double base[5 * 3], par[kMaxSpecies * 6];
 };
 
-// Where the value tables lie in dynamic LDS (bytes; tab_lds 0: in global memory).
+// Where the value tables lie in dynamic LDS (bytes). tab_lds: kGlobal none of them, kShared all, kMixed dE and MMM.
+constexpr int kGlobal = 0, kShared = 1, kMixed = 2;
 struct PairLayout {
   int de, la, lb, bytes, tab_lds;
 };
@@ -115,8 +116,8 @@ __device__ __forceinline__ void CopyTable(char *dst, const void *src, int bytes,
 }
 
 // The workgroup's tables for reference species code `ref` into LDS (all threads; the caller
-// synchronises). kTab: the value tables go to dynamic LDS, else they are read from global memory.
-template <bool kQ, bool kTab>
+// synchronises). kTab: where the value tables go; what stays in global memory is read there.
+template <bool kQ, int kTab>
 __device__ __forceinline__ PairTab LoadPairTables(const KTables &t, PairShared<kQ> &G, char *dyn,
                                                   const PairLayout &lay, int ref, int tid, int size) {
   const int rr = static_cast<int>((t.rank_lut >> (4 * ref)) & 15u);
@@ -150,17 +151,18 @@ __device__ __forceinline__ PairTab LoadPairTables(const KTables &t, PairShared<k
   const char *de = reinterpret_cast<const char *>(v);
   const char *la = reinterpret_cast<const char *>(v + at.la);
   const char *lb = reinterpret_cast<const char *>(v + at.lb);
-  if (kTab) {
+  T.de = de;
+  T.la = la;
+  T.lb = lb;
+  if (kTab != kGlobal) {
     CopyTable(dyn + lay.de, de, t.ne * T.de_row, tid, size);
     CopyTable(dyn + lay.la, la, t.ne * T.la_row, tid, size);
-    if (kQ) CopyTable(dyn + lay.lb, lb, t.ne * T.lb_row, tid, size);
     T.de = dyn + lay.de;
     T.la = dyn + lay.la;
+  }
+  if (kQ && kTab == kShared) {
+    CopyTable(dyn + lay.lb, lb, t.ne * T.lb_row, tid, size);
     T.lb = dyn + lay.lb;
-  } else {
-    T.de = de;
-    T.la = la;
-    T.lb = lb;
   }
   return T;
 }

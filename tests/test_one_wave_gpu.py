@@ -2,7 +2,7 @@
 unequal boxes, solvents and solute contents share a workgroup and its tables (those of its first
 replica's solvent). A sample of replicas from both ends and the middle of workgroups is replayed by the
 oracle, as are the atoms' jumps; first-order and chain steps, both barrier models, value tables in LDS
-(ternary E0) and in global memory (quaternary Quartic), environments past the sparse limit."""
+(ternary E0) and partly in global memory (quaternary Quartic), environments past the sparse limit."""
 import numpy as np
 import pytest
 
@@ -115,6 +115,27 @@ def test_large_batches_match_oracle(torch, coeffs, tmp_path, name, kind, chain, 
             assert [int(x[0]) for x in lines] == list(range(steps))  # every step below 99
             for s, x in enumerate(lines):
                 assert float(x[head.index("energy")]) == pytest.approx(energy[s], rel=1e-4, abs=1e-9)
+
+
+@pytest.mark.parametrize("name,kind", [("e0_4n", 1), ("q_3n", 2), ("q_4", 2)])
+def test_chain_teams_that_share_a_cu(torch, coeffs, name, kind):
+    """Two teams of a CU have half of its LDS each, so that less of the value tables is there than for the same
+    replicas in a smaller batch: none of a quaternary model's, where that has all (E0) or part (Quartic)."""
+    import latticemontecarlo_amd as L
+    path, els = coeffs[name]
+    model = L.Model(path, els, kind)
+    R = torch.cuda.get_device_properties(0).multi_processor_count + 44
+    sizes, occs = _batch(model.species, R)
+    print(f"{R} chain replicas, {name}", flush=True)
+    got = []
+    for many in (R, 40):
+        drv = L.KineticMcChain(model, None, sizes[:many], occs[:many], 650.0, 7, maximum_steps=10 ** 9)
+        drv.run(12)
+        model.check_errors()
+        got.append(drv.state())
+    assert np.array_equal(got[0]["vacancy"][:40], got[1]["vacancy"])
+    assert np.array_equal(got[0]["disp"][:40], got[1]["disp"])
+    np.testing.assert_allclose(got[0]["energy"][:40], got[1]["energy"], rtol=0, atol=TOL_E)
 
 
 @pytest.mark.parametrize("R", [5, 300])

@@ -17,8 +17,9 @@ def torch():
 
 
 @pytest.mark.parametrize("captured", [False, True])
-@pytest.mark.parametrize("name,kind,base", [("e0_3n", 1, "Mg"), ("e0_3n", 1, "Zn"), ("q_4", 2, "Mg")])
-def test_scan_of_another_base_metal(torch, coeffs, name, kind, base, captured):
+@pytest.mark.parametrize("name,kind,base,solute", [("e0_3n", 1, "Mg", 0.08), ("e0_3n", 1, "Zn", 0.08),
+                                                   ("q_4", 2, "Mg", 0.08), ("q_4", 2, "Cu", 0.25)])
+def test_scan_of_another_base_metal(torch, coeffs, name, kind, base, solute, captured):
     import latticemontecarlo_amd as L
     import oracle as O
     from latticemontecarlo_amd import capi
@@ -26,7 +27,7 @@ def test_scan_of_another_base_metal(torch, coeffs, name, kind, base, captured):
     n = 6
     gm = L.Model(path, els, kind)
     sp = gm.species
-    occ = random_alloc(n, sp, 0.08, seed=72)
+    occ = random_alloc(n, sp, solute, seed=72)
     al, code = sp.index("Al"), sp.index(base)
     occ = np.where(occ == al, code, np.where(occ == code, al, occ)).astype(np.uint8)
     vac = int(np.flatnonzero(occ == sp.index("X"))[0])

@@ -33,6 +33,10 @@ namespace {
 #define LMC_WAVES(lo, hi) __attribute__((amdgpu_waves_per_eu(lo, hi)))
 
 constexpr int kEvalWaves = 8;  // waves of an evaluation workgroup
+// kMaxSparse where they share the dense sums. Back-to-back calls of 12 vacancies (E0, ternary / Quartic,
+// quaternary) at 11, 16, 21, 27 and 32 such sites, us: sparse 6.1, 6.5, 6.9, 7.4 and 8.2 / 7.3, 8.0, 8.3, 9.2
+// and 10.0, dense 7.0 / 8.8 at any content.
+constexpr int kMaxShared = 20;
 constexpr int kTeam = 4;       // waves of a replica in the team shape
 constexpr int kChainTeam = kTeam + 1;  // of a team that makes chain steps, with the one that keeps the energies
 
@@ -49,8 +53,9 @@ __device__ __forceinline__ int WaveIndex() {
 // The 12 jumps of each replica r (vacancy vac[r] in occupancy occ + off[r] of ncell[r]^3 cells), or
 // with kScan of a vacancy placed at each site vac[r] of the single occupancy occ (scan_n^3 cells)
 // whose site sub_site holds sub_code. One wave per replica or site; the workgroups stride over
-// them, so that one copy of the tables serves many.
-template <bool kQ, int kTab, bool kScan>
+// them, so that one copy of the tables serves many. kShare: a workgroup to each, whose waves share the sums
+// where they are dense.
+template <bool kQ, int kTab, bool kScan, bool kShare>
 __global__ __launch_bounds__(64 * kEvalWaves) LMC_WAVES(1, 2) void EvalJumpsKernel(
     KTables t, KmcLayout lay, const uint8_t *occ, const int64_t *off, const int32_t *ncell,
     const int64_t *vac, int32_t R, int64_t *nb, double *ea, double *de, int32_t *err,
@@ -61,16 +66,29 @@ __global__ __launch_bounds__(64 * kEvalWaves) LMC_WAVES(1, 2) void EvalJumpsKern
   const PairTab T =
       LoadPairTables<kQ, kTab>(t, G, dyn, lay.tab, ref, threadIdx.x, 64 * kEvalWaves);
   __syncthreads();
-  TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[wave];
+  TeamLds &S = reinterpret_cast<TeamLds *>(dyn + lay.team)[kShare ? 0 : wave];
   WaveLds &W = reinterpret_cast<WaveLds *>(dyn + lay.wave)[wave];
+  int &listed = *reinterpret_cast<int *>(dyn + lay.extra);  // kShare: the first wave's K
+  if (kShare && wave != 0) {
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(listed) > kMaxShared) (void)DenseTerms<kQ, kEvalWaves>(G, T, S, W, 0, wave);
+    __syncthreads();
+    return;
+  }
   const LaneSites ls = LoadSites<!kScan>(t, 0);
   const ExpConst E = MakeExpConst();
-  for (int64_t r = static_cast<int64_t>(blockIdx.x) * kEvalWaves + wave; r < R;
-       r += static_cast<int64_t>(gridDim.x) * kEvalWaves) {
+  constexpr int kSites = kShare ? 1 : kEvalWaves;  // of a workgroup at a time
+  for (int64_t r = static_cast<int64_t>(blockIdx.x) * kSites + wave; r < R;
+       r += static_cast<int64_t>(gridDim.x) * kSites) {
     const int n = kScan ? scan_n : ncell[r];
     const int64_t site = vac[r];
     if (!ValidSite(n, site)) {
       if (lane == 0) atomicOr(err, 8);
+      if (kShare) {
+        if (lane == 0) listed = 0;
+        __syncthreads();
+        __syncthreads();
+      }
       continue;
     }
     const uint8_t *o = kScan ? occ : occ + off[r];
@@ -82,8 +100,23 @@ __global__ __launch_bounds__(64 * kEvalWaves) LMC_WAVES(1, 2) void EvalJumpsKern
     const bool bad = CheckCodes(t, a, dir, err);
     const int M = Bpermute(dir, a.code[0]);
     const EventConst ec = LoadConst(t, G, M);
-    const int K = ListSites<kQ>(t, G, T, S, ls, a);
-    const PairSums s = PairTerms<kQ, 1>(G, T, S, W, ls, K, MakeRow<kQ>(t, T, dir, M), 0);
+    const int K = ListSites<kQ, kShare ? kMaxShared : kMaxSparse>(t, G, T, S, ls, a);
+    PairSums s{0.0, 0.0, 0.0};
+    if (kShare) {
+      if (lane == 0) listed = K;
+      __syncthreads();
+      if (K > kMaxShared) (void)DenseTerms<kQ, kEvalWaves>(G, T, S, W, dir, 0);
+      else s = PairTerms<kQ, 1>(G, T, S, W, ls, K, MakeRow<kQ>(t, T, dir, M), 0);
+      __syncthreads();
+      for (int w = 0; K > kMaxShared && w < kEvalWaves; ++w) {
+        const double(&x)[3] = (&W)[w].sum[dir];
+        s.de += x[0];
+        s.la += x[1];
+        if (kQ) s.lb += x[2];
+      }
+    } else {
+      s = PairTerms<kQ, 1>(G, T, S, W, ls, K, MakeRow<kQ>(t, T, dir, M), 0);
+    }
     const EventValue e = FinishEvent<kQ>(E, ec, s, bad);
     const uint64_t id = Bpermute64(dir, a.id[0]);
     if (lane < 12) {
@@ -690,15 +723,21 @@ hipError_t LaunchEval(const KTables &t, const uint8_t *occ, const int64_t *off, 
                       hipStream_t s, uint8_t *env_out, double *ekra_out, int n, int64_t sub_site,
                       int sub_code) {
   if (R <= 0) return hipSuccess;
-  const KmcLayout lay = PlanLds(t, kEvalWaves, kEvalWaves, 0, 1);
+  const KmcLayout lay = PlanLds(t, kEvalWaves, kEvalWaves, 16, 1);
   // As many workgroups as are resident at once (one per CU for a ternary model's 92 KB; 2 where two fit), so
   // that none copies the tables again. Two per CU where one fits: 32 000 sites 73.8 us, one 71.8; 8 192
   // sites 48.7 and 45.5; Quartic 85.4 and 82.1, 52.5 and 49.0.
   const DeviceLimits &dl = CurrentDeviceLimits();
   const size_t lds = (t.kind == kQuartic ? sizeof(PairShared<true>) : sizeof(PairShared<false>)) + lay.bytes;
-  const int blocks = std::min((R + kEvalWaves - 1) / kEvalWaves, (2 * lds <= dl.lds_cu ? 2 : 1) * dl.cus);
+  // A CU to each where there is one: eight waves share the dense sums. Calls of 64 equiatomic boxes, us, from
+  // Python: ternary E0 32.6, by one wave 36.0, by sums over all clusters 32.5; quaternary Quartic 33.6, 40.7
+  // and 36.5.
+  const bool share = R <= dl.cus;
+  const int blocks = share ? R : std::min((R + kEvalWaves - 1) / kEvalWaves, (2 * lds <= dl.lds_cu ? 2 : 1) * dl.cus);
   return WithModel(t, lay, [&](auto q, auto tab) {
-    auto kernel = EvalJumpsKernel<decltype(q)::value, decltype(tab)::value, kScan>;
+    constexpr bool kQ = decltype(q)::value;
+    constexpr int kT = decltype(tab)::value;
+    auto kernel = share ? EvalJumpsKernel<kQ, kT, kScan, true> : EvalJumpsKernel<kQ, kT, kScan, false>;
     const hipError_t e = AllowLds(kernel, lay.bytes);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kEvalWaves), lay.bytes, s, t, lay, occ, off, ncell,

@@ -319,8 +319,8 @@ __device__ __forceinline__ EventRow MakeRow(const KTables &t, const PairTab &T, 
 }
 
 // Lists the non-reference sites of `a` in S.sol with blanks after them; returns their number
-// (uniform). With more than kMaxSparse, the inputs of DenseTerms are formed instead.
-template <bool kQ, typename Id>
+// (uniform). With more than kMax, the inputs of DenseTerms are formed instead.
+template <bool kQ, int kMax = kMaxSparse, typename Id>
 __device__ __forceinline__ int ListSites(const KTables &t, const PairShared<kQ> &G, const PairTab &T, TeamLds &S,
                                          const LaneSites &ls, const Around<Id> &a) {
   const int lane = LaneId();
@@ -333,7 +333,7 @@ __device__ __forceinline__ int ListSites(const KTables &t, const PairShared<kQ> 
     if (u == 2) mask[u] &= kThirdMask;
     K += __builtin_popcountll(mask[u]);
   }
-  if (K <= kMaxSparse) {
+  if (K <= kMax) {
     int at = 0;
 #pragma unroll
     for (int u = 0; u < 3; ++u) {

@@ -54,3 +54,36 @@ def test_sample_rows_hold_the_species_of_every_slot(torch, coeffs):
         for row, b in zip(env, L.fcc_neighbors(n, vac, 1)):
             assert row[:60].tolist() == [int(occ[s]) for s in L.jump_environment(n, vac, int(b))]
             assert not row[60:].any()
+
+
+@pytest.mark.parametrize("many", [1, 40, 0, 1000])
+@pytest.mark.parametrize("name,kind", [("e0_3n", 1), ("q_4", 2)])
+def test_shared_and_single_wave_sums_match_oracle(torch, coeffs, name, kind, many):
+    """One workgroup to each vacancy up to the number of CUs (0 here), eight vacancies to a workgroup above;
+    contents below and above both limits of the sparse sums, and an invalid vacancy among the others."""
+    import latticemontecarlo_amd as L
+    import oracle as O
+    from latticemontecarlo_amd import capi
+    path, els = coeffs[name]
+    R = many or torch.cuda.get_device_properties(0).multi_processor_count
+    model, n = L.Model(path, els, kind), 5
+    x = model.species.index("X")
+    occs = [random_alloc(n, model.species, (0.02, 0.06, 0.08, 0.10, 0.2)[r % 5], seed=500 + r) for r in range(R)]
+    vac = np.array([int(np.flatnonzero(o == x)[0]) for o in occs])
+    print(f"{R} vacancies, {name}", flush=True)
+    got = [v.cpu().numpy().reshape(R, 12) for v in L.eval_jumps(model, L.ReplicaBatch([n] * R, occs), vac)]
+    model.check_errors()
+    lat = O.Lattice(n)
+    om = O.Model(lat, path, els, kind)
+    for r in sorted({*range(min(R, 10)), *range(max(R - 5, 0), R)}):
+        for j, b in enumerate(sorted(int(b) for b in lat.neighbors(int(vac[r]), 1))):
+            ea, de = om.barrier_de(occs[r], int(vac[r]), b)
+            assert got[0][r, j] == b
+            assert abs(got[1][r, j] - ea) <= 1e-9 and abs(got[2][r, j] - de) <= 1e-9, (r, j)
+    bad = vac.copy()
+    bad[R // 2] = 4 * n ** 3
+    other = [v.cpu().numpy().reshape(R, 12) for v in L.eval_jumps(model, L.ReplicaBatch([n] * R, occs), bad)]
+    with pytest.raises(capi.LmcError):
+        model.check_errors()
+    keep = np.arange(R) != R // 2
+    assert all(np.array_equal(g[keep], o[keep]) for g, o in zip(got, other))

@@ -15,7 +15,7 @@
 //
 // Measured, 1 024 replicas of 20^3 cells (E0, 2-10 at.% solute), per step of the slowest replica: 2.4 us,
 // against 6.3 us of summing every cluster with 256 threads per replica (12.6 -> 4.7 ms per 2 000 steps;
-// 700 instructions and 4 700 cycles of a wave); 384 000 jumps of an exit-time scan 39 against 254 us.
+// 700 instructions and 4 700 cycles of a wave); 384 000 jumps of an exit-time scan 36 against 254 us.
 // kMaxSparse: a step by the dense sums takes 5.9 us at any composition (summing every cluster: 6.6 us). The
 // line at 24, 32, 40 and 48 sites gives, with one wave per replica (1 024 replicas), 5.7, 4.8, 4.1 and 4.1 us
 // at 2-9 at.% of each solute and 5.8, 5.8, 5.9 and 6.8 us at 3-15 %; with four (128 replicas) 2.7, 2.3, 2.3
